@@ -34,18 +34,18 @@ COMMON = [
 ]
 
 N_CFG = 3      # register-staged tile configurations (TileCfg)
-N_DL_CFG = 4   # gemm_f32_dl tile configurations (DlCfg 0..3; DlCfg 4 is gemm_f32_dlp)
+SP_CFG = (0, 1, 2, 3, 4, 6, 7)   # gemm_f32_sp tile configurations (SpCfg)
 
 
 def _units():
     units = []
     for cfg in range(N_CFG):
         units.append((CSRC / "gemm_instances.hip", OBJDIR / f"gemm_cfg{cfg}.o", [f"-DMT_CFG={cfg}"]))
-    for cfg in range(N_DL_CFG):
-        units.append((CSRC / "gemm_dl_instances.hip", OBJDIR / f"gemm_dl_cfg{cfg}.o",
+    for cfg in SP_CFG:
+        units.append((CSRC / "gemm_sp_instances.hip", OBJDIR / f"gemm_sp_cfg{cfg}.o",
                       [f"-DMT_CFG={cfg}"]))
+    units.append((CSRC / "gemm_dl_instances.hip", OBJDIR / "gemm_dl.o", []))
     units.append((CSRC / "gemm_dlp_instances.hip", OBJDIR / "gemm_dlp.o", []))
-    units.append((CSRC / "gemm_dl16_instances.hip", OBJDIR / "gemm_dl16.o", []))
     units.append((CSRC / "gemm_ksw_instances.hip", OBJDIR / "gemm_ksw.o", []))
     units.append((CSRC / "gemm_skinny_instances.hip", OBJDIR / "gemm_skinny.o", []))
     units.append((CSRC / "mtgemm_api.hip", OBJDIR / "mtgemm_api.o", []))

@@ -10,8 +10,8 @@ namespace mtk {
 
 // Block tile BM x BN x BK, wave tile WM x WN.  Threads = (BM/WM)*(BN/WN)*64.
 template <int CFG> struct TileCfg;
-// 256x256: one workgroup (8 waves, 2 per SIMD) fills a CU; 4096^2 -> 256 tiles.
-template <> struct TileCfg<0> { static constexpr int BM = 256, BN = 256, BK = 16, WM = 128, WN = 64; };
+// 256x128: 8 waves, 2 per SIMD.
+template <> struct TileCfg<0> { static constexpr int BM = 256, BN = 128, BK = 16, WM = 64, WN = 64; };
 // 128x128: 4 waves; several workgroups share a CU.
 template <> struct TileCfg<1> { static constexpr int BM = 128, BN = 128, BK = 16, WM = 64, WN = 64; };
 // 64x64: 4 waves of 32x32, for small and skinny problems (usually with split-K).
@@ -33,101 +33,104 @@ GemmLaunchFn launcher_cfg0(int la, int lb);
 GemmLaunchFn launcher_cfg1(int la, int lb);
 GemmLaunchFn launcher_cfg2(int la, int lb);
 
-// Direct-to-LDS kernel (gemm_dl_kernel.hpp) for operands whose layouts are both
-// L_KV or L_MV: block tile BM x BN, wave tile WM x WN, STAGES-deep LDS ring of
-// 16-deep K-chunks.  Same tile sizes, in the same order, as TileCfg.
+// The bf16-unit kernel gemm_f32_sp (gemm_sp_kernel.hpp): block tile BM x BN
+// (on blocks of BNB columns), wave tile WM x WN, WPE: waves per SIMD its
+// registers are sized for.  It makes configurations 0, 1, 3, 4, 6 and 7 below
+// (same index) and, for contiguous
+// operands of any alignment, the register-staged configurations (2: 64x64).
+template <int CFG> struct SpCfg;
+template <> struct SpCfg<0> { static constexpr int BM = 64, BN = 256, BNB = 256, WM = 64, WN = 64, WPE = 2; };
+template <> struct SpCfg<1> { static constexpr int BM = 128, BN = 128, BNB = 128, WM = 64, WN = 64, WPE = 2; };
+template <> struct SpCfg<2> { static constexpr int BM = 64, BN = 64, BNB = 64, WM = 32, WN = 32, WPE = 4; };
+template <> struct SpCfg<3> { static constexpr int BM = 256, BN = 128, BNB = 128, WM = 64, WN = 64, WPE = 2; };
+template <> struct SpCfg<4> { static constexpr int BM = 128, BN = 256, BNB = 256, WM = 64, WN = 64, WPE = 2; };
+template <> struct SpCfg<6> { static constexpr int BM = 128, BN = 64, BNB = 64, WM = 64, WN = 32, WPE = 3; };
+template <> struct SpCfg<7> { static constexpr int BM = 64, BN = 112, BNB = 128, WM = 32, WN = 64, WPE = 3; };
+constexpr bool is_sp_cfg(int cfg) {
+    return cfg == 0 || cfg == 1 || cfg == 3 || cfg == 4 || cfg == 6 || cfg == 7;
+}
+
+// Its launcher for (layout of A: L_KV, L_MV, L_KVI; of B: L_KV, L_MV, L_IM, L_IMW,
+// L_IMR), with the row sums of A if rs (two L_KV or two L_MV); nullptr where the
+// configuration has no such form.
+GemmLaunchFn sp_launcher_cfg0(int la, int lb, bool rs);
+GemmLaunchFn sp_launcher_cfg1(int la, int lb, bool rs);
+GemmLaunchFn sp_launcher_cfg2(int la, int lb, bool rs);
+GemmLaunchFn sp_launcher_cfg3(int la, int lb, bool rs);
+GemmLaunchFn sp_launcher_cfg4(int la, int lb, bool rs);
+GemmLaunchFn sp_launcher_cfg6(int la, int lb, bool rs);
+GemmLaunchFn sp_launcher_cfg7(int la, int lb, bool rs);
+
+// Configurations of the direct-to-LDS family, for operands whose layouts are
+// both L_KV or L_MV and the implicit convolution operands.
 template <int CFG> struct DlCfg;
-// 8 waves of 128x64; 2 x 32 KB ring.
-template <> struct DlCfg<0> { static constexpr int BM = 256, BN = 256, WM = 128, WN = 64, STAGES = 2; };
-// 8 waves of 64x32; 2 x 16 KB ring, up to four workgroups per CU.
-template <> struct DlCfg<1> { static constexpr int BM = 128, BN = 128, WM = 64, WN = 32, STAGES = 2; };
+template <> struct DlCfg<0> : SpCfg<0> {};
+template <> struct DlCfg<1> : SpCfg<1> {};
+// gemm_f32_dl (gemm_dl_kernel.hpp): STAGES-deep LDS ring of 16-deep K-chunks;
 // 4 waves of 32x32; 2 x 8 KB ring, up to eight workgroups per CU.  (Deeper
 // rings measured slower for these tiles: occupancy hides more latency.)
 template <> struct DlCfg<2> { static constexpr int BM = 64, BN = 64, WM = 32, WN = 32, STAGES = 2; };
-// 8 waves of 64x64; 2 x 24 KB ring.  Fills the chip where M is about 256
-// (e.g. convolutions with 256 output channels: 49 tiles x split 5 = 245).
-template <> struct DlCfg<3> { static constexpr int BM = 256, BN = 128, WM = 64, WN = 64, STAGES = 2; };
-// Configurations 4-6 are the fragment-prefetching kernel gemm_f32_dlp
-// (gemm_dlp_kernel.hpp): vector layouts, the weight-gradient operand L_IMW
-// and the row-sum form; no implicit-im2col (L_IM) form.  4: 4 waves of
-// 128x128 (one per SIMD); 5: 4 waves of 32x32; 6: 8 waves of 64x32 (two per
-// SIMD), the 128x128 tile for K ranges of 512 and more.
+template <> struct DlCfg<3> : SpCfg<3> {};
+// 4-6: not the implicit im2col operand of the forward convolution.
+template <> struct DlCfg<4> : SpCfg<4> {};
+// gemm_f32_dlp (gemm_dlp_kernel.hpp), with fragment prefetch: 4 waves of 32x32.
 // WPE: waves per SIMD its registers are sized for.
-template <> struct DlCfg<4> { static constexpr int BM = 256, BN = 256, WM = 128, WN = 128, STAGES = 2, WPE = 1; };
 template <> struct DlCfg<5> { static constexpr int BM = 64, BN = 64, WM = 32, WN = 32, STAGES = 2, WPE = 8; };
-template <> struct DlCfg<6> { static constexpr int BM = 128, BN = 128, WM = 64, WN = 32, STAGES = 2, WPE = 2; };
+template <> struct DlCfg<6> : SpCfg<6> {};
 
-// Configuration 7 is the convolution kernel on 16x16 MFMA blocks
-// gemm_f32_dl16 (gemm_dl16_kernel.hpp), B = L_IM only: block tile BM x BN,
-// wave tile WM x WN, KG groups of waves splitting the tile's K-chunks, a
-// STAGES-slot ring per group, PRE of a chunk's four MFMA k-steps issued
-// before each barrier.  112 = 7 blocks of 16 divides the pixel count of
-// ResNet layers (multiples of 7*7*16 at even batch sizes).  8 waves: two
-// groups of four 16x112 waves, two waves per SIMD; 72 KB of LDS, two
-// workgroups per CU.
-template <int CFG> struct Dl16Cfg;
-template <> struct Dl16Cfg<0> { static constexpr int BM = 64, BN = 112, WM = 16, WN = 112, KG = 2, STAGES = 3, PRE = 2; };
-constexpr int kNumDl16Cfg = 1;
+// Configuration 1's weight gradient (L_IMW) runs on gemm_f32_dl, whose 16-byte
+// gathers take four channels at once: 8 waves of 64x32, 2 x 16 KB ring.
+template <int CFG> struct DlwCfg;
+template <> struct DlwCfg<1> { static constexpr int BM = 128, BN = 128, WM = 64, WN = 32, STAGES = 2; };
 
-constexpr int kDlpFirstCfg = 4;    // configurations kDlpFirstCfg.. are gemm_f32_dlp
-constexpr int kDl16FirstCfg = 7;   // configurations kDl16FirstCfg.. are gemm_f32_dl16
-constexpr int kNumDlCfg = kDl16FirstCfg + kNumDl16Cfg;
-constexpr bool is_dlp_cfg(int cfg) { return cfg >= kDlpFirstCfg && cfg < kDl16FirstCfg; }
-constexpr bool is_dl16_cfg(int cfg) { return cfg >= kDl16FirstCfg; }
+// Wave tiles of the halo-patch kernel gemm_f32_dlh in the tiles of DlCfg 0-3.
+template <int CFG> struct DlhCfg;
+template <> struct DlhCfg<0> { static constexpr int BM = 64, BN = 256, WM = 64, WN = 64; };
+template <> struct DlhCfg<1> { static constexpr int BM = 128, BN = 128, WM = 64, WN = 32; };
+template <> struct DlhCfg<2> { static constexpr int BM = 64, BN = 64, WM = 32, WN = 32; };
+template <> struct DlhCfg<3> { static constexpr int BM = 256, BN = 128, WM = 64, WN = 64; };
 
-template <int CFG>
-constexpr int dl_threads() {
-    return (DlCfg<CFG>::BM / DlCfg<CFG>::WM) * (DlCfg<CFG>::BN / DlCfg<CFG>::WN) * 64;
-}
+// 7: the channels-last convolution operand only (L_IM), tiles of 112 columns on
+// blocks of 128 (4 waves of 32x64).  112 = 7*16 divides the pixel count of
+// ResNet layers (multiples of 7*7*16 at even batch sizes), so that such a layer
+// has no ragged tile: 28x28 with 128 channels at batch 32 is 448 tiles, two on
+// most CUs, where 128 columns give 392.
+template <> struct DlCfg<7> : SpCfg<7> {};
+constexpr int kNumDlCfg = 8;
+constexpr int kNarrowCfg = 7;
 
-// la, lb in {L_KV, L_MV}.
-GemmLaunchFn dl_launcher_cfg0(int la, int lb);
-GemmLaunchFn dl_launcher_cfg1(int la, int lb);
+constexpr bool is_dlp_cfg(int cfg) { return cfg == 5; }                 // gemm_f32_dlp
+constexpr bool is_wide_cfg(int cfg) { return cfg >= 4 && cfg <= 6; }    // no L_IM, L_IMR
+
+// Configuration 2 (gemm_f32_dl); la, lb in {L_KV, L_MV}.
 GemmLaunchFn dl_launcher_cfg2(int la, int lb);
-GemmLaunchFn dl_launcher_cfg3(int la, int lb);
-// Configurations 4-6 (gemm_f32_dlp); la, lb in {L_KV, L_MV}; tail: K is
-// not a multiple of 16.
-GemmLaunchFn dlp_launcher(int cfg, bool tail, int la, int lb);
-// Configurations 4-6 with the row sums of A (GemmParams::rowsum); A and B L_MV.
-GemmLaunchFn dlp_rowsum_launcher(int cfg, bool tail, bool kv);
-// Configurations 4-6 for the convolution weight gradient (A L_KV, B L_IMW).
-GemmLaunchFn dlp_convw_launcher(int cfg, bool tail);
-// Configurations 4-6 for the weight gradient with A = dY in NCHW (L_KVI).
-GemmLaunchFn dlp_convwi_launcher(int cfg);
+// Configuration 5 (gemm_f32_dlp); la, lb in {L_KV, L_MV}; tail: K is not a
+// multiple of 16.
+GemmLaunchFn dlp_launcher(bool tail, int la, int lb);
+// ... with the row sums of A (GemmParams::rowsum); A and B L_MV, or both L_KV.
+GemmLaunchFn dlp_rowsum_launcher(bool tail, bool kv);
+// ... for the convolution weight gradient (A L_KV, B L_IMW).
+GemmLaunchFn dlp_convw_launcher(bool tail);
+// ... for the weight gradient with A = dY in NCHW (L_KVI).
+GemmLaunchFn dlp_convwi_launcher();
 // Implicit-im2col convolution: A = weights (L_KV), B = L_IM (GemmParams::cv).
-GemmLaunchFn dl16_conv_launcher(int cfg16);   // gemm_f32_dl16, Dl16Cfg<cfg16>
-void dl16_tile(int cfg16, int* bm, int* bn);
-GemmLaunchFn dl_conv_launcher_cfg0();
-GemmLaunchFn dl_conv_launcher_cfg1();
 GemmLaunchFn dl_conv_launcher_cfg2();
-GemmLaunchFn dl_conv_launcher_cfg3();
 // Implicit-im2col convolution from an NCHW view: A = OIHW weights (L_KV), B = L_IMR.
-GemmLaunchFn dl_convr_launcher_cfg0();
-GemmLaunchFn dl_convr_launcher_cfg1();
 GemmLaunchFn dl_convr_launcher_cfg2();
-GemmLaunchFn dl_convr_launcher_cfg3();
 // The same convolution with B built in LDS from a halo patch (L_IMH,
-// gemm_dlh_kernel.hpp): ConvGeom::hp and pw set, LDS per workgroup
-// dlh_lds_floats of the configuration's tile.
-GemmLaunchFn dl_convh_launcher_cfg0();
-GemmLaunchFn dl_convh_launcher_cfg1();
-GemmLaunchFn dl_convh_launcher_cfg2();
-GemmLaunchFn dl_convh_launcher_cfg3();
+// gemm_dlh_kernel.hpp) in the tile of configuration cfg (0-3): ConvGeom::hp and
+// pw set, LDS per workgroup dlh_lds_floats of the configuration's tile.
+GemmLaunchFn dlh_launcher(int cfg);
 // Convolution weight gradient: A = dY [c_out][n*h_out*w_out] (L_KV), B = L_IMW.
-GemmLaunchFn dl_convw_launcher_cfg0();
-GemmLaunchFn dl_convw_launcher_cfg1();
 GemmLaunchFn dl_convw_launcher_cfg2();
-GemmLaunchFn dl_convw_launcher_cfg3();
 // The same with A = dY in NCHW (L_KVI; K a multiple of 16).
-GemmLaunchFn dl_convwi_launcher_cfg0();
-GemmLaunchFn dl_convwi_launcher_cfg1();
 GemmLaunchFn dl_convwi_launcher_cfg2();
-GemmLaunchFn dl_convwi_launcher_cfg3();
-// A and B mn-contiguous, with the row sums of A (GemmParams::rowsum).
-GemmLaunchFn dl_rowsum_launcher_cfg0(bool kv);
-GemmLaunchFn dl_rowsum_launcher_cfg1(bool kv);
+// Both in configuration 1's tile.
+GemmLaunchFn dl_convw_launcher_cfg1();
+GemmLaunchFn dl_convwi_launcher_cfg1();
+// Two mn-contiguous or two k-contiguous operands, with the row sums of A
+// (GemmParams::rowsum).
 GemmLaunchFn dl_rowsum_launcher_cfg2(bool kv);
-GemmLaunchFn dl_rowsum_launcher_cfg3(bool kv);
 
 // Wave-split kernel (gemm_ksw_kernel.hpp): tile (R*MB) x (R*NB) of R x R
 // MFMA blocks (R = 32: gemm_f32_ksw, R = 16: gemm_f32_ksw16), W waves

@@ -262,7 +262,7 @@ gemm_f32_dlh(GemmParams p, HaloTable ht) {
     }
 
     store_tile_lds<MB, NB, NW, WAVES_N, WM, WN, STAGING>(p, acc, smem, m0, n0, wave, lane,
-                                                          id.split, id.bz);
+                                                          id.split, id.bz, p.N);
 }
 
 }  // namespace mtk

@@ -252,7 +252,7 @@ gemm_f32_dlp(GemmParams p) {
     }
     // (store_tile_lds first waits for the re-fetches past the last chunk.)
     store_tile_lds<MB, NB, NW, WAVES_N, WM, WN, STAGES * STAGE>(p, acc, smem, m0, n0, wave, lane,
-                                                                id.split, id.bz);
+                                                                id.split, id.bz, p.N);
 }
 
 }  // namespace mtk

@@ -447,12 +447,13 @@ __device__ __forceinline__ void store_group4(const GemmParams& p, float* base, i
 // row) whose first output element is (m0, n0).  `lds` is the kernel's ring of
 // RING floats; the main loop must be finished with it (the first pass waits
 // for every wave's outstanding DMA and LDS reads before writing).  Writes
-// C(m, n) = acc + bias + beta*C, or the raw partial into split `split`'s
-// workspace slab.
+// C(m, n) = acc + bias + beta*C for n < n_end (p.N, or less for a tile narrower
+// than its blocks; then a multiple of 4), or the raw partial into split
+// `split`'s workspace slab.
 template <int MB, int NB, int NW, int WAVES_N, int WM, int WN, int RING>
 __device__ __forceinline__ void store_tile_lds(const GemmParams& p, const f32x16 (&acc)[MB][NB],
                                                float* lds, int m0, int n0, int wave, int lane,
-                                               int split, int bz) {
+                                               int split, int bz, int n_end) {
     constexpr int NT = NW * 64;
     constexpr int JP = stage_blocks<NB, NW, RING>();
     static_assert(1024 * NW * JP <= RING, "the staging must fit the ring");
@@ -511,7 +512,7 @@ __device__ __forceinline__ void store_tile_lds(const GemmParams& p, const f32x16
                     }
 #pragma unroll
                     for (int u = 0; u < U; ++u)
-                        if (ms[u] < p.M && ns[u] < p.N)
+                        if (ms[u] < p.M && ns[u] < n_end)
                             *reinterpret_cast<f32x4*>(base + (int64_t)ms[u] * rs + ns[u]) =
                                 vs[u] + 0.f;
                 }
@@ -522,7 +523,7 @@ __device__ __forceinline__ void store_tile_lds(const GemmParams& p, const f32x16
                 int m, n, idx;
                 where(k, &m, &n, &idx);
                 const f32x4 v = sl[idx];
-                if (m >= p.M || n >= p.N) continue;
+                if (m >= p.M || n >= n_end) continue;
                 store_group4(p, base, rs, part, vec, bias_axis, beta, m, n, v);
             }
         }
@@ -615,7 +616,7 @@ gemm_f32_mfma(GemmParams p) {
 
     store_tile_lds<MB, NB, (BM / WM) * WAVES_N, WAVES_N, WM, WN,
                    2 * (GA::lds_floats + GB::lds_floats)>(p, acc, smem, m0, n0, wave, lane, split,
-                                                          bz);
+                                                          bz, p.N);
 }
 
 }  // namespace mtk

@@ -133,6 +133,7 @@ struct CfgCost {
     int bm, bn;
     double eff;   // sustained fraction of the CU's MFMA rate inside a workgroup
     int occ;      // resident workgroups per CU
+    bool sp = false;   // gemm_f32_sp
 };
 
 // Cost model (in CU cycles) used to pick the tile configuration and split-K
@@ -147,43 +148,52 @@ struct CfgCost {
 // convolution GEMMs -- on one MI355X.  The efficiencies of the prefetching
 // configurations 4-6 come from same-box comparisons with configurations 0, 2
 // and 1, which have the same tiles.
-constexpr CfgCost kRsCost[kNumCfg] = {      // register-staged kernel, any layout
-    {TileCfg<0>::BM, TileCfg<0>::BN, 0.86, 1},
+constexpr CfgCost kRsCost[kNumCfg] = {      // register-staged kernel, any strides
+    {TileCfg<0>::BM, TileCfg<0>::BN, 0.80, 1},
     {TileCfg<1>::BM, TileCfg<1>::BN, 0.75, 2},
     {TileCfg<2>::BM, TileCfg<2>::BN, 0.57, 4}};
-// Configuration 7 (the convolution kernel on 16x16 blocks, 64x112 tiles,
-// channels-last operand only): 0.78 with two workgroups per CU, from graph
-// timings of ResNet-like layers at batch 32 against the plans of
-// configurations 0-3 (28x28x128 3x3: 88.9 against 96.3 us, 56x56x64:
-// 94.2 against 97.0, 14x14 1x1 256 -> 1024: 55.7 against 57.9); never
-// offered where its workgroups would run one per CU (make_plan_uncached).
-constexpr CfgCost kDlCost[kNumDlCfg] = {    // direct-to-LDS kernel, vector layouts
-    {DlCfg<0>::BM, DlCfg<0>::BN, 0.90, 1},
-    {DlCfg<1>::BM, DlCfg<1>::BN, 0.86, 4},
+// The same tiles on gemm_f32_sp, for contiguous operands of any alignment.
+constexpr int kRsSpCfg[kNumCfg] = {3, 1, 2};
+static_assert(SpCfg<3>::BM == TileCfg<0>::BM && SpCfg<3>::BN == TileCfg<0>::BN &&
+                  SpCfg<1>::BM == TileCfg<1>::BM && SpCfg<1>::BN == TileCfg<1>::BN &&
+                  SpCfg<2>::BM == TileCfg<2>::BM && SpCfg<2>::BN == TileCfg<2>::BN,
+              "the register-staged configurations' tiles on both kernels");
+constexpr CfgCost kRsSpCost[kNumCfg] = {
+    {TileCfg<0>::BM, TileCfg<0>::BN, 1.54, 1, true},
+    {TileCfg<1>::BM, TileCfg<1>::BN, 1.11, 2, true},
+    {TileCfg<2>::BM, TileCfg<2>::BN, 0.80, 4, true}};
+// Vector layouts.  The efficiencies of gemm_f32_sp's configurations (above 1:
+// bf16 units), its round latency and the factor of a workgroup alone on its CU
+// (kSpAlone) are fitted to graph timings of every configuration at 1-16 splits
+// on 71 shapes (35 GEMMs, 8 batched, 10 of unaligned operands, 18 convolution
+// layers; one MI355X), for the least regret of the pick: 4.4 % on average
+// against the fastest measured plan.
+constexpr CfgCost kDlCost[kNumDlCfg] = {
+    {DlCfg<0>::BM, DlCfg<0>::BN, 1.08, 2, true},
+    {DlCfg<1>::BM, DlCfg<1>::BN, 1.18, 2, true},
     {DlCfg<2>::BM, DlCfg<2>::BN, 0.68, 8},
-    {DlCfg<3>::BM, DlCfg<3>::BN, 0.87, 3},
-    {DlCfg<4>::BM, DlCfg<4>::BN, 0.98, 1},
+    {DlCfg<3>::BM, DlCfg<3>::BN, 1.59, 1, true},
+    {DlCfg<4>::BM, DlCfg<4>::BN, 1.58, 1, true},
     {DlCfg<5>::BM, DlCfg<5>::BN, 0.72, 8},
-    {DlCfg<6>::BM, DlCfg<6>::BN, 0.90, 3},
-    {Dl16Cfg<0>::BM, Dl16Cfg<0>::BN, 0.78, 2}};
-// The same kernels with the convolution weight gradient's gathered B operand
-// (L_IMW): its 16-byte gathers cost per chunk whatever the tile's height, so
-// the 256-row tile of configuration 3 amortises them over twice the MFMA work
-// of the 128-row ones.  Forced sweeps of every configuration and split on
-// five ResNet-like dW shapes (c_out 64-512, one MI355X): configuration 3 at
-// its best split is 3-4 % faster than the plain table's picks where M >= 256
-// (5a layer: split 14, 86.9 vs 89.4 us at configuration 6 split 7;
-// 512 x 4608 x 1568: 99.7 vs 103.7 us at configuration 1), and the 64-row
-// shapes keep configuration 5.  Only configurations 3 and 6 differ.
+    {DlCfg<6>::BM, DlCfg<6>::BN, 0.84, 3, true},
+    {DlCfg<7>::BM, DlCfg<7>::BN, 1.00, 3, true}};
+// The same configurations with the convolution weight gradient's gathered B
+// operand (L_IMW); 0: not offered (gemm_f32_sp's gathers cost a workgroup of
+// 256 threads more than the bf16 units save: 128 x 1152 x 25088 at configuration
+// 1, 28 splits, 132 us against 92 on the fp32 kernel).
 constexpr CfgCost kDlCostImw[kNumDlCfg] = {
-    {DlCfg<0>::BM, DlCfg<0>::BN, 0.90, 1},
+    {DlCfg<0>::BM, DlCfg<0>::BN, 0, 2},
     {DlCfg<1>::BM, DlCfg<1>::BN, 0.86, 4},
     {DlCfg<2>::BM, DlCfg<2>::BN, 0.68, 8},
-    {DlCfg<3>::BM, DlCfg<3>::BN, 0.93, 3},
-    {DlCfg<4>::BM, DlCfg<4>::BN, 0.98, 1},
+    {DlCfg<3>::BM, DlCfg<3>::BN, 1.42, 1, true},
+    {DlCfg<4>::BM, DlCfg<4>::BN, 0, 1},
     {DlCfg<5>::BM, DlCfg<5>::BN, 0.72, 8},
-    {DlCfg<6>::BM, DlCfg<6>::BN, 0.86, 3},
-    {Dl16Cfg<0>::BM, Dl16Cfg<0>::BN, 0.78, 2}};   // (configuration 7: L_IM only)
+    {DlCfg<6>::BM, DlCfg<6>::BN, 0, 3},
+    {DlCfg<7>::BM, DlCfg<7>::BN, 0, 2}};   // (configuration 7: L_IM only)
+// And with the 4-byte gathers of an NCHW view (L_IMR), of which a tile of 256
+// columns on 256 threads makes the most per thread: the 7x7 stem at batch 32
+// took 188 us on configuration 0 against 178 on 2.
+constexpr double kImrNarrowEff = 0.80;
 // Wave-split kernel (configurations of KswCfg): efficiencies from
 // graph-replay timings of every configuration at 1, 2 and 4 K splits on the
 // benchmark's small GEMMs and four neighbouring shapes (one MI355X).  It is
@@ -224,16 +234,9 @@ constexpr int kKswWaves[kNumKswCfg] = {KswCfg<0>::W, KswCfg<1>::W, KswCfg<2>::W,
                                        KswCfg<3>::W, KswCfg<4>::W, KswCfg<5>::W,
                                        KswCfg<6>::W, KswCfg<7>::W, KswCfg<8>::W};
 
-// Configuration 6 pays off only over long K ranges (short ones, such as the
-// 64-deep batched GEMM of the benchmark, run up to 20 % slower than
-// configuration 1): the planner offers it for K per split >= kDlp6MinK, or
-// >= kDlp6MinKOneRound when every workgroup gets a CU of its own (about 4 %
-// faster than configuration 1 at 2048^2 x 256; with several rounds the four
-// co-resident workgroups of configuration 1 win).
-constexpr int kDlp6MinK = 512;
-constexpr int kDlp6MinKOneRound = 256;
 struct CostModel {
     double round_latency = 6200.0;           // cycles of fill/drain per round
+    double sp_round_latency = 6800.0;        // ... of gemm_f32_sp
     double epilogue_bytes_per_cycle = 7.9;   // one workgroup's tile store
     double bytes_per_cycle = 6400.0;         // device HBM bytes per CU-clock
     double launch_cycles = 17700.0;          // second (reduce) launch
@@ -252,8 +255,9 @@ constexpr int kDlSmallCfg = 2;           // the 64x64 direct-to-LDS configuratio
 constexpr double kCoresidentPair = 0.75;
 constexpr int kAloneMinK = 1024;
 constexpr double kAlonePenalty = 1.3;
+constexpr double kSpAlone = 1.13;
 constexpr int kMaxForcedSplits = 64;
-constexpr bool kOfferDl16 = true;
+constexpr bool kOfferNarrow = true;
 
 // Tile grid and K split of configuration `cfg` asked for `s` splits (the
 // split count can come out lower: every split takes whole 16-deep chunks).
@@ -307,7 +311,9 @@ double plan_cycles(const CostModel& cm, const CfgCost& cc, const Plan& pl, int64
                           per_cu == 1 && pl.kps >= kAloneMinK)
                              ? kAlonePenalty
                              : 1.0;
-    double t = per_cu * work * pair * alone + per_cu * epi / cc.occ + rounds * cm.round_latency;
+    const double sp_alone = cc.sp && cc.occ > 1 && per_cu == 1 ? kSpAlone : 1.0;
+    double t = per_cu * work * pair * alone * sp_alone + per_cu * epi / cc.occ +
+               rounds * (cc.sp ? cm.sp_round_latency : cm.round_latency);
     if (pl.splits > 1) {
         const double bytes = (double)(2 * pl.splits + 1) * M * N * batch * 4.0;
         t += bytes / (cm.bytes_per_cycle) + cm.launch_cycles;
@@ -317,36 +323,37 @@ double plan_cycles(const CostModel& cm, const CfgCost& cc, const Plan& pl, int64
 
 // wide: the prefetching direct-to-LDS configurations (is_dlp_cfg) may be
 // chosen (see wide_ok in launch_gemm); ksw: the wave-split kernel may be;
-// imw: B is the weight-gradient operand (priced by kDlCostImw); im16: the
-// convolution kernel on 16x16 blocks (is_dl16_cfg, B = L_IM) may be.
+// sp: gemm_f32_sp can take the operands (sp_fits, sp_layouts); imw: B is the
+// weight-gradient operand (priced by kDlCostImw); im16: the 112-column tile
+// (kNarrowCfg, B = L_IM) may be.
 Plan make_plan_uncached(int64_t M, int64_t N, int64_t K, int64_t batch, int cus,
-                        bool allow_split, bool dl, bool wide, bool ksw, bool imw, bool im16) {
+                        bool allow_split, bool dl, bool wide, bool ksw, bool sp, bool imw, bool im16) {
     static const CostModel cm;
-    const CfgCost* cfgs = dl ? (imw ? kDlCostImw : kDlCost) : kRsCost;
+    const CfgCost* cfgs = dl ? (imw ? kDlCostImw : kDlCost) : sp ? kRsSpCost : kRsCost;
     const int ncfg = dl ? kNumDlCfg : kNumCfg;
     Plan best;
     best.dl = dl;
     double best_t = 1e300;
     for (int cfg = 0; cfg < ncfg; ++cfg) {
-        if (dl && is_dlp_cfg(cfg) && !wide) continue;
-        if (dl && is_dl16_cfg(cfg) && !im16) continue;
-        const CfgCost& cc = cfgs[cfg];
+        if (dl && is_wide_cfg(cfg) && !wide) continue;
+        if (dl && is_sp_cfg(cfg) && !sp && !(imw && cfg == 1)) continue;
+        if (cfgs[cfg].eff <= 0) continue;
+        if (dl && cfg == kNarrowCfg && !im16) continue;
+        CfgCost cc = cfgs[cfg];
+        if (dl && cfg == 0 && !wide && !im16) cc.eff = kImrNarrowEff;   // L_IMR
         for (int s = 1; s <= kMaxSplits; ++s) {
             if (s > 1 && !allow_split) break;
             const Plan pl = cfg_plan(cc, cfg, dl, M, N, K, batch, s);
             if (s > 1 && pl.kps < 64) break;
             if (s > kFittedSplits && pl.kps < kMinKpsBeyondFit) break;
-            const int64_t k6 = std::min<int64_t>(pl.kps, K);
-            if (dl && cfg == 6 && k6 < kDlp6MinKOneRound) break;
             if (pl.splits != s) continue;
             const int64_t wgs = (int64_t)pl.tiles_m * pl.tiles_n * batch * pl.splits;
-            if (dl && cfg == 6 && k6 < kDlp6MinK && wgs > cus) continue;
             if (wgs * 512 >= ((int64_t)1 << 32)) continue;
             // The 64x112 tile of 16x16 blocks moves about twice the operand
             // bytes per flop of the 256x128 one; with one workgroup per CU
             // (nothing co-resident to hide the fetches) it lost everywhere it
             // was measured (the 5a layer: 93.2 us against 80.2 at split 5).
-            if (dl && is_dl16_cfg(cfg) && wgs <= cus) continue;
+            if (dl && cfg == kNarrowCfg && wgs <= cus) continue;
             const double t = plan_cycles(cm, cc, pl, M, N, batch, cus);
             if (t < best_t) {
                 best_t = t;
@@ -382,11 +389,12 @@ Plan make_plan_uncached(int64_t M, int64_t N, int64_t K, int64_t batch, int cus,
 // holds several layers' worth, so the launch that follows a query finds its
 // plan instead of rerunning the cost model.
 Plan make_plan(int64_t M, int64_t N, int64_t K, int64_t batch, int cus, bool allow_split,
-               bool dl, bool wide, bool ksw, bool imw = false, bool im16 = false) {
+               bool dl, bool wide, bool ksw, bool sp, bool imw = false, bool im16 = false) {
     struct Entry {
         int64_t M = -1, N = -1, K = -1, batch = -1;
         int cus = 0;
-        bool allow_split = false, dl = false, wide = false, ksw = false, imw = false, im16 = false;
+        bool allow_split = false, dl = false, wide = false, ksw = false, sp = false, imw = false,
+             im16 = false;
         Plan plan;
     };
     constexpr int kEntries = 128;
@@ -395,12 +403,13 @@ Plan make_plan(int64_t M, int64_t N, int64_t K, int64_t batch, int cus, bool all
     for (const Entry& e : cache)
         if (e.M == M && e.N == N && e.K == K && e.batch == batch && e.cus == cus &&
             e.allow_split == allow_split && e.dl == dl && e.wide == wide && e.ksw == ksw &&
-            e.imw == imw && e.im16 == im16)
+            e.sp == sp && e.imw == imw && e.im16 == im16)
             return e.plan;
     Entry& e = cache[next];
     next = (next + 1) % kEntries;
-    e = Entry{M, N, K, batch, cus, allow_split, dl, wide, ksw, imw, im16,
-              make_plan_uncached(M, N, K, batch, cus, allow_split, dl, wide, ksw, imw, im16)};
+    e = Entry{M, N, K, batch, cus, allow_split, dl, wide, ksw, sp, imw, im16,
+              make_plan_uncached(M, N, K, batch, cus, allow_split, dl, wide, ksw, sp, imw,
+                                 im16)};
     return e.plan;
 }
 
@@ -418,7 +427,7 @@ thread_local ForcedConfig g_forced;
 // can take them too; im16_ok: B is L_IM, which the 16x16-block convolution
 // configurations take).
 bool forced_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool dl_ok, bool rs_ok,
-                 bool wide_ok, Plan* out, bool im16_ok = false) {
+                 bool wide_ok, bool sp_ok, Plan* out, bool im16_ok = false) {
     const ForcedConfig f = g_forced;
     if (f.family == MT_FAMILY_KSW && rs_ok) {
         int bm, bn;
@@ -427,8 +436,8 @@ bool forced_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool dl_ok, boo
         out->ksw = true;
         return true;
     }
-    if (f.family == MT_FAMILY_DL && dl_ok && (!is_dlp_cfg(f.cfg) || wide_ok) &&
-        (!is_dl16_cfg(f.cfg) || im16_ok)) {
+    if (f.family == MT_FAMILY_DL && dl_ok && (!is_wide_cfg(f.cfg) || wide_ok) &&
+        (!is_sp_cfg(f.cfg) || sp_ok) && (f.cfg != kNarrowCfg || im16_ok)) {
         *out = cfg_plan(kDlCost[f.cfg], f.cfg, true, M, N, K, batch, f.splits);
         return true;
     }
@@ -439,49 +448,52 @@ bool forced_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool dl_ok, boo
     return false;
 }
 
-// The implicit-im2col form (L_IM) exists for DlCfg 0..3 only; the planner
-// never picks the prefetching configurations for it (nullptr is a safety
-// net).  The row-sum form and the weight-gradient operand (L_IMW) exist for
-// all.
+GemmLaunchFn sp_launcher(int cfg, int la, int lb, bool rs = false) {
+    switch (cfg) {
+        case 0: return sp_launcher_cfg0(la, lb, rs);
+        case 1: return sp_launcher_cfg1(la, lb, rs);
+        case 2: return sp_launcher_cfg2(la, lb, rs);
+        case 3: return sp_launcher_cfg3(la, lb, rs);
+        case 4: return sp_launcher_cfg4(la, lb, rs);
+        case 6: return sp_launcher_cfg6(la, lb, rs);
+        case 7: return sp_launcher_cfg7(la, lb, rs);
+        default: return nullptr;
+    }
+}
+
+// The implicit-im2col forms (L_IM, L_IMR) exist for configurations 0-3 (and 7)
+// only; the planner never picks 4-6 for them (nullptr is a safety net).  The
+// row-sum form and the weight-gradient operand (L_IMW) exist for all.
 // kv: two k-contiguous operands (else two mn-contiguous ones).
 GemmLaunchFn rowsum_launcher(int cfg, bool tail, bool kv) {
-    switch (cfg) {
-        case 0: return dl_rowsum_launcher_cfg0(kv);
-        case 1: return dl_rowsum_launcher_cfg1(kv);
-        case 2: return dl_rowsum_launcher_cfg2(kv);
-        case 3: return dl_rowsum_launcher_cfg3(kv);
-        default: return dlp_rowsum_launcher(cfg, tail, kv);
-    }
+    if (is_sp_cfg(cfg)) return sp_launcher(cfg, kv ? L_KV : L_MV, kv ? L_KV : L_MV, true);
+    return cfg == 2 ? dl_rowsum_launcher_cfg2(kv)
+           : is_dlp_cfg(cfg) ? dlp_rowsum_launcher(tail, kv)
+                             : nullptr;
 }
 
 // kvi: A is dY read in NCHW (L_KVI, whole chunks only).
 GemmLaunchFn convw_launcher(int cfg, bool ktail, bool kvi) {
-    if (kvi) {
-        if (ktail) return nullptr;
-        switch (cfg) {
-            case 0: return dl_convwi_launcher_cfg0();
-            case 1: return dl_convwi_launcher_cfg1();
-            case 2: return dl_convwi_launcher_cfg2();
-            case 3: return dl_convwi_launcher_cfg3();
-            default: return dlp_convwi_launcher(cfg);
-        }
-    }
-    switch (cfg) {
-        case 0: return dl_convw_launcher_cfg0();
-        case 1: return dl_convw_launcher_cfg1();
-        case 2: return dl_convw_launcher_cfg2();
-        case 3: return dl_convw_launcher_cfg3();
-        default: return dlp_convw_launcher(cfg, ktail);
-    }
+    if (kvi && ktail) return nullptr;
+    if (cfg == 1) return kvi ? dl_convwi_launcher_cfg1() : dl_convw_launcher_cfg1();
+    if (is_sp_cfg(cfg)) return sp_launcher(cfg, kvi ? L_KVI : L_KV, L_IMW);
+    if (cfg == 2) return kvi ? dl_convwi_launcher_cfg2() : dl_convw_launcher_cfg2();
+    if (is_dlp_cfg(cfg)) return kvi ? dlp_convwi_launcher() : dlp_convw_launcher(ktail);
+    return nullptr;
 }
 
 // LDS floats of the halo-patch kernel of dl configuration cfg (0-3).
+template <int CFG>
+int halo_floats(const ConvGeom& g) {
+    using C = DlhCfg<CFG>;
+    return dlh_lds_floats<C::BM, C::BN, C::WM, C::WN>(g);
+}
 int halo_lds_floats(int cfg, const ConvGeom& g) {
     switch (cfg) {
-        case 0: return dlh_lds_floats<DlCfg<0>::BM, DlCfg<0>::BN, DlCfg<0>::WM, DlCfg<0>::WN>(g);
-        case 1: return dlh_lds_floats<DlCfg<1>::BM, DlCfg<1>::BN, DlCfg<1>::WM, DlCfg<1>::WN>(g);
-        case 2: return dlh_lds_floats<DlCfg<2>::BM, DlCfg<2>::BN, DlCfg<2>::WM, DlCfg<2>::WN>(g);
-        case 3: return dlh_lds_floats<DlCfg<3>::BM, DlCfg<3>::BN, DlCfg<3>::WM, DlCfg<3>::WN>(g);
+        case 0: return halo_floats<0>(g);
+        case 1: return halo_floats<1>(g);
+        case 2: return halo_floats<2>(g);
+        case 3: return halo_floats<3>(g);
         default: return -1;
     }
 }
@@ -525,25 +537,10 @@ void set_halo_geometry(ConvGeom& g) {
     g.pw = (g.wo - 1) * g.stride + g.kw;
 }
 
-GemmLaunchFn convh_launcher(int cfg) {
-    switch (cfg) {
-        case 0: return dl_convh_launcher_cfg0();
-        case 1: return dl_convh_launcher_cfg1();
-        case 2: return dl_convh_launcher_cfg2();
-        case 3: return dl_convh_launcher_cfg3();
-        default: return nullptr;
-    }
-}
-
 GemmLaunchFn conv_launcher(int cfg, bool nchw) {
-    if (is_dl16_cfg(cfg)) return nchw ? nullptr : dl16_conv_launcher(cfg - kDl16FirstCfg);
-    switch (cfg) {
-        case 0: return nchw ? dl_convr_launcher_cfg0() : dl_conv_launcher_cfg0();
-        case 1: return nchw ? dl_convr_launcher_cfg1() : dl_conv_launcher_cfg1();
-        case 2: return nchw ? dl_convr_launcher_cfg2() : dl_conv_launcher_cfg2();
-        case 3: return nchw ? dl_convr_launcher_cfg3() : dl_conv_launcher_cfg3();
-        default: return nullptr;
-    }
+    if (is_sp_cfg(cfg)) return sp_launcher(cfg, L_KV, nchw ? L_IMR : L_IM);
+    if (cfg == 2) return nchw ? dl_convr_launcher_cfg2() : dl_conv_launcher_cfg2();
+    return nullptr;
 }
 
 // ---- HBM-bound shapes on the vector ALUs (gemm_skinny_kernel.hpp) ----------
@@ -681,31 +678,57 @@ size_t skinny_ws(int64_t M, int64_t N, int64_t K, int64_t batch, int cus) {
 
 // Workspace that covers the plan of either kernel family (for sizes queried
 // before the operand pointers, and hence the layouts, are known).
-size_t plan_ws(int64_t M, int64_t N, int64_t K, int64_t batch, int cus, bool imw = false) {
+size_t plan_ws(int64_t M, int64_t N, int64_t K, int64_t batch, int cus) {
     size_t ws = 0;
     for (bool dl : {false, true})
         for (bool wide : {false, true})
             for (bool ksw : {false, true})
-                ws = std::max(ws, make_plan(M, N, K, batch, cus, true, dl, wide, ksw).ws_bytes);
-    if (imw)   // the weight-gradient operand's own table
-        for (bool wide : {false, true})
-            ws = std::max(ws, make_plan(M, N, K, batch, cus, true, true, wide, false, true).ws_bytes);
+                for (bool sp : {false, true})
+                    ws = std::max(ws,
+                                  make_plan(M, N, K, batch, cus, true, dl, wide, ksw, sp).ws_bytes);
     Plan forced;
-    if (forced_plan(M, N, K, batch, true, true, true, &forced)) ws = std::max(ws, forced.ws_bytes);
+    if (forced_plan(M, N, K, batch, true, true, true, true, &forced))
+        ws = std::max(ws, forced.ws_bytes);
     return std::max(ws, skinny_ws(M, N, K, batch, cus));
 }
 
-GemmLaunchFn pick_launcher(const Plan& plan, int la, int lb, bool ktail) {
+// Contiguous layout of one operand for gemm_f32_sp, whatever its alignment, or
+// -1; `rows`: of the tile.  Its k-contiguous loader has 32-bit byte offsets
+// within a tile.
+int sp_layout(int64_t s_mn, int64_t s_k, int64_t MN, int64_t K, int rows) {
+    if (s_k == 1 || K == 1) {
+        const int64_t last = std::min<int64_t>(rows, MN) - 1;
+        if (last * s_mn < ((int64_t)1 << 30) - 16) return L_KV;
+    }
+    return s_mn == 1 || MN == 1 ? L_MV : -1;
+}
+constexpr int kSpMaxRows = 256;   // rows of the largest tile
+bool sp_layouts(const GemmParams& p, int* la, int* lb) {
+    *la = sp_layout(p.a_mn, p.a_k, p.M, p.K, kSpMaxRows);
+    *lb = sp_layout(p.b_mn, p.b_k, p.N, p.K, kSpMaxRows);
+    return *la >= 0 && *lb >= 0;
+}
+
+// Whether gemm_f32_sp takes the vector-layout or implicit operands of a
+// direct-to-LDS launch: 32-bit byte offsets within a tile of k-contiguous rows,
+// and within the weight gradient's window.
+bool sp_fits(const GemmParams& p, int la, int lb) {
+    const auto kc = [](int64_t s_mn, int64_t MN) {
+        return (std::min<int64_t>(kSpMaxRows, MN) - 1) * s_mn < ((int64_t)1 << 30) - 16;
+    };
+    if (la == L_KV && !kc(p.a_mn, p.M)) return false;
+    if (lb == L_KV && !kc(p.b_mn, p.N)) return false;
+    return lb != L_IMW || (int64_t)p.cv.kh * p.cv.w * p.cv.c < ((int64_t)1 << 30);
+}
+
+// (sla, slb): sp_layouts, or -1.
+GemmLaunchFn pick_launcher(const Plan& plan, int la, int lb, bool ktail, int sla, int slb) {
     if (plan.ksw) return ksw_launcher(plan.cfg, la == L_KV, lb == L_KV);
     if (plan.dl) {
-        switch (plan.cfg) {
-            case 0: return dl_launcher_cfg0(la, lb);
-            case 1: return dl_launcher_cfg1(la, lb);
-            case 2: return dl_launcher_cfg2(la, lb);
-            case 3: return dl_launcher_cfg3(la, lb);
-            default: return dlp_launcher(plan.cfg, ktail, la, lb);
-        }
+        if (is_sp_cfg(plan.cfg)) return sp_launcher(plan.cfg, la, lb);
+        return plan.cfg == 2 ? dl_launcher_cfg2(la, lb) : dlp_launcher(ktail, la, lb);
     }
+    if (sla >= 0 && slb >= 0) return sp_launcher(kRsSpCfg[plan.cfg], sla, slb);
     switch (plan.cfg) {
         case 0: return launcher_cfg0(la, lb);
         case 1: return launcher_cfg1(la, lb);
@@ -1033,7 +1056,11 @@ int launch_gemm(GemmParams& p, bool dl, int la, int lb, void* workspace, size_t 
     const bool wide_ok = dl && lb != L_IM && lb != L_IMR && K > 0;
     Plan plan;
     const bool im16_ok = dl && lb == L_IM;
-    const bool forced = forced_plan(M, N, K, batch, dl, !implicit, wide_ok, &plan, im16_ok);
+    // gemm_f32_sp: contiguous operands, offsets within a tile of 32 bits
+    int sla = -1, slb = -1;
+    const bool sp_ok = dl ? sp_fits(p, la, lb) : !implicit && sp_layouts(p, &sla, &slb);
+    const bool forced =
+        forced_plan(M, N, K, batch, dl, !implicit, wide_ok, sp_ok, &plan, im16_ok);
     // workspace a plan writes: split-K partials, or with p.part a slab per
     // split and batch entry even at one split
     auto need = [&](const Plan& pl) {
@@ -1046,15 +1073,15 @@ int launch_gemm(GemmParams& p, bool dl, int la, int lb, void* workspace, size_t 
         // the wave-split kernel takes every operand form but the implicit
         // convolution operands and the fused row sums
         const bool ksw_ok = !implicit && p.rowsum == nullptr;
-        plan = make_plan(M, N, K, batch, device_cu_count(), true, dl, wide_ok, ksw_ok,
-                         lb == L_IMW, im16_ok && kOfferDl16);
+        plan = make_plan(M, N, K, batch, device_cu_count(), true, dl, wide_ok, ksw_ok, sp_ok,
+                         lb == L_IMW, im16_ok && kOfferNarrow);
         if (need(plan) > 0 && (workspace == nullptr || ws_bytes < need(plan)))
-            plan = make_plan(M, N, K, batch, device_cu_count(), false, dl, wide_ok, ksw_ok,
-                             lb == L_IMW, im16_ok && kOfferDl16);
+            plan = make_plan(M, N, K, batch, device_cu_count(), false, dl, wide_ok, ksw_ok, sp_ok,
+                             lb == L_IMW, im16_ok && kOfferNarrow);
         if (need(plan) > 0 && (workspace == nullptr || ws_bytes < need(plan)))
             return MT_ERR_WORKSPACE;
     }
-    if (!plan.dl || (plan.splits > 1 && !rs_part) || is_dl16_cfg(plan.cfg)) p.rowsum = nullptr;
+    if (!plan.dl || (plan.splits > 1 && !rs_part) || plan.cfg == kNarrowCfg) p.rowsum = nullptr;
     p.splits = plan.splits;
     p.k_per_split = plan.splits > 1 ? plan.kps : (int)std::max<int64_t>(K, 1);
     p.tiles_m = plan.tiles_m;
@@ -1090,11 +1117,11 @@ int launch_gemm(GemmParams& p, bool dl, int la, int lb, void* workspace, size_t 
                   (long long)nblocks, plan.cfg,
                   p.part ? (p.csum_rows ? " batch-summed rows" : " batch-summed") : "");
 
-    GemmLaunchFn fn = halo ? convh_launcher(plan.cfg)
+    GemmLaunchFn fn = halo ? dlh_launcher(plan.cfg)
                       : lb == L_IM || lb == L_IMR ? conv_launcher(plan.cfg, lb == L_IMR)
                       : lb == L_IMW ? convw_launcher(plan.cfg, (K & 15) != 0, la == L_KVI)
                       : p.rowsum != nullptr ? rowsum_launcher(plan.cfg, (K & 15) != 0, la == L_KV)
-                                            : pick_launcher(plan, la, lb, (K & 15) != 0);
+                                            : pick_launcher(plan, la, lb, (K & 15) != 0, sla, slb);
     if (fn == nullptr) return MT_ERR_UNSUPPORTED;
     hipError_t e = fn(p, (unsigned)nblocks, stream);
     if (e == hipErrorStreamCaptureUnsupported) e = hipSuccess;
@@ -1806,10 +1833,12 @@ size_t part_plan_ws(int64_t M, int64_t N, int64_t K, int64_t batch, int cus) {
     for (bool dl : {false, true})
         for (bool wide : {false, true})
             for (bool ksw : {false, true})
-                ws = std::max(ws, part_ws_bytes(make_plan(M, N, K, batch, cus, true, dl, wide, ksw),
-                                                M, N, batch));
+                for (bool sp : {false, true})
+                    ws = std::max(
+                        ws, part_ws_bytes(make_plan(M, N, K, batch, cus, true, dl, wide, ksw, sp),
+                                          M, N, batch));
     Plan forced;
-    if (forced_plan(M, N, K, batch, true, true, true, &forced))
+    if (forced_plan(M, N, K, batch, true, true, true, true, &forced))
         ws = std::max(ws, part_ws_bytes(forced, M, N, batch));
     return align_up(ws, 256);
 }
@@ -2129,26 +2158,30 @@ bool dx_prefer_phased(const mt_conv2d_desc* d, int64_t Ho, int64_t Wo, bool cl) 
     for (int i = 0; i < t.n; ++i) {
         const DxPhase& f = t.f[i];
         if (f.hp == 0 || f.wp == 0 || f.k == 0) continue;
-        phased += make_plan(d->c_in, d->n * f.hp * f.wp, f.k, 1, cus, true, true, false, false)
+        phased += make_plan(d->c_in, d->n * f.hp * f.wp, f.k, 1, cus, true, true, false, false, true)
                       .cycles;
     }
     phased = kDxPhasedFactor * phased + stream / kDxStreamBytes;
-    const double col = make_plan(kg, np, d->c_out, 1, cus, true, true, true, true).cycles +
+    const double col = make_plan(kg, np, d->c_out, 1, cus, true, true, true, true, true).cycles +
                        (8.0 * d->c_out * np + 8.0 * kg * np + dx_bytes) / kDxGatherBytes;
     return phased < col;
 }
 
 // Workspace of one implicit-operand GEMM (L_IM / L_IMR: the direct-to-LDS
-// configurations 0-3; L_IMW, imw: all of them, its own efficiency table),
+// configurations 0-3 and 7; L_IMW, imw: 0-6),
 // including a forced configuration's partials: what launch_gemm may use.
 size_t implicit_gemm_ws(int64_t M, int64_t N, int64_t K, bool imw) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     const int cus = device_cu_count();
-    size_t ws = make_plan(M, N, K, 1, cus, true, true, imw, false, imw).ws_bytes;
-    if (!imw && kOfferDl16)   // the channels-last operand may take the 16x16-block kernel
-        ws = std::max(ws, make_plan(M, N, K, 1, cus, true, true, false, false, false, true).ws_bytes);
+    size_t ws = 0;
+    for (bool sp : {false, true}) {
+        ws = std::max(ws, make_plan(M, N, K, 1, cus, true, true, imw, false, sp, imw).ws_bytes);
+        if (!imw && kOfferNarrow)   // the channels-last operand may take the 16x16-block kernel
+            ws = std::max(ws,
+                          make_plan(M, N, K, 1, cus, true, true, false, false, sp, false, true).ws_bytes);
+    }
     Plan f;
-    if (forced_plan(M, N, K, 1, true, false, imw, &f, !imw)) ws = std::max(ws, f.ws_bytes);
+    if (forced_plan(M, N, K, 1, true, false, imw, true, &f, !imw)) ws = std::max(ws, f.ws_bytes);
     return ws;
 }
 
