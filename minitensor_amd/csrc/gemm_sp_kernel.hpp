@@ -466,15 +466,27 @@ gemm_f32_sp(GemmParams p) {
             put(buf, xa, IA{}, std::integral_constant<int, BM>{});
             put(buf + 3 * sp_plane<BM>(), xb, IB{}, std::integral_constant<int, BN>{});
         };
+        // The last product (h·l) of a chunk is left for the next step, which
+        // issues it between its barrier and the arrival of its fragments.
+        SplitFrag fa[MB], fb[NB];
+#pragma unroll
+        for (int i = 0; i < MB; ++i) fa[i].h = u32x4{0, 0, 0, 0};
+#pragma unroll
+        for (int j = 0; j < NB; ++j) fb[j].l = u32x4{0, 0, 0, 0};
         auto multiply = [&](int kt) {
             const char* const buf = smem + (kt & 1) * BUF;
-            SplitFrag fa[MB], fb[NB];
+            SplitFrag na[MB], nb[NB];
 #pragma unroll
-            for (int i = 0; i < MB; ++i) sp_frag<BM>(buf, ra + 32 * i + lrow, half, fa[i]);
+            for (int i = 0; i < MB; ++i) sp_frag<BM>(buf, ra + 32 * i + lrow, half, na[i]);
 #pragma unroll
             for (int j = 0; j < NB; ++j)
-                sp_frag<BN>(buf + 3 * sp_plane<BM>(), rb + 32 * j + lrow, half, fb[j]);
-            mfma_split_chunk<MB, NB>(acc, sml, fa, fb);
+                sp_frag<BN>(buf + 3 * sp_plane<BM>(), rb + 32 * j + lrow, half, nb[j]);
+            mfma_split<MB, NB, 5, 6>(acc, sml, fa, fb);
+            mfma_split<MB, NB, 0, 5>(acc, sml, na, nb);
+#pragma unroll
+            for (int i = 0; i < MB; ++i) fa[i].h = na[i].h;
+#pragma unroll
+            for (int j = 0; j < NB; ++j) fb[j].l = nb[j].l;
         };
         // Chunk kt out of LDS; xa / xb hold chunk kt+1, ya / yb take chunk
         // kt+2.  The barrier: every wave's part of chunk kt is in LDS, and its
@@ -493,11 +505,20 @@ gemm_f32_sp(GemmParams p) {
             __builtin_amdgcn_sched_barrier(0);   // not behind the MFMAs
             multiply(kt);
             cut(kt + 1, xa, xb);
-            // four vector instructions beside each MFMA
+            // The fragment reads under the first MFMAs (read where they are used,
+            // as the compiler had it, each exposed its latency: 3-4 % of the
+            // kernel), then the cutting, whose values have had that much longer
+            // to arrive, spread over the other MFMAs.
+            constexpr int NM = 6 * MB * NB, NR = 3 * (MB + NB), NP = MB * NB;
+            constexpr int WORK = ((BM + BN) * 16 / NT * 13 / 2 + 16) / (NM - NP) + 1;
+            constexpr int MOST = LB == L_IMR ? 5 : 6;   // (its addresses take registers)
+            constexpr int NV = WORK < MOST ? WORK : MOST;
+            __builtin_amdgcn_sched_group_barrier(0x100, MB + NB, 0);
 #pragma unroll
-            for (int g = 0; g < 6 * MB * NB; ++g) {
+            for (int g = 0; g < NM; ++g) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+                if (MB + NB + 2 * g < NR) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+                if (g >= NP) __builtin_amdgcn_sched_group_barrier(0x002, NV, 0);
             }
         };
         f32x4 xa[IA::NI], xb[IB::NI], ya[IA::NI], yb[IB::NI];
@@ -522,6 +543,7 @@ gemm_f32_sp(GemmParams p) {
             if (kt + 1 < nk) step(kt, ya, yb, xa, xb);
             sp_barrier();
             multiply(nk - 1);
+            mfma_split<MB, NB, 5, 6>(acc, sml, fa, fb);
         }
         if (split_finish<MB, NB>(acc, sml)) bad = 1;
     }

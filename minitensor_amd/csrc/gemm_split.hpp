@@ -84,14 +84,13 @@ __device__ __forceinline__ f32x16 mfma_bf16(const u32x4& a, const u32x4& b, cons
                                                    __builtin_bit_cast(bf16x8, a), c, 0, 0, 0);
 }
 
-// One 16-deep chunk: acc + sml += A·B at the scale of 2^48; consecutive MFMAs
-// feed different accumulators.
-template <int MB, int NB>
-__device__ __forceinline__ void mfma_split_chunk(f32x16 (&acc)[MB][NB], f32x16 (&sml)[MB][NB],
-                                                 const SplitFrag (&a)[MB],
-                                                 const SplitFrag (&b)[NB]) {
+// Products P0..P1-1 (of six) of one 16-deep chunk: acc + sml += A·B at the scale
+// of 2^48; consecutive MFMAs feed different accumulators.
+template <int MB, int NB, int P0, int P1>
+__device__ __forceinline__ void mfma_split(f32x16 (&acc)[MB][NB], f32x16 (&sml)[MB][NB],
+                                           const SplitFrag (&a)[MB], const SplitFrag (&b)[NB]) {
 #pragma unroll
-    for (int p = 0; p < 6; ++p)
+    for (int p = P0; p < P1; ++p)
 #pragma unroll
         for (int i = 0; i < MB; ++i)
 #pragma unroll
