@@ -3,7 +3,8 @@
 The product is the C-ABI library ``minitensor_amd/lib/libmtgemm.so`` (declared in
 ``include/mtgemm.h``) and the header-only C++20 host layer in
 ``minitensor_amd/cpp``.  This module binds the same C ABI from Python with
-ctypes; torch is used only for device memory and streams.  There is no CPU or
+ctypes, and its plain calls through a small torch extension (_native.so); torch
+is used only for device memory and streams.  There is no CPU or
 library fallback: every call goes through the HIP kernels, and a missing
 library raises.
 
@@ -137,6 +138,24 @@ def lib() -> ctypes.CDLL:
     return _lib_handle
 
 
+_native_handle = None
+
+
+def native():
+    """The torch binding (_native.so), which takes the plain calls from tensors
+    to the C ABI in one step; raises if it has not been built."""
+    global _native_handle
+    if _native_handle is None:
+        lib()
+        path = _PKG / "_native.so"
+        if not path.exists():
+            raise RuntimeError(
+                f"{path} is missing: build it with `python -m minitensor_amd.build`")
+        from . import _native
+        _native_handle = _native
+    return _native_handle
+
+
 def _check(rc: int, what: str) -> None:
     if rc == MT_OK:
         return
@@ -171,6 +190,10 @@ def mat(t: torch.Tensor) -> MatF32:
     return MatF32(base, t.storage_offset(), rows, cols, rs, cs, batch, bs)
 
 
+def _handle(stream) -> Optional[int]:
+    return None if stream is None else stream.cuda_stream
+
+
 def _stream(stream=None) -> int:
     s = stream if stream is not None else torch.cuda.current_stream()
     return s.cuda_stream
@@ -196,6 +219,8 @@ def _api(fn):
     @functools.wraps(fn)
     def wrapper(*args, **kwargs):
         stream = args[pos] if len(args) > pos else kwargs.get("stream")
+        if stream is None:
+            return fn(*args, **kwargs)
         with _on(stream):
             return fn(*args, **kwargs)
     return wrapper
@@ -216,6 +241,9 @@ def gemm(A: torch.Tensor, B: torch.Tensor, out: Optional[torch.Tensor] = None,
          bias: Optional[torch.Tensor] = None, bias_axis: int = BIAS_NONE, beta: float = 0.0,
          ws: Optional[torch.Tensor] = None, stream=None) -> torch.Tensor:
     """C = A·B (+bias) (+beta·C) on the GPU through mt_gemm_f32; views are read in place."""
+    r = native().gemm(A, B, out, bias, bias_axis, beta, ws, _handle(stream))
+    if r is not None:
+        return r
     _require_gpu(A, B, out, bias)
     if A.dim() != B.dim() or A.dim() not in (2, 3):
         raise ValueError("gemm: A and B must both be 2-D or both 3-D")
@@ -271,6 +299,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None,
            out: Optional[torch.Tensor] = None, ws: Optional[torch.Tensor] = None,
            stream=None) -> torch.Tensor:
     """F::linear: y = x·wᵀ + b with w [out,in] (bias fused in the GEMM epilogue)."""
+    r = native().linear(x, w, b, out, ws, _handle(stream))
+    if r is not None:
+        return r
     _require_gpu(x, w, b, out)
     if x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1]:
         raise ValueError("linear: expected x [B,in] and w [out,in]")
@@ -292,6 +323,10 @@ def linear_backward(dy: torch.Tensor, x: torch.Tensor, w: torch.Tensor, need_dx:
                     need_dw: bool = True, need_db: bool = True, dx=None, dw=None, db=None,
                     beta_w: float = 0.0, beta_b: float = 0.0, ws=None, stream=None):
     """dX = dY·W, dW = dYᵀ·X (+beta_w·dW), db = Σ_rows dY (+beta_b·db)."""
+    r = native().linear_backward(dy, x, w, bool(need_dx), bool(need_dw), bool(need_db), dx, dw, db,
+                                 beta_w, beta_b, ws, _handle(stream))
+    if r is not None:
+        return r
     _require_gpu(dy, x, w, dx, dw, db)
     Bn, in_f, out_f = x.shape[0], x.shape[1], w.shape[0]
     dev = x.device
@@ -338,6 +373,9 @@ def conv2d(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None, s
 
     x may be any NCHW view (read in place through its strides); the weight
     and bias are made dense."""
+    r = native().conv2d(x, w, b, stride, padding, ws, _handle(stream))
+    if r is not None:
+        return r
     _require_gpu(x, w, b)
     if x.dim() != 4 or w.dim() != 4 or x.shape[1] != w.shape[1]:
         raise ValueError("conv2d: expected input [N,C,H,W] and weight [Cout,C,kh,kw]")
@@ -369,6 +407,10 @@ def conv2d_backward(x: torch.Tensor, w: torch.Tensor, dy: torch.Tensor, stride: 
 
     dW = beta_w·dw + ∂L/∂W when an existing dense `dw` is passed (gradient
     accumulation)."""
+    r = native().conv2d_backward(x, w, dy, stride, padding, bool(need_dx), bool(need_dw),
+                                 bool(need_db), ws, dw, beta_w, _handle(stream))
+    if r is not None:
+        return r
     _require_gpu(x, w, dy)
     x, w, dy = x.contiguous(), w.contiguous(), dy.contiguous()
     n, c, h, wd = x.shape

@@ -112,6 +112,34 @@ def build(verbose: bool = False) -> Path:
     return LIB
 
 
+NATIVE = PKG / "_native.so"
+
+
+def build_native(verbose: bool = False) -> Path:
+    """Compile the torch binding (csrc/torch_binding.cpp) against libmtgemm.so."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    torch_lib = Path(torch.__file__).parent / "lib"
+    tmp = NATIVE.with_suffix(".so.tmp")
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared",
+           "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f"-I{ROOT / 'include'}", *[f"-I{d}" for d in include_paths()], f"-I{ROCM / 'include'}",
+           f"-I{sysconfig.get_paths()['include']}", str(CSRC / "torch_binding.cpp"),
+           "-o", str(tmp), f"-L{LIBDIR}", "-lmtgemm", f"-L{torch_lib}", "-ltorch_python",
+           "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN/lib"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"torch binding build failed:\n{r.stdout}")
+    os.replace(tmp, NATIVE)
+    return NATIVE
+
+
 HOST_TESTS = LIBDIR / "mt_host_tests"
 
 
@@ -133,4 +161,5 @@ def build_host_tests(verbose: bool = False) -> Path:
 
 if __name__ == "__main__":
     print(build(verbose="-v" in sys.argv))
+    print(build_native(verbose="-v" in sys.argv))
     print(build_host_tests(verbose="-v" in sys.argv))

@@ -380,36 +380,34 @@ Plan make_plan_uncached(int64_t M, int64_t N, int64_t K, int64_t batch, int cus,
     return best;
 }
 
+// Slot of a key in a table of 2^bits entries (Fibonacci hashing of its words).
+template <class... T>
+size_t hash_slot(int bits, T... words) {
+    uint64_t h = 0;
+    ((h = (h ^ (uint64_t)words) * 0x9E3779B97F4A7C15ull, h ^= h >> 29), ...);
+    return (size_t)(h >> (64 - bits));
+}
+
 // The cost model is a pure function of its arguments; a training loop asks
 // for the same few shapes again and again (workspace query, then launch), so
-// each thread keeps its last kEntries plans.  A workspace query of one GEMM
-// visits up to 10 keys (both families, with and without the prefetching
-// configurations and the wave-split kernel, the weight-gradient table), and
-// one convolution backward query four such shapes (about 34 keys): the cache
-// holds several layers' worth, so the launch that follows a query finds its
-// plan instead of rerunning the cost model.
+// each thread keeps plans, one per slot of a table indexed by a hash of the
+// key.  A workspace query of one GEMM visits 12 keys, one convolution backward
+// query four such shapes: the table holds several layers' worth.
 Plan make_plan(int64_t M, int64_t N, int64_t K, int64_t batch, int cus, bool allow_split,
                bool dl, bool wide, bool ksw, bool sp, bool imw = false, bool im16 = false) {
     struct Entry {
         int64_t M = -1, N = -1, K = -1, batch = -1;
-        int cus = 0;
-        bool allow_split = false, dl = false, wide = false, ksw = false, sp = false, imw = false,
-             im16 = false;
+        int cus = 0, flags = 0;
         Plan plan;
     };
-    constexpr int kEntries = 128;
-    thread_local Entry cache[kEntries];
-    thread_local int next = 0;
-    for (const Entry& e : cache)
-        if (e.M == M && e.N == N && e.K == K && e.batch == batch && e.cus == cus &&
-            e.allow_split == allow_split && e.dl == dl && e.wide == wide && e.ksw == ksw &&
-            e.sp == sp && e.imw == imw && e.im16 == im16)
-            return e.plan;
-    Entry& e = cache[next];
-    next = (next + 1) % kEntries;
-    e = Entry{M, N, K, batch, cus, allow_split, dl, wide, ksw, sp, imw, im16,
-              make_plan_uncached(M, N, K, batch, cus, allow_split, dl, wide, ksw, sp, imw,
-                                 im16)};
+    constexpr int kBits = 9;
+    thread_local Entry cache[1 << kBits];
+    const int flags = allow_split | dl << 1 | wide << 2 | ksw << 3 | sp << 4 | imw << 5 | im16 << 6;
+    Entry& e = cache[hash_slot(kBits, M, N, K, batch, flags)];
+    if (e.M != M || e.N != N || e.K != K || e.batch != batch || e.cus != cus || e.flags != flags)
+        e = Entry{M, N, K, batch, cus, flags,
+                  make_plan_uncached(M, N, K, batch, cus, allow_split, dl, wide, ksw, sp, imw,
+                                     im16)};
     return e.plan;
 }
 
@@ -678,18 +676,36 @@ size_t skinny_ws(int64_t M, int64_t N, int64_t K, int64_t batch, int cus) {
 
 // Workspace that covers the plan of either kernel family (for sizes queried
 // before the operand pointers, and hence the layouts, are known).
-size_t plan_ws(int64_t M, int64_t N, int64_t K, int64_t batch, int cus) {
+size_t plan_ws_uncached(int64_t M, int64_t N, int64_t K, int64_t batch, int cus) {
     size_t ws = 0;
     for (bool dl : {false, true})
-        for (bool wide : {false, true})
+        for (bool wide : {false, true}) {
+            if (wide && !dl) continue;   // of the direct-to-LDS family alone
             for (bool ksw : {false, true})
                 for (bool sp : {false, true})
                     ws = std::max(ws,
                                   make_plan(M, N, K, batch, cus, true, dl, wide, ksw, sp).ws_bytes);
-    Plan forced;
-    if (forced_plan(M, N, K, batch, true, true, true, true, &forced))
-        ws = std::max(ws, forced.ws_bytes);
+        }
     return std::max(ws, skinny_ws(M, N, K, batch, cus));
+}
+
+size_t plan_ws(int64_t M, int64_t N, int64_t K, int64_t batch, int cus) {
+    if (g_forced.family != MT_FAMILY_AUTO) {
+        Plan forced;
+        const bool f = forced_plan(M, N, K, batch, true, true, true, true, &forced);
+        return std::max(f ? forced.ws_bytes : 0, plan_ws_uncached(M, N, K, batch, cus));
+    }
+    struct Entry {
+        int64_t M = -1, N = -1, K = -1, batch = -1;
+        int cus = 0;
+        size_t ws = 0;
+    };
+    constexpr int kBits = 7;
+    thread_local Entry cache[1 << kBits];
+    Entry& e = cache[hash_slot(kBits, M, N, K, batch)];
+    if (e.M != M || e.N != N || e.K != K || e.batch != batch || e.cus != cus)
+        e = Entry{M, N, K, batch, cus, plan_ws_uncached(M, N, K, batch, cus)};
+    return e.ws;
 }
 
 // Contiguous layout of one operand for gemm_f32_sp, whatever its alignment, or
