@@ -61,6 +61,8 @@ enum : int {
                // (ci, r, s), gathered by 4-byte DMA
     L_IMH = 7, // B only (gemm_f32_dlh): L_IMR's operand built in LDS from a halo
                // patch of the input
+    L_IM4 = 9, // B only, gemm_f32_sp: L_IM's operand for any c % 4 == 0
+    L_IMQ = 10, // B only, gemm_f32_sp: L_IMW's operand, four columns per load (256-column tiles)
     L_KVI = 8  // A only, direct-to-LDS kernels: k-contiguous rows split into images,
                // A(m, k) = A[(k / a_hw)*a_img + m*a_mn + k % a_hw] (dY of a
                // convolution read in NCHW as [c_out][n*h_out*w_out])
@@ -76,6 +78,8 @@ enum : int {
 //          consecutive channels of one tap);
 // both read xt[img][oh*stride - pad + r][ow*stride - pad + s][ci], zero
 // outside the image.
+//   L_IM4: as L_IM, with c % 4 == 0: four consecutive k are four channels of one
+//          tap, and a chunk may hold several taps;
 //   L_IMR: B(k, n) with k = (ci*kh + r)*kw + s -- the OIHW weights' own K
 //          order, so they need no reorder -- and n as for L_IM, read from an
 //          NCHW view of any strides (img_stride, sc, sh, sw) of the input.

@@ -1,8 +1,9 @@
 // gemm_sp_instances.hip -- instantiates gemm_f32_sp for one configuration
 // (selected with -DMT_CFG=<n>): the 2x2 contiguous operand layouts with and
-// without the row sums of A, the forward convolution operands (L_IM, L_IMR;
-// configurations 0, 1, 3) and the weight gradient's (L_IMW, with dY copied or
-// read in NCHW; not 1 and 2).  Configuration 7: L_IM only.
+// without the row sums of A, the forward convolution operands (L_IM and L_IMR:
+// configurations 0, 1, 3; L_IM4: 1, 3) and the weight gradient's (L_IMW, with dY copied or
+// read in NCHW; not 1 and 2).  Configuration 7: L_IM and
+// L_IM4 only.
 #include "gemm_configs.hpp"
 #include "gemm_sp_kernel.hpp"
 
@@ -23,11 +24,17 @@ hipError_t launch_sp(const GemmParams& p, unsigned nblocks, hipStream_t s) {
 
 #if MT_CFG == 7
 GemmLaunchFn launcher(int la, int lb, bool rs) {
-    return la == L_KV && lb == L_IM && !rs ? launch_sp<L_KV, L_IM> : nullptr;
+    if (la == L_KV && lb == L_IM && !rs) return launch_sp<L_KV, L_IM>;
+    if (la == L_KV && lb == L_IM4 && !rs) return launch_sp<L_KV, L_IM4>;
+    return nullptr;
 }
 #else
 GemmLaunchFn launcher(int la, int lb, bool rs) {
     if (rs) {
+#if MT_CFG == 0
+        if (la == L_KV && lb == L_IMW) return launch_sp<L_KV, L_IMQ, true>;
+        if (la == L_KVI && lb == L_IMW) return launch_sp<L_KVI, L_IMQ, true>;
+#endif
         if (la == L_KV && lb == L_KV) return launch_sp<L_KV, L_KV, true>;
         if (la == L_MV && lb == L_MV) return launch_sp<L_MV, L_MV, true>;
         return nullptr;
@@ -38,9 +45,15 @@ GemmLaunchFn launcher(int la, int lb, bool rs) {
     if (la == L_MV && lb == L_MV) return launch_sp<L_MV, L_MV>;
 #if MT_CFG == 0 || MT_CFG == 1 || MT_CFG == 3
     if (la == L_KV && lb == L_IM) return launch_sp<L_KV, L_IM>;
+#if MT_CFG != 0
+    if (la == L_KV && lb == L_IM4) return launch_sp<L_KV, L_IM4>;
+#endif
     if (la == L_KV && lb == L_IMR) return launch_sp<L_KV, L_IMR>;
 #endif
-#if MT_CFG != 1 && MT_CFG != 2
+#if MT_CFG == 0
+    if (la == L_KV && lb == L_IMW) return launch_sp<L_KV, L_IMQ>;
+    if (la == L_KVI && lb == L_IMW) return launch_sp<L_KVI, L_IMQ>;
+#elif MT_CFG != 1 && MT_CFG != 2
     if (la == L_KV && lb == L_IMW) return launch_sp<L_KV, L_IMW>;
     if (la == L_KVI && lb == L_IMW) return launch_sp<L_KVI, L_IMW>;
 #endif

@@ -16,13 +16,13 @@
 //     along mn one value of each of four k; the four are cut together and go to
 //     LDS as 8 bytes per part.
 //   * LDS: per operand and part the two 8-k groups of the chunk, each a column
-//     of 16-byte entries, one per row (+128 bytes, so that the groups of a row
-//     fall on different banks): a fragment read is 512 contiguous bytes per
+//     of 16-byte entries, one per row (128 bytes more, so that the groups of a
+//     row fall on different banks): a fragment read is 512 contiguous bytes per
 //     half wave.
 //   * A workgroup whose sums are not finite takes its tile again with fp32
 //     MFMAs, from the same loaders.
 // Operand forms: L_KV / L_MV (any alignment and, across, any stride), L_IM,
-// L_IMW, L_IMR and L_KVI as in gemm_dl_kernel.hpp.
+// L_IMW, L_IMR and L_KVI as in gemm_dl_kernel.hpp, and L_IM4 and L_IMQ.
 #pragma once
 
 #include <type_traits>
@@ -34,8 +34,15 @@ namespace mtk {
 
 typedef f32x4 f32x4_u __attribute__((aligned(4)));   // a 16-byte load at any element
 
+// A global load of a selected address (a select with the zero page makes the
+// pointer generic to the compiler, and a flat load waits for LDS too).
+template <class T>
+__device__ __forceinline__ T sp_global(const float* p) {
+    return *(const T __attribute__((address_space(1)))*)p;
+}
+
 template <int L>
-constexpr bool sp_kc() { return L == L_KV || L == L_KVI || L == L_IM; }
+constexpr bool sp_kc() { return L == L_KV || L == L_KVI || L == L_IM || L == L_IM4; }
 
 // Items of four consecutive k of one row: BMN x 4 per chunk.  k-contiguous
 // forms put the four items of a row on consecutive lanes; the others put
@@ -52,6 +59,26 @@ struct SpItems {
         const int v = i * NT + t;
         return sp_kc<L>() ? v & 3 : __builtin_amdgcn_readfirstlane(v / BMN);
     }
+    // the row's entry in a group of the LDS tile
+    static constexpr int kEntries = BMN + 8;
+    __device__ __forceinline__ static int entry(int row) { return row; }
+};
+
+// L_IMQ: a thread's four items are the same four k of four consecutive rows.
+// Their entries lie in four runs (row % 4), so that consecutive lanes write
+// consecutive entries; a run is BMN/4 entries and 64 bytes more, which puts
+// the rows of a fragment read on different banks.
+template <int BMN, int NT>
+struct SpItems<L_IMQ, BMN, NT> {
+    static constexpr int NI = 4;
+    static_assert(BMN == 256 && NT == 256, "one quad per thread");
+    __device__ __forceinline__ static int row(int i, int t) { return (t & 63) * 4 + i; }
+    __device__ __forceinline__ static int kq(int, int t) {
+        return __builtin_amdgcn_readfirstlane(t >> 6);
+    }
+    static constexpr int kRun = BMN / 4 + 4;
+    static constexpr int kEntries = 4 * kRun + 8;
+    __device__ __forceinline__ static int entry(int row) { return (row & 3) * kRun + (row >> 2); }
 };
 
 // load(): the items of the next chunk in order (0, 1, 2, ... from the k0 given
@@ -204,7 +231,7 @@ struct SpLoader<L_IM, BMN, NT> {
             const bool ok = (unsigned)(ih0[i] + rt) < (unsigned)h &&
                             (unsigned)(iw0[i] + st) < (unsigned)w;
             const float* src = ok ? pix[i] + toff : dl_zero_page;
-            x[i] = *reinterpret_cast<const f32x4*>(src);
+            x[i] = sp_global<f32x4>(src);
         }
         ci0 += adv ? 16 : 0;
         if (ci0 == c) {
@@ -267,49 +294,100 @@ struct SpLoader<L_IMR, BMN, NT> {
                 const bool ok = (!PART || 4 * kq[i] + e < left) && (unsigned)(ih0[i] + rr) < (unsigned)h &&
                                 (unsigned)(iw0[i] + ss) < (unsigned)w;
                 const float* src = ok ? pix[i] + o : dl_zero_page;
-                x[i][e] = *src;
+                x[i][e] = sp_global<float>(src);
                 o += sw;
-                if (++ss == kw) {
-                    ss = 0;
-                    o += carry_s;
-                    if (++rr == kh) { rr = 0; o += carry_r; }
-                }
+                ++ss;
+                carry(rr, ss, o);
             }
             ss += ds;
             rr += dr;
             o += step;
-            if (ss >= kw) { ss -= kw; ++rr; o += carry_s; }
-            if (rr >= kh) { rr -= kh; o += carry_r; }
+            carry(rr, ss, o);
             r[i] = adv ? rr : r[i];
             s[i] = adv ? ss : s[i];
             off[i] = adv ? o : off[i];
         }
     }
+    __device__ __forceinline__ void carry(int& rr, int& ss, int64_t& o) const {
+        const bool a = ss >= kw;
+        ss -= a ? kw : 0;
+        rr += a;
+        o += a ? carry_s : 0;
+        const bool b = rr >= kh;
+        rr -= b ? kh : 0;
+        o += b ? carry_r : 0;
+    }
+};
+
+// The window origins of consecutive output pixels (img, oh, ow) of a
+// channels-last input, in scalar registers, by additions alone.
+struct SpPixels {
+    int st, ih0, iw0, ih1, iw1;    // first and one-past-last origins
+    int dy, dq;                    // 12 pixels in mixed radix (img, oh, ow), scaled
+    int64_t pix_step, row_step, img_step, step12;
+    struct At {
+        int y, q;                  // the origin, and its address (which may lie in
+        const float* org;          // the padding)
+    };
+
+    __device__ __forceinline__ void init(const ConvGeom& g) {
+        st = g.stride;
+        ih0 = -g.pad; iw0 = -g.pad_w;
+        ih1 = g.ho * st - g.pad; iw1 = g.wo * st - g.pad_w;
+        const int64_t pitch = (int64_t)st * g.w * g.c;
+        pix_step = (int64_t)st * g.c;
+        row_step = pitch - g.wo * pix_step;
+        img_step = g.img_stride - g.ho * pitch;
+        const int hw = g.ho * g.wo, img = 12 / hw, rem = 12 - img * hw, oh = rem / g.wo;
+        dy = oh * st;
+        dq = (rem - oh * g.wo) * st;
+        step12 = img * g.img_stride + oh * pitch + (rem - oh * g.wo) * pix_step;
+    }
+    __device__ __forceinline__ At at(const ConvGeom& g, const float* X, int k) const {
+        const int hw = g.ho * g.wo, img = k / hw, rem = k - img * hw;
+        const int oh = rem / g.wo, ow = rem - oh * g.wo;
+        const int y = oh * st - g.pad, q = ow * st - g.pad_w;
+        return {y, q, X + (int64_t)img * g.img_stride + ((int64_t)y * g.w + q) * g.c};
+    }
+    __device__ __forceinline__ void carry(At& a) const {
+        const bool r = a.q >= iw1;
+        a.q -= r ? iw1 - iw0 : 0;
+        a.y += r ? st : 0;
+        a.org += r ? row_step : 0;
+        const bool i = a.y >= ih1;
+        a.y -= i ? ih1 - ih0 : 0;
+        a.org += i ? img_step : 0;
+    }
+    __device__ __forceinline__ void next(At& a) const {
+        a.q += st;
+        a.org += pix_step;
+        carry(a);
+    }
+    __device__ __forceinline__ void next12(At& a) const {
+        a.q += dq;
+        a.y += dy;
+        a.org += step12;
+        carry(a);
+    }
 };
 
 // Implicit im2colᵀ of a channels-last input (the weight gradient): a lane
-// keeps its column (tap, channel), and the window origin of the output pixels
-// of its item's four k steps in scalar registers (by additions alone).
+// keeps its column (tap, channel); the output pixels of its item's four k are
+// scalar.
 template <int BMN, int NT>
 struct SpLoader<L_IMW, BMN, NT> {
     using I = SpItems<L_IMW, BMN, NT>;
     uint32_t off[I::NI];           // (r*w + s)*c + ci of the lane's column
     int r[I::NI], s[I::NI];        // its tap (r: far out for a column past N)
-    int kq[I::NI], ih[I::NI], iw[I::NI];   // the origin of the item's first k, and
-    const float* org[I::NI];               // its address (which may lie in the padding)
-    int h, w, st, ih0, iw0, ih1, iw1;      // first and one-past-last origins
-    int64_t pix_step, row_step, img_step;
+    int kq[I::NI], h, w;
+    SpPixels px;
+    SpPixels::At at[I::NI];        // the pixel of the item's first k
 
     __device__ __forceinline__ void init(const GemmParams& p, const float* X, int64_t, int64_t,
                                          int MN, int mn0, int k0, int t) {
         const ConvGeom& g = p.cv;
-        h = g.h; w = g.w; st = g.stride;
-        ih0 = -g.pad; iw0 = -g.pad_w;
-        ih1 = g.ho * st - g.pad; iw1 = g.wo * st - g.pad_w;
-        pix_step = (int64_t)st * g.c;
-        row_step = ((int64_t)st * g.w - (int64_t)g.wo * st) * g.c;
-        img_step = g.img_stride - (int64_t)g.ho * st * g.w * g.c;
-        const int hw = g.ho * g.wo;
+        h = g.h; w = g.w;
+        px.init(g);
 #pragma unroll
         for (int i = 0; i < I::NI; ++i) {
             const int row = mn0 + I::row(i, t), n = min(row, MN - 1);
@@ -319,65 +397,141 @@ struct SpLoader<L_IMW, BMN, NT> {
             r[i] = row < MN ? rr : -(1 << 29);
             off[i] = (uint32_t)((rr * g.w + s[i]) * g.c + ci);
             kq[i] = I::kq(i, t);
-            const int k = k0 + 4 * kq[i], img = k / hw, rem = k - img * hw;
-            const int oh = rem / g.wo, ow = rem - oh * g.wo;
-            ih[i] = oh * st - g.pad;
-            iw[i] = ow * st - g.pad_w;
-            org[i] = X + (int64_t)img * g.img_stride + ((int64_t)ih[i] * g.w + iw[i]) * g.c;
+            at[i] = px.at(g, X, k0 + 4 * kq[i]);
         }
     }
     template <bool PART>
     __device__ __forceinline__ void load(f32x4 (&x)[I::NI], int left, bool adv) {
 #pragma unroll
         for (int i = 0; i < I::NI; ++i) {
-            int y = ih[i], q = iw[i];
-            const float* o = org[i];
+            SpPixels::At a = at[i];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const bool ok = (!PART || 4 * kq[i] + e < left) &&
-                                (unsigned)(y + r[i]) < (unsigned)h &&
-                                (unsigned)(q + s[i]) < (unsigned)w;
-                const float* src = ok ? o + off[i] : dl_zero_page;
-                x[i][e] = *src;
-                q += st;
-                o += pix_step;
-                if (q == iw1) next_row(y, q, o, iw0);
+                                (unsigned)(a.y + r[i]) < (unsigned)h &&
+                                (unsigned)(a.q + s[i]) < (unsigned)w;
+                const float* src = ok ? a.org + off[i] : dl_zero_page;
+                x[i][e] = sp_global<float>(src);
+                px.next(a);
             }
-            q += 12 * st;
-            o += 12 * pix_step;
-            while (q >= iw1) next_row(y, q, o, q - (iw1 - iw0));
-            ih[i] = adv ? y : ih[i];
-            iw[i] = adv ? q : iw[i];
-            org[i] = adv ? o : org[i];
-        }
-    }
-    __device__ __forceinline__ void next_row(int& y, int& q, const float*& o, int q_new) const {
-        q = q_new;
-        y += st;
-        o += row_step;
-        if (y == ih1) {
-            y = ih0;
-            o += img_step;
+            px.next12(a);
+            at[i].y = adv ? a.y : at[i].y;
+            at[i].q = adv ? a.q : at[i].q;
+            at[i].org = adv ? a.org : at[i].org;
         }
     }
 };
 
-// LDS of one operand's chunk: three parts of two 8-k groups of BMN 16-byte
+// L_IMW with four consecutive channels of one tap per load: the four k of a
+// thread's quad of columns are four 16-byte loads, and change places in
+// registers.
+template <int BMN, int NT>
+struct SpLoader<L_IMQ, BMN, NT> {
+    using I = SpItems<L_IMQ, BMN, NT>;
+    uint32_t off;                  // (r*w + s)*c + ci of the quad
+    int r, s;                      // its tap (r: far out for columns past N)
+    int kq, h, w;
+    SpPixels px;
+    SpPixels::At at;               // the pixel of the first k
+
+    __device__ __forceinline__ void init(const GemmParams& p, const float* X, int64_t, int64_t,
+                                         int MN, int mn0, int k0, int t) {
+        const ConvGeom& g = p.cv;
+        h = g.h; w = g.w;
+        px.init(g);
+        const int row = mn0 + I::row(0, t), n = min(row, MN - 4);   // MN % 4 == 0
+        const int tap = n / g.c, ci = n - tap * g.c, rr = tap / g.kw;
+        s = tap - rr * g.kw;
+        r = row < MN ? rr : -(1 << 29);
+        off = (uint32_t)((rr * g.w + s) * g.c + ci);
+        kq = I::kq(0, t);
+        at = px.at(g, X, k0 + 4 * kq);
+    }
+    template <bool PART>
+    __device__ __forceinline__ void load(f32x4 (&x)[I::NI], int left, bool adv) {
+        SpPixels::At a = at;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const bool ok = (!PART || 4 * kq + e < left) && (unsigned)(a.y + r) < (unsigned)h &&
+                            (unsigned)(a.q + s) < (unsigned)w;
+            const f32x4 v = sp_global<f32x4>(ok ? a.org + off : dl_zero_page);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) x[j][e] = v[j];
+            px.next(a);
+        }
+        px.next12(a);
+        at.y = adv ? a.y : at.y;
+        at.q = adv ? a.q : at.q;
+        at.org = adv ? a.org : at.org;
+    }
+};
+
+// L_IM for any c % 4 == 0: the tap and channel of a thread's items are its own
+// (an item of each chunk: the k of its lane's group).
+template <int BMN, int NT>
+struct SpLoader<L_IM4, BMN, NT> {
+    using I = SpItems<L_IM4, BMN, NT>;
+    const float* pix[I::NI];
+    int ih0[I::NI], iw0[I::NI];
+    int rt, st, ci, kq;
+    int c, h, w, kw, dr, ds, dc;   // 16 k in mixed radix (r, s, ci)
+
+    __device__ __forceinline__ void init(const GemmParams& p, const float* X, int64_t, int64_t,
+                                         int MN, int mn0, int k0, int t) {
+        const ConvGeom& g = p.cv;
+        c = g.c; h = g.h; w = g.w; kw = g.kw;
+        const int hw = g.ho * g.wo;
+#pragma unroll
+        for (int i = 0; i < I::NI; ++i) {
+            const int n = mn0 + I::row(i, t);
+            const int img = n / hw, rem = n - img * hw;
+            const int oh = rem / g.wo, ow = rem - oh * g.wo;
+            ih0[i] = n < MN ? oh * g.stride - g.pad : -(1 << 30);   // past N: zeros
+            iw0[i] = ow * g.stride - g.pad_w;
+            pix[i] = X + (int64_t)img * g.img_stride + ((int64_t)ih0[i] * g.w + iw0[i]) * g.c;
+        }
+        kq = t & 3;
+        const int k = k0 + 4 * kq, tap = k / c, dtap = 16 / c;
+        ci = k - tap * c;
+        rt = tap / kw;
+        st = tap - rt * kw;
+        dc = 16 - dtap * c;
+        dr = dtap / kw;
+        ds = dtap - dr * kw;
+    }
+    template <bool PART>
+    __device__ __forceinline__ void load(f32x4 (&x)[I::NI], int left, bool adv) {
+        const int toff = (rt * w + st) * c + ci;
+#pragma unroll
+        for (int i = 0; i < I::NI; ++i) {
+            const bool ok = (!PART || 4 * kq < left) && (unsigned)(ih0[i] + rt) < (unsigned)h &&
+                            (unsigned)(iw0[i] + st) < (unsigned)w;
+            const float* src = ok ? pix[i] + toff : dl_zero_page;
+            x[i] = sp_global<f32x4>(src);
+        }
+        ci += adv ? dc : 0;
+        const bool cc = ci >= c;
+        ci -= cc ? c : 0;
+        st += adv ? ds + cc : 0;
+        const bool cs = st >= kw;
+        st -= cs ? kw : 0;
+        rt += adv ? dr + cs : 0;
+    }
+};
+
+// LDS of one operand's chunk: three parts of two 8-k groups of 16-byte
 // entries, in bytes.
-template <int BMN>
-constexpr int sp_group() { return BMN * 16 + 128; }
-template <int BMN>
-constexpr int sp_plane() { return 2 * sp_group<BMN>(); }
+template <class I>
+constexpr int sp_group() { return I::kEntries * 16; }
+template <class I>
+constexpr int sp_plane() { return 2 * sp_group<I>(); }
 
-template <int BM, int BN>
-constexpr int sp_lds_bytes() { return 2 * 3 * (sp_plane<BM>() + sp_plane<BN>()); }
-
-template <int BMN>
+template <class I>
 __device__ __forceinline__ void sp_frag(const char* lds, int row, int half, SplitFrag& f) {
-    const char* p = lds + half * sp_group<BMN>() + row * 16;
+    const char* p = lds + half * sp_group<I>() + I::entry(row) * 16;
     f.h = *reinterpret_cast<const u32x4*>(p);
-    f.m = *reinterpret_cast<const u32x4*>(p + sp_plane<BMN>());
-    f.l = *reinterpret_cast<const u32x4*>(p + 2 * sp_plane<BMN>());
+    f.m = *reinterpret_cast<const u32x4*>(p + sp_plane<I>());
+    f.l = *reinterpret_cast<const u32x4*>(p + 2 * sp_plane<I>());
 }
 
 // A barrier that orders LDS alone: global loads stay in flight across it.
@@ -396,9 +550,9 @@ gemm_f32_sp(GemmParams p) {
     constexpr int NW = (BM / WM) * WAVES_N;
     constexpr int NT = NW * 64;
     constexpr int MB = WM / 32, NB = WN / 32;
-    constexpr int BUF = 3 * (sp_plane<BM>() + sp_plane<BN>());
     using IA = SpItems<LA, BM, NT>;
     using IB = SpItems<LB, BN, NT>;
+    constexpr int BUF = 3 * (sp_plane<IA>() + sp_plane<IB>());
     __shared__ __attribute__((aligned(1024))) char smem[2 * BUF];
 
     const int t = threadIdx.x;
@@ -446,25 +600,25 @@ gemm_f32_sp(GemmParams p) {
         f32x16 sml[MB][NB];
         zero_blocks<MB, NB>(sml);
         start();
-        auto put = [&](char* dst, auto& x, auto items, auto bmn) {
+        auto put = [&](char* dst, auto& x, auto items) {
             using It = decltype(items);
-            constexpr int B = decltype(bmn)::value;
 #pragma unroll
             for (int i = 0; i < It::NI; ++i) {
                 u32x2 h, m, l;
                 split4(x[i], h, m, l);
                 const int kq = It::kq(i, t);
-                char* q = dst + (kq >> 1) * sp_group<B>() + It::row(i, t) * 16 + (kq & 1) * 8;
+                char* q = dst + (kq >> 1) * sp_group<It>() + It::entry(It::row(i, t)) * 16 +
+                          (kq & 1) * 8;
                 *reinterpret_cast<u32x2*>(q) = h;
-                *reinterpret_cast<u32x2*>(q + sp_plane<B>()) = m;
-                *reinterpret_cast<u32x2*>(q + 2 * sp_plane<B>()) = l;
+                *reinterpret_cast<u32x2*>(q + sp_plane<It>()) = m;
+                *reinterpret_cast<u32x2*>(q + 2 * sp_plane<It>()) = l;
             }
         };
         auto cut = [&](int chunk, f32x4 (&xa)[IA::NI], f32x4 (&xb)[IB::NI]) {
             char* const buf = smem + (chunk & 1) * BUF;
             add_rows(xa);
-            put(buf, xa, IA{}, std::integral_constant<int, BM>{});
-            put(buf + 3 * sp_plane<BM>(), xb, IB{}, std::integral_constant<int, BN>{});
+            put(buf, xa, IA{});
+            put(buf + 3 * sp_plane<IA>(), xb, IB{});
         };
         // The last product (h·l) of a chunk is left for the next step, which
         // issues it between its barrier and the arrival of its fragments.
@@ -477,10 +631,10 @@ gemm_f32_sp(GemmParams p) {
             const char* const buf = smem + (kt & 1) * BUF;
             SplitFrag na[MB], nb[NB];
 #pragma unroll
-            for (int i = 0; i < MB; ++i) sp_frag<BM>(buf, ra + 32 * i + lrow, half, na[i]);
+            for (int i = 0; i < MB; ++i) sp_frag<IA>(buf, ra + 32 * i + lrow, half, na[i]);
 #pragma unroll
             for (int j = 0; j < NB; ++j)
-                sp_frag<BN>(buf + 3 * sp_plane<BM>(), rb + 32 * j + lrow, half, nb[j]);
+                sp_frag<IB>(buf + 3 * sp_plane<IA>(), rb + 32 * j + lrow, half, nb[j]);
             mfma_split<MB, NB, 5, 6>(acc, sml, fa, fb);
             mfma_split<MB, NB, 0, 5>(acc, sml, na, nb);
 #pragma unroll

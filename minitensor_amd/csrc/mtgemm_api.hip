@@ -105,6 +105,7 @@ const char* layout_name(int l) {
         case L_IM: return "im2col";
         case L_IMW: return "im2colT";
         case L_IMR: return "im2col_nchw";
+        case L_IM4: return "im2col_nchw_c4";   // an NCHW input, padded on its way
         case L_IMH: return "im2col_halo";
         case L_KVI: return "kv_nchw";
         case L_KS: return "ks";
@@ -134,6 +135,7 @@ struct CfgCost {
     double eff;   // sustained fraction of the CU's MFMA rate inside a workgroup
     int occ;      // resident workgroups per CU
     bool sp = false;   // gemm_f32_sp
+    double alone = 0;  // factor of a workgroup alone on its CU (0: the model's own rules)
 };
 
 // Cost model (in CU cycles) used to pick the tile configuration and split-K
@@ -176,20 +178,22 @@ constexpr CfgCost kDlCost[kNumDlCfg] = {
     {DlCfg<4>::BM, DlCfg<4>::BN, 1.58, 1, true},
     {DlCfg<5>::BM, DlCfg<5>::BN, 0.72, 8},
     {DlCfg<6>::BM, DlCfg<6>::BN, 0.84, 3, true},
-    {DlCfg<7>::BM, DlCfg<7>::BN, 1.00, 3, true}};
+    {DlCfg<7>::BM, DlCfg<7>::BN, 0.95, 3, true}};
 // The same configurations with the convolution weight gradient's gathered B
-// operand (L_IMW); 0: not offered (gemm_f32_sp's gathers cost a workgroup of
-// 256 threads more than the bf16 units save: 128 x 1152 x 25088 at configuration
-// 1, 28 splits, 132 us against 92 on the fp32 kernel).
+// operand (L_IMW); 0: not offered.  Its gather costs every tile more than a
+// contiguous operand does, the 64x64 ones the most, and a workgroup alone on
+// its CU has nothing to hide it behind.  Fitted to graph timings of the
+// configurations at 1-64 splits on 16 layers (mean error of a time 6 %; the
+// pick is 0.9 % above the fastest measured plan on average).
 constexpr CfgCost kDlCostImw[kNumDlCfg] = {
-    {DlCfg<0>::BM, DlCfg<0>::BN, 0, 2},
-    {DlCfg<1>::BM, DlCfg<1>::BN, 0.86, 4},
-    {DlCfg<2>::BM, DlCfg<2>::BN, 0.68, 8},
-    {DlCfg<3>::BM, DlCfg<3>::BN, 1.42, 1, true},
+    {DlCfg<0>::BM, DlCfg<0>::BN, 0.86, 2, true, 1.11},
+    {DlCfg<1>::BM, DlCfg<1>::BN, 0.64, 4, false, 1.0},
+    {DlCfg<2>::BM, DlCfg<2>::BN, 0.50, 8, false, 1.24},
+    {DlCfg<3>::BM, DlCfg<3>::BN, 1.15, 1, true},
     {DlCfg<4>::BM, DlCfg<4>::BN, 0, 1},
-    {DlCfg<5>::BM, DlCfg<5>::BN, 0.72, 8},
+    {DlCfg<5>::BM, DlCfg<5>::BN, 0.52, 8, false, 1.47},
     {DlCfg<6>::BM, DlCfg<6>::BN, 0, 3},
-    {DlCfg<7>::BM, DlCfg<7>::BN, 0, 2}};   // (configuration 7: L_IM only)
+    {DlCfg<7>::BM, DlCfg<7>::BN, 0, 2}};   // (configuration 7: L_IM, L_IM4)
 // And with the 4-byte gathers of an NCHW view (L_IMR), of which a tile of 256
 // columns on 256 threads makes the most per thread: the 7x7 stem at batch 32
 // took 188 us on configuration 0 against 178 on 2.
@@ -242,6 +246,9 @@ struct CostModel {
     double launch_cycles = 17700.0;          // second (reduce) launch
 };
 constexpr int kMaxSplits = 256;
+// Of the weight gradient, whose K is every output pixel of the batch: two
+// workgroups per CU of a single-tile dW.
+constexpr int kMaxImwSplits = 512;
 // The cost model was fitted on splits 1-16.  Beyond 16, a split must keep at
 // least kMinKpsBeyondFit of K: on random GEMMs (K <= 4700) the model's picks
 // of 19-59 splits at 64-208 per split ran 2-12 % slower than 16 splits (it
@@ -299,7 +306,8 @@ double plan_cycles(const CostModel& cm, const CfgCost& cc, const Plan& pl, int64
     // workgroup per CU) does not see.  Measured, 63 x 4096 x 4096: split 8
     // (two per CU) 26.2 us against 29.4 us at split 4; 8-16 rows 24.4 against
     // 27.2.
-    const double pair = (pl.dl && pl.cfg == kDlpSmallCfg && pl.tiles_m == 1 && per_cu == 2)
+    const double pair = (pl.dl && pl.cfg == kDlpSmallCfg && pl.tiles_m == 1 && per_cu == 2 &&
+                         cc.alone == 0)
                             ? kCoresidentPair
                             : 1.0;
     // A 64x64 tile alone on its CU over a long K range (one wave per SIMD,
@@ -307,12 +315,13 @@ double plan_cycles(const CostModel& cm, const CfgCost& cc, const Plan& pl, int64
     // which comes from CUs holding several.  Measured on random shapes
     // (bench.py --audit): 1456 x 532 x 2500 at split 1 (207 workgroups) 64.6 us
     // against 48.0 at split 6; the factor moves such shapes to split-K.
-    const double alone = (pl.dl && (pl.cfg == kDlSmallCfg || pl.cfg == kDlpSmallCfg) &&
-                          per_cu == 1 && pl.kps >= kAloneMinK)
-                             ? kAlonePenalty
-                             : 1.0;
-    const double sp_alone = cc.sp && cc.occ > 1 && per_cu == 1 ? kSpAlone : 1.0;
-    double t = per_cu * work * pair * alone * sp_alone + per_cu * epi / cc.occ +
+    const bool small = pl.dl && (pl.cfg == kDlSmallCfg || pl.cfg == kDlpSmallCfg);
+    const double alone = per_cu > 1                          ? 1.0
+                         : cc.alone > 0                      ? cc.alone
+                         : small && pl.kps >= kAloneMinK     ? kAlonePenalty
+                         : cc.sp && cc.occ > 1               ? kSpAlone
+                                                             : 1.0;
+    double t = per_cu * work * pair * alone + per_cu * epi / cc.occ +
                rounds * (cc.sp ? cm.sp_round_latency : cm.round_latency);
     if (pl.splits > 1) {
         const double bytes = (double)(2 * pl.splits + 1) * M * N * batch * 4.0;
@@ -325,9 +334,10 @@ double plan_cycles(const CostModel& cm, const CfgCost& cc, const Plan& pl, int64
 // chosen (see wide_ok in launch_gemm); ksw: the wave-split kernel may be;
 // sp: gemm_f32_sp can take the operands (sp_fits, sp_layouts); imw: B is the
 // weight-gradient operand (priced by kDlCostImw); im16: the 112-column tile
-// (kNarrowCfg, B = L_IM) may be.
+// (kNarrowCfg, B = L_IM) may be; im4: B is L_IM4 (configurations 1, 3 and 7).
 Plan make_plan_uncached(int64_t M, int64_t N, int64_t K, int64_t batch, int cus,
-                        bool allow_split, bool dl, bool wide, bool ksw, bool sp, bool imw, bool im16) {
+                        bool allow_split, bool dl, bool wide, bool ksw, bool sp, bool imw, bool im16,
+                        bool im4) {
     static const CostModel cm;
     const CfgCost* cfgs = dl ? (imw ? kDlCostImw : kDlCost) : sp ? kRsSpCost : kRsCost;
     const int ncfg = dl ? kNumDlCfg : kNumCfg;
@@ -338,10 +348,11 @@ Plan make_plan_uncached(int64_t M, int64_t N, int64_t K, int64_t batch, int cus,
         if (dl && is_wide_cfg(cfg) && !wide) continue;
         if (dl && is_sp_cfg(cfg) && !sp && !(imw && cfg == 1)) continue;
         if (cfgs[cfg].eff <= 0) continue;
-        if (dl && cfg == kNarrowCfg && !im16) continue;
+        if (dl && cfg == kNarrowCfg && !im16 && !im4) continue;
+        if (im4 && cfg != 1 && cfg != 3 && cfg != kNarrowCfg) continue;
         CfgCost cc = cfgs[cfg];
-        if (dl && cfg == 0 && !wide && !im16) cc.eff = kImrNarrowEff;   // L_IMR
-        for (int s = 1; s <= kMaxSplits; ++s) {
+        if (dl && cfg == 0 && !wide && !im16 && !im4) cc.eff = kImrNarrowEff;   // L_IMR
+        for (int s = 1; s <= (imw ? kMaxImwSplits : kMaxSplits); ++s) {
             if (s > 1 && !allow_split) break;
             const Plan pl = cfg_plan(cc, cfg, dl, M, N, K, batch, s);
             if (s > 1 && pl.kps < 64) break;
@@ -394,7 +405,8 @@ size_t hash_slot(int bits, T... words) {
 // key.  A workspace query of one GEMM visits 12 keys, one convolution backward
 // query four such shapes: the table holds several layers' worth.
 Plan make_plan(int64_t M, int64_t N, int64_t K, int64_t batch, int cus, bool allow_split,
-               bool dl, bool wide, bool ksw, bool sp, bool imw = false, bool im16 = false) {
+               bool dl, bool wide, bool ksw, bool sp, bool imw = false, bool im16 = false,
+               bool im4 = false) {
     struct Entry {
         int64_t M = -1, N = -1, K = -1, batch = -1;
         int cus = 0, flags = 0;
@@ -402,12 +414,13 @@ Plan make_plan(int64_t M, int64_t N, int64_t K, int64_t batch, int cus, bool all
     };
     constexpr int kBits = 9;
     thread_local Entry cache[1 << kBits];
-    const int flags = allow_split | dl << 1 | wide << 2 | ksw << 3 | sp << 4 | imw << 5 | im16 << 6;
+    const int flags = allow_split | dl << 1 | wide << 2 | ksw << 3 | sp << 4 | imw << 5 | im16 << 6 |
+                      im4 << 7;
     Entry& e = cache[hash_slot(kBits, M, N, K, batch, flags)];
     if (e.M != M || e.N != N || e.K != K || e.batch != batch || e.cus != cus || e.flags != flags)
         e = Entry{M, N, K, batch, cus, flags,
                   make_plan_uncached(M, N, K, batch, cus, allow_split, dl, wide, ksw, sp, imw,
-                                     im16)};
+                                     im16, im4)};
     return e.plan;
 }
 
@@ -535,10 +548,10 @@ void set_halo_geometry(ConvGeom& g) {
     g.pw = (g.wo - 1) * g.stride + g.kw;
 }
 
-GemmLaunchFn conv_launcher(int cfg, bool nchw) {
-    if (is_sp_cfg(cfg)) return sp_launcher(cfg, L_KV, nchw ? L_IMR : L_IM);
-    if (cfg == 2) return nchw ? dl_convr_launcher_cfg2() : dl_conv_launcher_cfg2();
-    return nullptr;
+GemmLaunchFn conv_launcher(int cfg, int lb) {
+    if (is_sp_cfg(cfg)) return sp_launcher(cfg, L_KV, lb);
+    if (cfg != 2 || lb == L_IM4) return nullptr;
+    return lb == L_IMR ? dl_convr_launcher_cfg2() : dl_conv_launcher_cfg2();
 }
 
 // ---- HBM-bound shapes on the vector ALUs (gemm_skinny_kernel.hpp) ----------
@@ -932,10 +945,32 @@ __device__ __forceinline__ void channel_sum(const GemmParams& p, int m, float* r
     if (threadIdx.x == 0) p.csum[m] = (p.csum_beta != 0.f ? p.csum_beta * p.csum[m] : 0.f) + r;
 }
 
+// One group of four output columns of the vector forms: bias and beta·C added
+// to v, stored as one 16-byte vector when C allows (c_vec), else element by
+// element through col(n).
+__device__ __forceinline__ void reduce_store(const GemmParams& p, float* crow, int n, float brow,
+                                             f32x4 v) {
+    f32x4 bcol = {0.f, 0.f, 0.f, 0.f}, old = bcol;
+    if (p.bias_axis == 2)
+        for (int e = 0; e < 4; ++e) bcol[e] = p.bias[(int64_t)(n + e) * p.bias_stride];
+    if (p.beta != 0.f) {
+        if (p.c_vec) old = *reinterpret_cast<const f32x4*>(crow + col_offset(p, n));
+        else
+            for (int e = 0; e < 4; ++e) old[e] = crow[col_offset(p, n + e)];
+    }
+    v += brow;
+    if (p.bias_axis == 2) v += bcol;
+    if (p.beta != 0.f) v += p.beta * old;
+    if (p.c_vec) {
+        *reinterpret_cast<f32x4*>(crow + col_offset(p, n)) = v;
+    } else {
+        for (int e = 0; e < 4; ++e) crow[col_offset(p, n + e)] = v[e];
+    }
+}
+
 // Vector form (ws_vec: N % 4 == 0, 16-byte partials): blockIdx.y walks output
-// rows (batch-major), threads walk 4-column groups; the group is stored as one
-// 16-byte vector when C allows (c_vec), else element by element through
-// col(n).  Same per-element summation order as the scalar form.
+// rows (batch-major), threads walk 4-column groups.  Same per-element summation
+// order as the scalar form.
 // CSUM: also the channel sums of GemmParams::csum (a separate instantiation,
 // so that the plain reduction carries neither its code nor its LDS).
 template <bool CSUM, int NT = 256>
@@ -953,24 +988,45 @@ __global__ void __launch_bounds__(NT) splitk_reduce_vec_f32(GemmParams p) {
         const float* src = p.ws + (int64_t)bz * MN + (int64_t)m * p.N;
         float* crow = p.C + (int64_t)bz * p.c_b + (int64_t)m * p.c_m;
         for (int n = (blockIdx.x * blockDim.x + threadIdx.x) * 4; n < p.N;
-             n += gridDim.x * blockDim.x * 4) {
-            f32x4 bcol = zero, old = zero;
-            if (p.bias_axis == 2)
-                for (int e = 0; e < 4; ++e) bcol[e] = p.bias[(int64_t)(n + e) * p.bias_stride];
-            if (p.beta != 0.f) {
-                if (p.c_vec) old = *reinterpret_cast<const f32x4*>(crow + col_offset(p, n));
-                else
-                    for (int e = 0; e < 4; ++e) old[e] = crow[col_offset(p, n + e)];
+             n += gridDim.x * blockDim.x * 4)
+            reduce_store(p, crow, n, brow,
+                         sum_partials<f32x4>(src + n, p.batch * MN, p.splits, zero));
+    }
+}
+
+// Many slabs of a small output, one batch entry: a thread of the form above
+// walks all of them in turn, eight loads at a time, and there are few threads
+// (the RGB stem's dW, 64 x 196 in 512 slabs: 3136 threads, 41 us for 26 MB).
+// Here 16 slices of the slabs go side by side, 16 column groups of 4 each, and
+// their sums meet in LDS in a fixed order: 12 us.  CSUM: the row sums from
+// GemmParams::csum_rows.
+constexpr int kSliceMinSplits = 32;
+template <bool CSUM>
+__global__ void __launch_bounds__(256) splitk_reduce_slices_f32(GemmParams p) {
+    __shared__ f32x4 part[16][16];
+    __shared__ float red[CSUM ? 256 : 1];
+    const int64_t MN = (int64_t)p.M * p.N;
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    const int col = threadIdx.x & 15, slice = threadIdx.x >> 4;
+    const int per = (p.splits + 15) / 16;
+    const int s0 = min(slice * per, p.splits), s1 = min(s0 + per, p.splits);
+    for (int m = blockIdx.y; m < p.M; m += gridDim.y) {
+        if constexpr (CSUM)
+            if (blockIdx.x == 0) channel_sum<256>(p, m, red);
+        const float brow = p.bias_axis == 1 ? p.bias[(int64_t)m * p.bias_stride] : 0.f;
+        const float* src = p.ws + s0 * MN + (int64_t)m * p.N;
+        float* crow = p.C + (int64_t)m * p.c_m;
+        for (int n0 = blockIdx.x * 64; n0 < p.N; n0 += gridDim.x * 64) {
+            const int n = n0 + col * 4;
+            part[slice][col] = n < p.N ? sum_partials<f32x4>(src + n, MN, s1 - s0, zero) : zero;
+            __syncthreads();
+            if (slice == 0 && n < p.N) {
+                f32x4 v = part[0][col];
+#pragma unroll
+                for (int i = 1; i < 16; ++i) v += part[i][col];
+                reduce_store(p, crow, n, brow, v);
             }
-            f32x4 v = sum_partials<f32x4>(src + n, p.batch * MN, p.splits, zero);
-            v += brow;
-            if (p.bias_axis == 2) v += bcol;
-            if (p.beta != 0.f) v += p.beta * old;
-            if (p.c_vec) {
-                *reinterpret_cast<f32x4*>(crow + col_offset(p, n)) = v;
-            } else {
-                for (int e = 0; e < 4; ++e) crow[col_offset(p, n + e)] = v[e];
-            }
+            __syncthreads();
         }
     }
 }
@@ -1045,7 +1101,7 @@ int launch_skinny(const GemmParams& p0, SkinnyPlan sp, void* workspace, size_t w
 int launch_gemm(GemmParams& p, bool dl, int la, int lb, void* workspace, size_t ws_bytes,
                 hipStream_t stream) {
     const int64_t M = p.M, N = p.N, K = p.K, batch = p.batch;
-    const bool implicit = lb == L_IM || lb == L_IMW || lb == L_IMR;
+    const bool implicit = lb == L_IM || lb == L_IMW || lb == L_IMR || lb == L_IM4;
     // 16-byte epilogue stores: four consecutive columns must be contiguous,
     // aligned, and (for a scattered output) never straddle a column group.
     p.c_vec = p.c_n == 1 && (N & 3) == 0 && ((uintptr_t)p.C & 15u) == 0 && (p.c_m & 3) == 0 &&
@@ -1059,7 +1115,8 @@ int launch_gemm(GemmParams& p, bool dl, int la, int lb, void* workspace, size_t 
     // A batch-summed product of two k-contiguous operands fuses them too, as
     // partials per (split, batch entry) that its reduction sums for csum.
     const bool rs_part = p.part && la == L_KV && lb == L_KV && p.csum != nullptr;
-    if (!rs_part && (batch != 1 || la != L_MV || lb != L_MV || p.part)) p.rowsum = nullptr;
+    if (!rs_part && lb != L_IMW && (batch != 1 || la != L_MV || lb != L_MV || p.part))
+        p.rowsum = nullptr;
     // The HBM-bound shapes (few rows or columns, or K <= 16) on the vector ALUs.
     if (!implicit && la != L_KVI && p.rowsum == nullptr && p.csum == nullptr && !p.part) {
         const SkinnyPlan sp =
@@ -1069,7 +1126,7 @@ int launch_gemm(GemmParams& p, bool dl, int la, int lb, void* workspace, size_t 
     // The prefetching configurations' contract: vector layouts or the
     // weight-gradient operand (not the implicit-im2col one), a non-empty K
     // range.
-    const bool wide_ok = dl && lb != L_IM && lb != L_IMR && K > 0;
+    const bool wide_ok = dl && lb != L_IM && lb != L_IMR && lb != L_IM4 && K > 0;
     Plan plan;
     const bool im16_ok = dl && lb == L_IM;
     // gemm_f32_sp: contiguous operands, offsets within a tile of 32 bits
@@ -1090,14 +1147,22 @@ int launch_gemm(GemmParams& p, bool dl, int la, int lb, void* workspace, size_t 
         // convolution operands and the fused row sums
         const bool ksw_ok = !implicit && p.rowsum == nullptr;
         plan = make_plan(M, N, K, batch, device_cu_count(), true, dl, wide_ok, ksw_ok, sp_ok,
-                         lb == L_IMW, im16_ok && kOfferNarrow);
+                         lb == L_IMW, im16_ok && kOfferNarrow, lb == L_IM4);
         if (need(plan) > 0 && (workspace == nullptr || ws_bytes < need(plan)))
             plan = make_plan(M, N, K, batch, device_cu_count(), false, dl, wide_ok, ksw_ok, sp_ok,
-                             lb == L_IMW, im16_ok && kOfferNarrow);
+                             lb == L_IMW, im16_ok && kOfferNarrow, lb == L_IM4);
         if (need(plan) > 0 && (workspace == nullptr || ws_bytes < need(plan)))
             return MT_ERR_WORKSPACE;
     }
-    if (!plan.dl || (plan.splits > 1 && !rs_part) || plan.cfg == kNarrowCfg) p.rowsum = nullptr;
+    // The weight gradient's row sums (db from the dY that it reads anyway):
+    // partials per split, where configuration 0 splits K and the workspace has
+    // room for them.
+    const bool rs_imw = lb == L_IMW && p.rowsum != nullptr && p.csum != nullptr && plan.dl &&
+                        plan.cfg == 0 && plan.splits > 1 &&
+                        ws_bytes >= plan.ws_bytes + (size_t)plan.splits * M * sizeof(float);
+    if (lb == L_IMW && !rs_imw) p.rowsum = nullptr;
+    if (!plan.dl || (plan.splits > 1 && !rs_part && !rs_imw) || plan.cfg == kNarrowCfg)
+        p.rowsum = nullptr;
     p.splits = plan.splits;
     p.k_per_split = plan.splits > 1 ? plan.kps : (int)std::max<int64_t>(K, 1);
     p.tiles_m = plan.tiles_m;
@@ -1111,11 +1176,11 @@ int launch_gemm(GemmParams& p, bool dl, int la, int lb, void* workspace, size_t 
     if (!p.ws_vec || (batch != 1 && !p.part)) p.csum = nullptr;
     // The fused row sums of a batch-summed product: partials after the slabs,
     // summed by the reduction in place of a second pass over csum_src.
-    if (rs_part && p.rowsum != nullptr && p.csum != nullptr) {
+    if ((rs_part || rs_imw) && p.rowsum != nullptr && p.csum != nullptr) {
         float* rows = p.ws + (int64_t)plan.splits * batch * M * N;
         p.rowsum = rows;
         p.csum_rows = rows;
-    } else if (rs_part) {
+    } else if (rs_part || rs_imw) {
         p.rowsum = nullptr;
     }
 
@@ -1134,7 +1199,8 @@ int launch_gemm(GemmParams& p, bool dl, int la, int lb, void* workspace, size_t 
                   p.part ? (p.csum_rows ? " batch-summed rows" : " batch-summed") : "");
 
     GemmLaunchFn fn = halo ? dlh_launcher(plan.cfg)
-                      : lb == L_IM || lb == L_IMR ? conv_launcher(plan.cfg, lb == L_IMR)
+                      : lb == L_IM || lb == L_IMR || lb == L_IM4 ? conv_launcher(plan.cfg, lb)
+                      : lb == L_IMW && p.rowsum != nullptr ? sp_launcher(plan.cfg, la, lb, true)
                       : lb == L_IMW ? convw_launcher(plan.cfg, (K & 15) != 0, la == L_KVI)
                       : p.rowsum != nullptr ? rowsum_launcher(plan.cfg, (K & 15) != 0, la == L_KV)
                                             : pick_launcher(plan, la, lb, (K & 15) != 0, sla, slb);
@@ -1150,7 +1216,14 @@ int launch_gemm(GemmParams& p, bool dl, int la, int lb, void* workspace, size_t 
             q.batch = 1;
             q.c_b = 0;
         }
-        if (q.ws_vec) {
+        if (q.ws_vec && q.splits >= kSliceMinSplits && q.batch == 1 && (!q.csum || q.csum_rows)) {
+            const dim3 grid((unsigned)std::min<int64_t>((N + 63) / 64, 1024),
+                            (unsigned)std::min<int64_t>(M, 65535));
+            if (q.csum)
+                hipLaunchKernelGGL(splitk_reduce_slices_f32<true>, grid, dim3(256), 0, stream, q);
+            else
+                hipLaunchKernelGGL(splitk_reduce_slices_f32<false>, grid, dim3(256), 0, stream, q);
+        } else if (q.ws_vec) {
             const int nt =
                 q.csum && !q.csum_rows ? csum_threads((int64_t)q.csum_n * q.csum_hw) : 256;
             const dim3 grid((unsigned)std::min<int64_t>((N / 4 + nt - 1) / nt, 64),
@@ -1544,6 +1617,49 @@ hipError_t launch_pad_channels(const float* in, float* out, int64_t n, int C, in
     return capture_safe_last_error();
 }
 
+// out[b][q][c] = c < C ? in[b][c][q] : 0 for c < CP, CP % 4 == 0: dense NCHW to
+// channels-last, padded with zero channels (b = image, q = pixel; or OIHW
+// weights to OHWI with b = output channel, q = tap).  A thread takes four
+// channels of one position: coalesced reads along q, one 16-byte store.  Two
+// jobs in one launch, the blocks of job 0 first.  The 224x224 RGB stem at batch
+// 32 moves 45 MB.
+struct PadJob {
+    const float* in;
+    float* out;
+    int C, CP;
+    int64_t B, HW;
+    int64_t items() const { return B * HW * (CP / 4); }
+};
+__global__ void __launch_bounds__(256)
+pad_channels_last_f32(PadJob j0, PadJob j1, int64_t n0, int64_t n1, unsigned blocks0) {
+    const bool second = blockIdx.x >= blocks0;
+    const PadJob j = second ? j1 : j0;
+    const int64_t n = second ? n1 : n0;
+    const int64_t blocks = second ? gridDim.x - blocks0 : blocks0;
+    for (int64_t e = (blockIdx.x - (second ? blocks0 : 0)) * 256ll + threadIdx.x; e < n;
+         e += blocks * 256) {
+        const int64_t bq = e / j.HW, q = e - bq * j.HW;
+        const int64_t b = bq / (j.CP / 4);
+        const int c = 4 * (int)(bq - b * (j.CP / 4));
+        f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+            if (c + x < j.C) v[x] = j.in[(b * j.C + c + x) * j.HW + q];
+        *reinterpret_cast<f32x4*>(j.out + (b * j.HW + q) * j.CP + c) = v;
+    }
+}
+
+hipError_t launch_pad_channels_last(const PadJob& a, const PadJob& b, hipStream_t s) {
+    const int64_t na = a.items(), nb = b.items();
+    const auto blocks = [](int64_t n) {
+        return (unsigned)std::min<int64_t>((n + 255) / 256, 1 << 16);
+    };
+    if (na + nb == 0) return hipSuccess;
+    hipLaunchKernelGGL(pad_channels_last_f32, dim3(blocks(na) + blocks(nb)), dim3(256), 0, s, a, b,
+                       na, nb, blocks(na));
+    return capture_safe_last_error();
+}
+
 // db[c] = beta*db[c] + Σ_{img, hw} dY[img][c][hw]; one workgroup per channel
 // (block_channel_sum: fixed order, deterministic).
 template <int NT>
@@ -1784,6 +1900,38 @@ hipError_t launch_im2col(const mt_conv2d_desc* d, int64_t Ho, int64_t Wo, const 
     return capture_safe_last_error();
 }
 
+// C[c_out, np] = wt[c_out, kg] · im2col(xt)[kg, np], k = (r*kw + s)*c_in + ci, over
+// a channels-last input and OHWI weights; lb: L_IM (c_in % 16 == 0) or L_IM4.
+int run_conv_cl(const mt_conv2d_desc* d, int64_t Ho, int64_t Wo, const float* xt,
+                int64_t img_stride, const float* wt, const float* bias, float* output, int lb,
+                void* workspace, size_t ws_bytes, hipStream_t s) {
+    const int64_t c = d->c_in, kg = c * d->kh * d->kw, hw = Ho * Wo, np = d->n * hw;
+    GemmParams p{};
+    p.A = wt; p.a_mn = kg; p.a_k = 1; p.a_b = 0;
+    p.B = xt;
+    p.C = output; p.c_m = hw; p.c_n = 1; p.c_b = 0;
+    p.c_n_inner = hw; p.c_n_outer = d->c_out * hw;
+    p.bias = bias; p.bias_stride = 1; p.bias_axis = bias ? MT_BIAS_ROW : MT_BIAS_NONE;
+    p.beta = 0.f;
+    p.M = (int)d->c_out; p.N = (int)np; p.K = (int)kg; p.batch = 1;
+    ConvGeom& g = p.cv;
+    g.img_stride = img_stride;
+    g.c = (int)c; g.h = (int)d->h; g.w = (int)d->w;
+    g.kh = (int)d->kh; g.kw = (int)d->kw; g.stride = (int)d->stride; g.pad = g.pad_w = (int)d->pad;
+    g.ho = (int)Ho; g.wo = (int)Wo;
+    return launch_gemm(p, true, L_KV, lb, workspace, ws_bytes, s);
+}
+
+// Whether run_conv_cl takes d as L_IM4: gemm_f32_sp's form alone, with 32-bit
+// tap offsets and weight rows within a tile (sp_fits).
+bool im4_fits(const mt_conv2d_desc* d) {
+    constexpr int64_t kMax = (int64_t)1 << 30;
+    return g_forced.family == MT_FAMILY_AUTO && (d->c_in & 3) == 0 &&
+           d->h + 2 * d->pad < kMax && d->w + 2 * d->pad < kMax &&
+           mul_capped(mul_capped(d->kh, d->w), d->c_in) >= 0 && d->kh * d->w * d->c_in < kMax &&
+           (kSpMaxRows - 1) * d->c_in * d->kh * d->kw < kMax - 16;
+}
+
 // Implicit-GEMM convolution: C[c_out, np] = Wt[c_out, kg] · im2col(xt)[kg, np]
 // with k = (r*kw + s)*c_in + ci, the im2col operand gathered by the kernel
 // from a channels-last input xt (the input itself when it already is one,
@@ -1794,7 +1942,7 @@ int run_conv_implicit(const mt_conv2d_desc* d, int64_t Ho, int64_t Wo, const flo
                       const int64_t in_strides[4], const float* bias, float* output, char* wsp,
                       size_t ws_bytes, const TJob& wjob, hipStream_t s) {
     const ImplicitWs iw = implicit_ws(d);
-    const int64_t c = d->c_in, kg = c * d->kh * d->kw, hw = Ho * Wo, np = d->n * hw;
+    const int64_t c = d->c_in;
     const bool nhwc = in_strides[1] == 1 && in_strides[3] == c && in_strides[2] == d->w * c &&
                       (in_strides[0] & 3) == 0 && ((uintptr_t)input & 15u) == 0;
     const float* xt = input;
@@ -1808,20 +1956,8 @@ int run_conv_implicit(const mt_conv2d_desc* d, int64_t Ho, int64_t Wo, const flo
         img_stride = d->h * d->w * c;
     }
     if (launch_transposes(xjob, wjob, s) != hipSuccess) return MT_ERR_HIP;
-    GemmParams p{};
-    p.A = reinterpret_cast<const float*>(wsp + iw.xt); p.a_mn = kg; p.a_k = 1; p.a_b = 0;
-    p.B = xt;
-    p.C = output; p.c_m = hw; p.c_n = 1; p.c_b = 0;
-    p.c_n_inner = hw; p.c_n_outer = d->c_out * hw;
-    p.bias = bias; p.bias_stride = 1; p.bias_axis = bias ? MT_BIAS_ROW : MT_BIAS_NONE;
-    p.beta = 0.f;
-    p.M = (int)d->c_out; p.N = (int)np; p.K = (int)kg; p.batch = 1;
-    ConvGeom& g = p.cv;
-    g.img_stride = img_stride;
-    g.c = (int)c; g.h = (int)d->h; g.w = (int)d->w;
-    g.kh = (int)d->kh; g.kw = (int)d->kw; g.stride = (int)d->stride; g.pad = g.pad_w = (int)d->pad;
-    g.ho = (int)Ho; g.wo = (int)Wo;
-    return launch_gemm(p, true, L_KV, L_IM, wsp + iw.xt + iw.wt, ws_bytes - iw.xt - iw.wt, s);
+    return run_conv_cl(d, Ho, Wo, xt, img_stride, reinterpret_cast<const float*>(wsp + iw.xt), bias,
+                       output, L_IM, wsp + iw.xt + iw.wt, ws_bytes - iw.xt - iw.wt, s);
 }
 
 // The implicit-GEMM convolution over an NCHW view (L_IMR) reads the OIHW
@@ -1927,9 +2063,12 @@ DwPadWs dw_pad_ws(const mt_conv2d_desc* d4) {
 
 // The forward of a layer that would take the column path because c_in*kh*kw
 // % 4 != 0, with a kernel of at least 25 taps (the 7x7 RGB stem) and c_in
-// rounded up to 4 adding at most a third of the work: the NCHW-view kernel on
-// the input and weights padded with zero channels (d4).  The stem at batch 32:
-// 178.5 us against 187.5 on the column path.
+// rounded up to 4 adding at most a third of the work: on the input and weights
+// padded with zero channels (d4), channels-last, so that four k are one 16-byte
+// load (L_IM4; the NCHW-view kernel, whose 4-byte loads were four times as
+// many, where a configuration without L_IM4 is forced or its 32-bit tap offsets
+// do not reach).  The stem at batch 32: 115 us, 178.5 on the NCHW view, 187.5
+// on the column path.
 bool fwd_padded(const mt_conv2d_desc* d, mt_conv2d_desc* d4) {
     if (d->c_in <= 0 || (d->c_in & 3) == 0 || d->kh * d->kw < 25) return false;
     const int64_t cp = (d->c_in + 3) / 4 * 4;
@@ -2186,16 +2325,21 @@ bool dx_prefer_phased(const mt_conv2d_desc* d, int64_t Ho, int64_t Wo, bool cl) 
 // Workspace of one implicit-operand GEMM (L_IM / L_IMR: the direct-to-LDS
 // configurations 0-3 and 7; L_IMW, imw: 0-6),
 // including a forced configuration's partials: what launch_gemm may use.
-size_t implicit_gemm_ws(int64_t M, int64_t N, int64_t K, bool imw) {
+size_t implicit_gemm_ws(int64_t M, int64_t N, int64_t K, bool imw, bool im4 = false) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     const int cus = device_cu_count();
     size_t ws = 0;
     for (bool sp : {false, true}) {
-        ws = std::max(ws, make_plan(M, N, K, 1, cus, true, true, imw, false, sp, imw).ws_bytes);
+        const Plan pl = make_plan(M, N, K, 1, cus, true, true, imw, false, sp, imw);
+        // (with the weight gradient's row sums: M floats per split)
+        ws = std::max(ws, pl.ws_bytes + (imw && pl.splits > 1 ? (size_t)pl.splits * M * 4 : 0));
         if (!imw && kOfferNarrow)   // the channels-last operand may take the 16x16-block kernel
             ws = std::max(ws,
                           make_plan(M, N, K, 1, cus, true, true, false, false, sp, false, true).ws_bytes);
     }
+    if (im4)
+        ws = std::max(ws, make_plan(M, N, K, 1, cus, true, true, false, false, true, false, false,
+                                    true).ws_bytes);
     Plan f;
     if (forced_plan(M, N, K, 1, true, false, imw, true, &f, !imw)) ws = std::max(ws, f.ws_bytes);
     return ws;
@@ -2471,7 +2615,7 @@ size_t mt_conv2d_workspace_f32(const mt_conv2d_desc* d) {
     if (fwd_padded(d, &d4)) {
         const DwPadWs pw = dw_pad_ws(&d4);
         return std::max(col, pw.xp + pw.dw4 +
-                                 implicit_gemm_ws(d->c_out, np, d4.c_in * d->kh * d->kw, false));
+                                 implicit_gemm_ws(d->c_out, np, d4.c_in * d->kh * d->kw, false, true));
     }
     return col;
 }
@@ -2545,6 +2689,15 @@ int mt_conv2d_fwd_strided_f32(const mt_conv2d_desc* d, const float* input,
         char* wsp = static_cast<char*>(workspace);
         float* xp = reinterpret_cast<float*>(wsp);
         float* wp = reinterpret_cast<float*>(wsp + pw.xp);
+        if (im4_fits(&d4)) {
+            if (launch_pad_channels_last(
+                    PadJob{input, xp, (int)d->c_in, (int)d4.c_in, d->n, d->h * d->w},
+                    PadJob{weight, wp, (int)d->c_in, (int)d4.c_in, d->c_out, d->kh * d->kw}, s) !=
+                hipSuccess)
+                return MT_ERR_HIP;
+            return run_conv_cl(&d4, Ho, Wo, xp, d->h * d->w * d4.c_in, wp, bias, output, L_IM4,
+                               wsp + pw.xp + pw.dw4, ws_bytes - pw.xp - pw.dw4, s);
+        }
         if (launch_pad_channels(input, xp, d->n, (int)d->c_in, (int)d4.c_in, d->h * d->w, s) !=
                 hipSuccess ||
             launch_pad_channels(weight, wp, d->c_out, (int)d->c_in, (int)d4.c_in,
@@ -2592,10 +2745,12 @@ namespace {
 
 // dW (+ beta·dW).  With grad_bias, the implicit path also hands db
 // (+ beta_b·db) to the split-K reduction of its GEMM when the plan has one
-// (GemmParams::csum); *db_done reports whether it did.
+// (GemmParams::csum); *db_done reports whether it did.  input_cl: the input
+// as a channels-last copy (implicit_dw geometries only), in place of `input`.
 int conv_bwd_weight(const mt_conv2d_desc* d, const float* input, const float* grad_out,
                     float* grad_weight, float beta, float* grad_bias, float beta_b,
-                    void* workspace, size_t ws_bytes, hipStream_t s, bool* db_done) {
+                    void* workspace, size_t ws_bytes, hipStream_t s, bool* db_done,
+                    const float* input_cl = nullptr) {
     *db_done = false;
     int64_t Ho, Wo;
     if (!conv_dims(d, &Ho, &Wo)) return MT_ERR_INVALID;
@@ -2604,8 +2759,8 @@ int conv_bwd_weight(const mt_conv2d_desc* d, const float* input, const float* gr
     if (!grad_weight) return MT_ERR_INVALID;
     const size_t col_b = align_up((size_t)kg * np * sizeof(float), 256);
     const size_t dyt_b = align_up((size_t)d->c_out * np * sizeof(float), 256);
-    if (np > 0 && (!input || !grad_out)) return MT_ERR_INVALID;
-    if (pointwise_strided(d, Ho, Wo)) {
+    if (np > 0 && ((!input && !input_cl) || !grad_out)) return MT_ERR_INVALID;
+    if (!input_cl && pointwise_strided(d, Ho, Wo)) {
         // A strided 1x1 layer reads only x[oh*s][ow*s]: those pixels copied
         // out (n*c_in*Ho*Wo floats), then the batch-summed 1x1 product on
         // them.  The 56x56 256 -> 512 shortcut at batch 32: dW + db 81 against
@@ -2622,7 +2777,7 @@ int conv_bwd_weight(const mt_conv2d_desc* d, const float* input, const float* gr
         return conv_bwd_weight(&d1, xs, grad_out, grad_weight, beta, grad_bias, beta_b,
                                static_cast<char*>(workspace) + xs_b, ws_bytes - xs_b, s, db_done);
     }
-    if (pointwise(d) && np > 0) {
+    if (!input_cl && pointwise(d) && np > 0) {
         // dW[c_out][c_in] = Σ_b dY_b[c_out][hw] · X_b[c_in][hw]ᵀ: one product per
         // image into the workspace, summed (with beta·dW, and db as the channel
         // sums of dY) by the reduction launch.
@@ -2657,11 +2812,19 @@ int conv_bwd_weight(const mt_conv2d_desc* d, const float* input, const float* gr
         char* wsp = static_cast<char*>(workspace);
         float* xp = reinterpret_cast<float*>(wsp);
         float* dw4 = reinterpret_cast<float*>(wsp + pw.xp);
-        if (launch_pad_channels(input, xp, d->n, (int)d->c_in, (int)d4.c_in, d->h * d->w, s) !=
-            hipSuccess)
-            return MT_ERR_HIP;
-        const int rc = conv_bwd_weight(&d4, xp, grad_out, dw4, 0.f, grad_bias, beta_b,
-                                       wsp + pw.xp + pw.dw4, ws_bytes - pw.xp - pw.dw4, s, db_done);
+        // a 1x1 layer reads the padded NCHW input (per-image products), others a
+        // channels-last one
+        const bool nchw = pointwise(&d4) || pointwise_strided(&d4, Ho, Wo);
+        const hipError_t e =
+            nchw ? launch_pad_channels(input, xp, d->n, (int)d->c_in, (int)d4.c_in, d->h * d->w, s)
+                 : launch_pad_channels_last(
+                       PadJob{input, xp, (int)d->c_in, (int)d4.c_in, d->n, d->h * d->w}, PadJob{},
+                       s);
+        if (e != hipSuccess) return MT_ERR_HIP;
+        const int rc = conv_bwd_weight(&d4, nchw ? xp : nullptr, grad_out, dw4, 0.f, grad_bias,
+                                       beta_b, wsp + pw.xp + pw.dw4,
+                                       ws_bytes - pw.xp - pw.dw4, s, db_done,
+                                       nchw ? nullptr : xp);
         if (rc != MT_OK) return rc;
         // dW[co][ci*khw + t] = beta*dW + dW4[co][ci*khw + t] for the real channels ci
         const int64_t khw = d->kh * d->kw;
@@ -2689,8 +2852,9 @@ int conv_bwd_weight(const mt_conv2d_desc* d, const float* input, const float* gr
         float* dyt = reinterpret_cast<float*>(wsp + xt_b);
         int64_t st[4];
         dense_strides(d, st);
-        if (launch_transposes(tjob(input, st[0], st[1], st[2], st[3], d->w, d->c_in, d->h * d->w,
-                                   d->n, xt),
+        if (launch_transposes(input_cl ? TJob{}
+                                       : tjob(input, st[0], st[1], st[2], st[3], d->w, d->c_in,
+                                              d->h * d->w, d->n, xt),
                               kvi ? TJob{}
                                   : tjob(grad_out, hw, 1, d->c_out * hw, 0, 1, hw, d->n, d->c_out,
                                          dyt),
@@ -2703,7 +2867,7 @@ int conv_bwd_weight(const mt_conv2d_desc* d, const float* input, const float* gr
         } else {
             p.A = dyt; p.a_mn = np; p.a_k = 1; p.a_b = 0;
         }
-        p.B = xt;
+        p.B = input_cl ? input_cl : xt;
         p.C = grad_weight; p.c_m = kg; p.c_n = d->kh * d->kw; p.c_b = 0;
         p.c_n_inner = d->c_in; p.c_n_outer = 1;
         p.bias = nullptr; p.bias_stride = 0; p.bias_axis = MT_BIAS_NONE;
@@ -2717,6 +2881,7 @@ int conv_bwd_weight(const mt_conv2d_desc* d, const float* input, const float* gr
         if (grad_bias) {
             p.csum_src = grad_out; p.csum = grad_bias; p.csum_n = (int)d->n;
             p.csum_hw = hw; p.csum_beta = beta_b;
+            p.rowsum = grad_bias;   // as partials, where the plan can take them
         }
         const int rc = launch_gemm(p, true, kvi ? L_KVI : L_KV, L_IMW, wsp + xt_b + dyb,
                                    ws_bytes - xt_b - dyb, s);
