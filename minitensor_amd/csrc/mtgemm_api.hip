@@ -1013,22 +1013,29 @@ __device__ __forceinline__ void channel_sum(const GemmParams& p, int m, float* r
     if (threadIdx.x == 0) p.csum[m] = (p.csum_beta != 0.f ? p.csum_beta * p.csum[m] : 0.f) + r;
 }
 
-// One group of four output columns of the vector forms: bias and beta·C added
-// to v, stored as one 16-byte vector when C allows (c_vec), else element by
-// element through col(n).
-__device__ __forceinline__ void reduce_store(const GemmParams& p, float* crow, int n, float brow,
-                                             f32x4 v) {
-    f32x4 bcol = {0.f, 0.f, 0.f, 0.f}, old = bcol;
+// The epilogue of one group of four output columns of the vector forms: its
+// loads, issued before the sum of the partials, then bias and beta·C added to
+// the sum and one 16-byte store when C allows (c_vec), else element by element
+// through col(n).
+struct ReduceGroup {
+    f32x4 bcol, old;
+};
+__device__ __forceinline__ ReduceGroup reduce_load(const GemmParams& p, const float* crow, int n) {
+    ReduceGroup g{f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
     if (p.bias_axis == 2)
-        for (int e = 0; e < 4; ++e) bcol[e] = p.bias[(int64_t)(n + e) * p.bias_stride];
+        for (int e = 0; e < 4; ++e) g.bcol[e] = p.bias[(int64_t)(n + e) * p.bias_stride];
     if (p.beta != 0.f) {
-        if (p.c_vec) old = *reinterpret_cast<const f32x4*>(crow + col_offset(p, n));
+        if (p.c_vec) g.old = *reinterpret_cast<const f32x4*>(crow + col_offset(p, n));
         else
-            for (int e = 0; e < 4; ++e) old[e] = crow[col_offset(p, n + e)];
+            for (int e = 0; e < 4; ++e) g.old[e] = crow[col_offset(p, n + e)];
     }
+    return g;
+}
+__device__ __forceinline__ void reduce_store(const GemmParams& p, float* crow, int n, float brow,
+                                             const ReduceGroup& g, f32x4 v) {
     v += brow;
-    if (p.bias_axis == 2) v += bcol;
-    if (p.beta != 0.f) v += p.beta * old;
+    if (p.bias_axis == 2) v += g.bcol;
+    if (p.beta != 0.f) v += p.beta * g.old;
     if (p.c_vec) {
         *reinterpret_cast<f32x4*>(crow + col_offset(p, n)) = v;
     } else {
@@ -1056,9 +1063,11 @@ __global__ void __launch_bounds__(NT) splitk_reduce_vec_f32(GemmParams p) {
         const float* src = p.ws + (int64_t)bz * MN + (int64_t)m * p.N;
         float* crow = p.C + (int64_t)bz * p.c_b + (int64_t)m * p.c_m;
         for (int n = (blockIdx.x * blockDim.x + threadIdx.x) * 4; n < p.N;
-             n += gridDim.x * blockDim.x * 4)
-            reduce_store(p, crow, n, brow,
-                         sum_partials<f32x4>(src + n, p.batch * MN, p.splits, zero));
+             n += gridDim.x * blockDim.x * 4) {
+            const ReduceGroup g = reduce_load(p, crow, n);
+            const f32x4 v = sum_partials<f32x4>(src + n, p.batch * MN, p.splits, zero);
+            reduce_store(p, crow, n, brow, g, v);
+        }
     }
 }
 
@@ -1066,9 +1075,11 @@ __global__ void __launch_bounds__(NT) splitk_reduce_vec_f32(GemmParams p) {
 // walks all of them in turn, eight loads at a time, and there are few threads
 // (the RGB stem's dW, 64 x 196 in 512 slabs: 3136 threads, 41 us for 26 MB).
 // Here 16 slices of the slabs go side by side, 16 column groups of 4 each, and
-// their sums meet in LDS in a fixed order: 12 us.  CSUM: the row sums from
-// GemmParams::csum_rows.
+// their sums meet in LDS in a fixed order: 12 us.  Outputs with threads enough
+// for the form above stay there (512 x 256 in 32 slabs: 9.1 us, 14.1 here).
+// CSUM: the row sums from GemmParams::csum_rows.
 constexpr int kSliceMinSplits = 32;
+constexpr int64_t kSliceMaxOutputs = 64 * 1024;   // a wave per CU of four outputs a thread
 template <bool CSUM>
 __global__ void __launch_bounds__(256) splitk_reduce_slices_f32(GemmParams p) {
     __shared__ f32x4 part[16][16];
@@ -1092,7 +1103,7 @@ __global__ void __launch_bounds__(256) splitk_reduce_slices_f32(GemmParams p) {
                 f32x4 v = part[0][col];
 #pragma unroll
                 for (int i = 1; i < 16; ++i) v += part[i][col];
-                reduce_store(p, crow, n, brow, v);
+                reduce_store(p, crow, n, brow, reduce_load(p, crow, n), v);
             }
             __syncthreads();
         }
@@ -1284,7 +1295,8 @@ int launch_gemm(GemmParams& p, bool dl, int la, int lb, void* workspace, size_t 
             q.batch = 1;
             q.c_b = 0;
         }
-        if (q.ws_vec && q.splits >= kSliceMinSplits && q.batch == 1 && (!q.csum || q.csum_rows)) {
+        if (q.ws_vec && q.splits >= kSliceMinSplits && M * N <= kSliceMaxOutputs &&
+            q.batch == 1 && (!q.csum || q.csum_rows)) {
             const dim3 grid((unsigned)std::min<int64_t>((N + 63) / 64, 1024),
                             (unsigned)std::min<int64_t>(M, 65535));
             if (q.csum)
@@ -1725,6 +1737,58 @@ hipError_t launch_pad_channels_last(const PadJob& a, const PadJob& b, hipStream_
     if (na + nb == 0) return hipSuccess;
     hipLaunchKernelGGL(pad_channels_last_f32, dim3(blocks(na) + blocks(nb)), dim3(256), 0, s, a, b,
                        na, nb, blocks(na));
+    return capture_safe_last_error();
+}
+
+// out[b][c][oh][ow] = x[b*sn + c*sc + oh*st*sh + ow*st*sw], dense: the pixels a
+// strided 1x1 layer reads.  A thread makes V consecutive outputs of a row (V = 4:
+// one 16-byte store; PAIR: stride 2 over contiguous aligned rows, two 16-byte
+// loads).  The 56x56 layer of 256 channels at batch 32 touches 77 MB: 16.4 us
+// against 26 one pixel per thread.
+struct SubView {
+    const float* x;
+    int64_t sn, sc, sh, sw;
+    int st;
+};
+template <int V, bool PAIR>
+__global__ void __launch_bounds__(256)
+subsample_f32(SubView in, float* out, int64_t total, int C, int Ho, int Wo) {
+    const int wq = Wo / V;
+    for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < total;
+         e += (int64_t)gridDim.x * 256) {
+        const int64_t row = total < ((int64_t)1 << 32) ? (uint32_t)e / (uint32_t)wq : e / wq;
+        const int ow = (int)(e - row * wq) * V;
+        const int64_t plane = row / Ho;
+        const int oh = (int)(row - plane * Ho);
+        const int64_t b = plane / C;
+        const float* src = in.x + b * in.sn + (plane - b * C) * in.sc +
+                           (int64_t)oh * in.st * in.sh + (int64_t)ow * in.st * in.sw;
+        if constexpr (PAIR) {
+            const f32x4 lo = *reinterpret_cast<const f32x4*>(src);
+            const f32x4 hi = *reinterpret_cast<const f32x4*>(src + 4);
+            *reinterpret_cast<f32x4*>(out + e * 4) = f32x4{lo[0], lo[2], hi[0], hi[2]};
+        } else if constexpr (V == 4) {
+            f32x4 v;
+#pragma unroll
+            for (int x = 0; x < 4; ++x) v[x] = src[(int64_t)x * in.st * in.sw];
+            *reinterpret_cast<f32x4*>(out + e * 4) = v;
+        } else {
+            out[e] = src[0];
+        }
+    }
+}
+
+// out is 16-byte aligned (a workspace).
+hipError_t launch_subsample(const SubView& in, float* out, int64_t n, int64_t C, int64_t W,
+                            int64_t Ho, int64_t Wo, hipStream_t s) {
+    const bool v4 = (Wo & 3) == 0;
+    const int64_t total = n * C * Ho * (v4 ? Wo / 4 : Wo);
+    if (total == 0) return hipSuccess;
+    const bool pair = v4 && in.st == 2 && in.sw == 1 && 2 * Wo <= W && ((uintptr_t)in.x & 15u) == 0 &&
+                      (in.sh & 1) == 0 && (in.sc & 3) == 0 && (in.sn & 3) == 0;
+    auto k = pair ? subsample_f32<4, true> : v4 ? subsample_f32<4, false> : subsample_f32<1, false>;
+    const unsigned grid = (unsigned)std::min<int64_t>((total + 255) / 256, 1 << 16);
+    hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, s, in, out, total, (int)C, (int)Ho, (int)Wo);
     return capture_safe_last_error();
 }
 
@@ -2291,58 +2355,65 @@ struct DxPhaseOut {
 };
 
 // dX[plane][ih][iw] = z[(ih%S)*S + iw%S][plane][ih/S][iw/S], plane = img*c_in
-// + ci: blockIdx.y walks planes, threads walk items of V pixels of one row,
-// stored as one 16-byte vector when V == 4 (W % 4 == 0, aligned).  The phase
-// is chosen by compares against every index (an indexed read of the argument
-// arrays would go through scratch).  Reads and writes dX's bytes once each.
-template <int S, int V>
+// + ci: threads walk items of V pixels of one row, stored as one 16-byte
+// vector when V == 4 (W % 4 == 0, aligned); whole blocks over all planes (784
+// items of a 56x56 plane had left the last of its four blocks nearly empty:
+// 34.7 us for 129 MB, now 29.5).  The phase is chosen by compares against every
+// index (an indexed read of the argument arrays would go through scratch).
+// Reads and writes dX's bytes once each.
+template <int S, int V, class I>
 __global__ void __launch_bounds__(256)
-dx_interleave_f32(DxPhaseOut o, float* dx, int64_t planes, int H, int W) {
-    const int wq = W / V;
-    const int per = H * wq;
-    for (int64_t plane = blockIdx.y; plane < planes; plane += gridDim.y) {
-        float* dplane = dx + plane * H * W;
-        for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < per; q += gridDim.x * blockDim.x) {
-            const int ih = q / wq, iw0 = (q - ih * wq) * V;
-            const int ph = ih % S, i = ih / S;
-            float v[V];
+dx_interleave_f32(DxPhaseOut o, float* dx, int64_t total, int H, int W) {
+    const I wq = W / V;
+    for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < total;
+         e += (int64_t)gridDim.x * 256) {
+        const I row = (I)e / wq;
+        const int iw0 = (int)((I)e - row * wq) * V;
+        const I plane = row / (I)H;
+        const int ih = (int)(row - plane * (I)H);
+        const int ph = ih % S, i = ih / S;
+        float v[V];
 #pragma unroll
-            for (int e = 0; e < V; ++e) {
-                const int iw = iw0 + e;
-                const int f = ph * S + iw % S;
-                const float* z = o.z[0];
-                int hp = o.hp[0], wp = o.wp[0];
+        for (int x = 0; x < V; ++x) {
+            const int iw = iw0 + x;
+            const int f = ph * S + iw % S;
+            const float* z = o.z[0];
+            int hp = o.hp[0], wp = o.wp[0];
 #pragma unroll
-                for (int c = 1; c < S * S; ++c)
-                    if (f == c) {
-                        z = o.z[c];
-                        hp = o.hp[c];
-                        wp = o.wp[c];
-                    }
-                v[e] = z ? z[(plane * hp + i) * wp + iw / S] : 0.f;
-            }
-            float* dst = dplane + (int64_t)ih * W + iw0;
-            if constexpr (V == 4)
-                *reinterpret_cast<f32x4*>(dst) = f32x4{v[0], v[1], v[2], v[3]};
-            else
-                dst[0] = v[0];
+            for (int c = 1; c < S * S; ++c)
+                if (f == c) {
+                    z = o.z[c];
+                    hp = o.hp[c];
+                    wp = o.wp[c];
+                }
+            v[x] = z ? z[((int64_t)plane * hp + i) * wp + iw / S] : 0.f;
         }
+        float* dst = dx + e * V;
+        if constexpr (V == 4)
+            *reinterpret_cast<f32x4*>(dst) = f32x4{v[0], v[1], v[2], v[3]};
+        else
+            dst[0] = v[0];
     }
 }
 
 // For strides 2-4 (at stride 1 the one phase is dX itself).
+template <int S>
+void run_dx_interleave(const DxPhaseOut& o, float* dx, int64_t planes, int H, int W, hipStream_t st) {
+    const bool vec = (W & 3) == 0 && ((uintptr_t)dx & 15u) == 0;
+    const int64_t total = planes * H * (vec ? W / 4 : W);
+    const bool narrow = total < ((int64_t)1 << 32);   // 32-bit divisions
+    auto k = vec ? (narrow ? dx_interleave_f32<S, 4, uint32_t> : dx_interleave_f32<S, 4, int64_t>)
+                 : (narrow ? dx_interleave_f32<S, 1, uint32_t> : dx_interleave_f32<S, 1, int64_t>);
+    const unsigned grid = (unsigned)std::min<int64_t>((total + 255) / 256, 1 << 16);
+    hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, st, o, dx, total, H, W);
+}
 hipError_t launch_dx_interleave(const DxPhaseOut& o, int s, float* dx, int64_t planes, int H,
                                 int W, hipStream_t st) {
     if (s < 2 || s > kDxMaxStride) return hipErrorInvalidValue;
-    const bool vec = (W & 3) == 0 && ((uintptr_t)dx & 15u) == 0;
-    const int per = H * (vec ? W / 4 : W);
-    const dim3 grid((unsigned)std::min<int64_t>((per + 255) / 256, 1024),
-                    (unsigned)std::min<int64_t>(planes, 65535));
-    if (planes == 0 || per == 0) return hipSuccess;
-    auto k = s == 2 ? (vec ? dx_interleave_f32<2, 4> : dx_interleave_f32<2, 1>)
-             : s == 3 ? (vec ? dx_interleave_f32<3, 4> : dx_interleave_f32<3, 1>)
-                      : (vec ? dx_interleave_f32<4, 4> : dx_interleave_f32<4, 1>);
-    hipLaunchKernelGGL(k, grid, dim3(256), 0, st, o, dx, planes, H, W);
+    if (planes == 0 || H == 0 || W == 0) return hipSuccess;
+    s == 2   ? run_dx_interleave<2>(o, dx, planes, H, W, st)
+    : s == 3 ? run_dx_interleave<3>(o, dx, planes, H, W, st)
+             : run_dx_interleave<4>(o, dx, planes, H, W, st);
     return capture_safe_last_error();
 }
 
@@ -2675,7 +2746,10 @@ size_t mt_conv2d_workspace_f32(const mt_conv2d_desc* d) {
                         nchw_weight_ws(d) + implicit_gemm_ws(d->c_out, np, kg, false));
     if (implicit_geometry(d) && d->h * d->w < kMaxDim) {   // channels-last kernel
         const ImplicitWs iw = implicit_ws(d);
-        return iw.xt + iw.wt + implicit_gemm_ws(d->c_out, np, kg, false);
+        const size_t cl = iw.xt + iw.wt + implicit_gemm_ws(d->c_out, np, kg, false);
+        if (!pointwise_strided(d, Ho, Wo)) return cl;
+        return std::max(cl, pointwise_strided_zb(d, Ho, Wo) +
+                                plan_ws(d->c_out, Ho * Wo, d->c_in, d->n, device_cu_count()));
     }
     // the NCHW-view kernel: split-K partials, and room for an aligned copy of
     // the weights (used only when the caller's are not 16-byte aligned)
@@ -2726,6 +2800,24 @@ int mt_conv2d_fwd_strided_f32(const mt_conv2d_desc* d, const float* input,
         if (!workspace || ws_bytes < iw.xt + iw.wt || ((uintptr_t)workspace & 15u) != 0)
             return MT_ERR_WORKSPACE;
         char* wsp = static_cast<char*>(workspace);
+        // A strided 1x1 layer: the pixels that it reads copied out, then one
+        // product per image, as in its dW (56x56, 256 -> 512 channels, stride 2
+        // at batch 32: 86 us against 112 through the channels-last copy of
+        // the whole input).  A channels-last input is gathered in place.
+        if (pointwise_strided(d, Ho, Wo) && g_forced.family == MT_FAMILY_AUTO &&
+            in_strides[1] != 1) {
+            const size_t xs_b = pointwise_strided_zb(d, Ho, Wo);
+            const SubView in{input, in_strides[0], in_strides[1], in_strides[2], in_strides[3],
+                             (int)d->stride};
+            float* xs = reinterpret_cast<float*>(wsp);
+            if (launch_subsample(in, xs, d->n, d->c_in, d->w, Ho, Wo, s) != hipSuccess)
+                return MT_ERR_HIP;
+            const int64_t dense[4] = {d->c_in * hw, hw, Wo, 1};
+            mt_conv2d_desc d1 = *d;
+            d1.h = Ho; d1.w = Wo; d1.stride = 1;
+            return mt_conv2d_fwd_strided_f32(&d1, xs, dense, weight, bias, output, wsp + xs_b,
+                                             ws_bytes - xs_b, s);
+        }
         float* wt = reinterpret_cast<float*>(wsp + iw.xt);      // OIHW -> OHWI
         const TJob wjob = tjob(weight, kg, d->kh * d->kw, d->kw, 1, d->kw, d->c_in,
                                d->kh * d->kw, d->c_out, wt);
@@ -2841,8 +2933,8 @@ int conv_bwd_weight(const mt_conv2d_desc* d, const float* input, const float* gr
         if (!workspace || ws_bytes < xs_b || ((uintptr_t)workspace & 15u) != 0)
             return MT_ERR_WORKSPACE;
         float* xs = static_cast<float*>(workspace);
-        if (launch_axpby(input, d->h * d->w, d->stride * d->w, d->stride, 1.f, xs, hw, Wo, 1, 0.f,
-                         d->n * d->c_in, Ho, Wo, s) != hipSuccess)
+        const SubView in{input, d->c_in * d->h * d->w, d->h * d->w, d->w, 1, (int)d->stride};
+        if (launch_subsample(in, xs, d->n, d->c_in, d->w, Ho, Wo, s) != hipSuccess)
             return MT_ERR_HIP;
         mt_conv2d_desc d1 = *d;
         d1.h = Ho; d1.w = Wo; d1.stride = 1;
