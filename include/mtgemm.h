@@ -264,11 +264,12 @@ const char* mt_last_config(void);
 enum {
     MT_FAMILY_AUTO = 0,  /* the cost model chooses (default)                   */
     MT_FAMILY_RS = 1,    /* register-staged kernel: any operand layout          */
-    MT_FAMILY_DL = 2,    /* direct-to-LDS kernel: k- or mn-contiguous operands;
-                            configurations 0-3 gemm_f32_dl, 4-6 with fragment
-                            prefetch (not the channels-last convolution
-                            operand), 7 the channels-last convolution operand
-                            only (64x112 tiles of 16x16 MFMA blocks)          */
+    MT_FAMILY_DL = 2,    /* k- or mn-contiguous operands of 16-byte alignment:
+                            configurations 0 (64x256), 1 (128x128), 3 (256x128),
+                            4 (128x256) and 6 (128x64) on the bf16 matrix units,
+                            2 and 5 (64x64) direct-to-LDS on the fp32 ones; 4-6
+                            not for the channels-last convolution operand, 7
+                            (64x112, bf16 units) for that one only             */
     MT_FAMILY_KSW = 3,   /* wave-split kernel: small tiles, K split across the
                             waves of a workgroup; any operand layout;
                             configurations 0-3 on 32x32 MFMA blocks, 4-8 on
@@ -287,8 +288,7 @@ int mt_gemm_config_count(int family);
 /* Forces tile configuration `cfg` of `family`, asked for `splits` K splits
  * (1..64; fewer when K is short), on every later GEMM launch of the calling
  * thread whose operands that family takes; the others keep the cost model.
- * (Direct-to-LDS configurations 4-6, the fragment-prefetching kernel with
- * 256x256, 64x64 and 128x128 tiles, take the convolution weight gradient's
+ * (Configurations 4-6 of MT_FAMILY_DL take the convolution weight gradient's
  * implicit operand and the fused row sums but not the forward convolution's
  * implicit im2col operand.)
  * A forced direct-to-LDS configuration also builds the im2col operand of a

@@ -36,8 +36,8 @@ GemmLaunchFn launcher_cfg2(int la, int lb);
 // The bf16-unit kernel gemm_f32_sp (gemm_sp_kernel.hpp): block tile BM x BN
 // (on blocks of BNB columns), wave tile WM x WN, WPE: waves per SIMD its
 // registers are sized for.  It makes configurations 0, 1, 3, 4, 6 and 7 below
-// (same index) and, for contiguous
-// operands of any alignment, the register-staged configurations (2: 64x64).
+// (same index)
+// and, for contiguous operands of any alignment, the register-staged ones (2: 64x64).
 template <int CFG> struct SpCfg;
 template <> struct SpCfg<0> { static constexpr int BM = 64, BN = 256, BNB = 256, WM = 64, WN = 64, WPE = 2; };
 template <> struct SpCfg<1> { static constexpr int BM = 128, BN = 128, BNB = 128, WM = 64, WN = 64, WPE = 2; };
@@ -50,9 +50,9 @@ constexpr bool is_sp_cfg(int cfg) {
     return cfg == 0 || cfg == 1 || cfg == 3 || cfg == 4 || cfg == 6 || cfg == 7;
 }
 
-// Its launcher for (layout of A: L_KV, L_MV, L_KVI; of B: L_KV, L_MV, L_IM, L_IMW,
-// L_IMR), with the row sums of A if rs (two L_KV or two L_MV); nullptr where the
-// configuration has no such form.
+// Its launcher for (layout of A: L_KV, L_MV, L_KVI; of B: L_KV, L_MV, L_IM, L_IM4,
+// L_IMW, L_IMR), with the row sums of A if rs (two L_KV, two L_MV, or B L_IMW);
+// nullptr where the configuration has no such form.
 GemmLaunchFn sp_launcher_cfg0(int la, int lb, bool rs);
 GemmLaunchFn sp_launcher_cfg1(int la, int lb, bool rs);
 GemmLaunchFn sp_launcher_cfg2(int la, int lb, bool rs);
@@ -90,7 +90,7 @@ template <> struct DlhCfg<1> { static constexpr int BM = 128, BN = 128, WM = 64,
 template <> struct DlhCfg<2> { static constexpr int BM = 64, BN = 64, WM = 32, WN = 32; };
 template <> struct DlhCfg<3> { static constexpr int BM = 256, BN = 128, WM = 64, WN = 64; };
 
-// 7: the channels-last convolution operand only (L_IM), tiles of 112 columns on
+// 7: the channels-last convolution operands only (L_IM, L_IM4), tiles of 112 columns on
 // blocks of 128 (4 waves of 32x64).  112 = 7*16 divides the pixel count of
 // ResNet layers (multiples of 7*7*16 at even batch sizes), so that such a layer
 // has no ragged tile: 28x28 with 128 channels at batch 32 is 448 tiles, two on

@@ -1,26 +1,16 @@
 // gemm_dlp_kernel.hpp -- direct-to-LDS fp32 MFMA GEMM whose waves read the
 // next K-chunk's fragments while the current chunk's MFMAs issue.
 //
-// Three tile shapes (direct-to-LDS configurations 4, 5 and 6):
-//   * 256x256 block tile, four waves of 128x128 (one wave per SIMD, 256
-//     accumulator registers).  Per 16-deep K-chunk a wave reads 16 KB of
-//     fragments from LDS for 128 MFMAs, against 12 KB for 64 MFMAs with the
-//     8-wave 128x64 split of gemm_f32_dl: two thirds of the LDS read traffic
-//     per flop.  The headline kernel.
-//   * 64x64 block tile, four waves of 32x32: the small GEMMs that run about
-//     one workgroup per CU, where each SIMD again holds a single wave and the
-//     fragment-read latency after every barrier is exposed.
-//   * 128x128 block tile, eight waves of 64x32 (two per SIMD), for K ranges
-//     of at least 512 per split (256 when every workgroup has a CU).
+// One tile shape is in use, direct-to-LDS configuration 5: a 64x64 block tile of
+// four waves of 32x32, for the small GEMMs that run about one workgroup per CU,
+// where each SIMD holds a single wave and the fragment-read latency after every
+// barrier is exposed.  (Larger tiles are gemm_f32_sp's.)
 // Structure:
 //   * With no second wave on the SIMD to cover the LDS latency, chunk kt+1's
 //     fragments are read while chunk kt's MFMAs issue: two register sets
 //     alternate (the loop is unrolled by two so that each set is a fixed set
-//     of registers).  The body has no branches, so the scheduler can spread
-//     the fragment reads and the next DMA over the MFMA stream (the
-//     sched_group_barrier patterns in dlp_interleave for the 256x256 tile
-//     and dlp_interleave_reads for the 128x128 one; the 64x64 tile's 8
-//     MFMAs per step do best left to the compiler).
+//     of registers).  The body has no branches, so the compiler can spread the
+//     fragment reads and the next DMA over the MFMA stream.
 //   * Ring of STAGES LDS slots, one s_barrier per chunk.  At the barrier of
 //     step kt, chunk kt+1 has landed (each wave waited for its own DMA) and
 //     every wave has retired its reads of chunk kt's slot, which the step then
@@ -42,42 +32,6 @@
 
 namespace mtk {
 
-// Spread the instructions that follow a step's barrier over its NM MFMAs:
-// the DMA of the refill (up to 8 wave instructions) first, one per MFMA, then
-// the fragment reads of the next chunk (up to 40 LDS instructions), one per
-// one or two MFMAs.  Groups without instructions of their kind stay empty.
-template <int NM>
-__device__ __forceinline__ void dlp_interleave() {
-    constexpr int kMfma = 0x008, kVmemRead = 0x020, kDsRead = 0x100;
-    __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
-#pragma unroll
-    for (int g = 0; g < 8; ++g) {
-        __builtin_amdgcn_sched_group_barrier(kVmemRead, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
-    }
-#pragma unroll
-    for (int g = 0; g < 40; ++g) {
-        __builtin_amdgcn_sched_group_barrier(kDsRead, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(kMfma, NM >= 100 ? 2 : 1, 0);
-    }
-    __builtin_amdgcn_sched_group_barrier(kMfma, NM, 0);
-}
-
-// The 64x32 wave tile (configuration 6): the refill's DMA first, then one
-// fragment read (up to 24 LDS instructions) per MFMA.  Left to itself the
-// scheduler packs the reads behind the MFMAs: 16 % slower with an
-// n-contiguous B (2048^2 x 1024), 2-4 % with the other layouts.
-template <int LOADS>
-__device__ __forceinline__ void dlp_interleave_reads() {
-    constexpr int kMfma = 0x008, kVmemRead = 0x020, kDsRead = 0x100;
-    __builtin_amdgcn_sched_group_barrier(kVmemRead, LOADS, 0);
-#pragma unroll
-    for (int g = 0; g < 24; ++g) {
-        __builtin_amdgcn_sched_group_barrier(kDsRead, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
-    }
-}
-
 // The MFMAs of k-steps S0..S1-1 of one chunk.
 template <int MB, int NB, int S0, int S1>
 __device__ __forceinline__ void mfma_steps(f32x16 (&acc)[MB][NB], const float (&fa)[MB][8],
@@ -91,8 +45,7 @@ __device__ __forceinline__ void mfma_steps(f32x16 (&acc)[MB][NB], const float (&
                 acc[i][j] = mfma_32x32x2(fa[i][s], fb[j][s], acc[i][j]);
 }
 
-// WPE: waves per SIMD the register allocation targets (1 lets the 128x128
-// wave tile keep its 256 accumulators in AGPRs beside 256 VGPRs).
+// WPE: waves per SIMD the register allocation targets.
 // RS: also produce the row sums of A (GemmParams::rowsum), as gemm_f32_dl's
 // row-sum form does: same waves, same order of additions.
 template <int BM, int BN, int WM, int WN, int LA, int LB, int STAGES, int WPE, bool TAIL,
@@ -187,17 +140,13 @@ gemm_f32_dlp(GemmParams p) {
     // into na/nb and refilling chunk kt's slot with chunk kt+STAGES.  The
     // barrier guards only the refill and the reads, so the first PRE k-steps
     // of MFMAs issue before it: the MFMA pipe has work queued while the waves
-    // synchronize (about 1 % at 4096^3, 3-9 % for the 64x64 tile).  Three
-    // k-steps for the 64x32 wave tile (8 waves of the 128x128 tile): about
-    // 1 % more at 2048^2 x 1024; equal or slower for the other two.
-    constexpr int PRE = (MB == 2 && NB == 1) ? 3 : 2;
+    // synchronize (3-9 % for the 64x64 tile).
+    constexpr int PRE = 2;
     auto step = [&](int kt, const float (&ca)[MB][8], const float (&cb)[NB][8],
                     float (&na)[MB][8], float (&nb)[NB][8]) {
-        if constexpr (PRE > 0) {
-            __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(63));   // ca/cb landed
-            mfma_steps<MB, NB, 0, PRE>(acc, ca, cb);
-            __builtin_amdgcn_sched_barrier(0);
-        }
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(63));   // ca/cb landed
+        mfma_steps<MB, NB, 0, PRE>(acc, ca, cb);
+        __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(LOADS * (STAGES - 2)));
         __builtin_amdgcn_s_barrier();
         float* const refill = smem + (kt % STAGES) * STAGE;
@@ -207,8 +156,6 @@ gemm_f32_dlp(GemmParams p) {
         dl_frags<LAF, BM, MB>(next, ra, lane, na);
         dl_frags<LBF, BN, NB>(next + TA::floats, rb, lane, nb);
         mfma_steps<MB, NB, PRE, 8>(acc, ca, cb);
-        if constexpr (MB * NB * 8 >= 128) dlp_interleave<(8 - PRE) * MB * NB>();
-        else if constexpr (MB == 2 && NB == 1) dlp_interleave_reads<LOADS>();
         add_rows(ca);
     };
 

@@ -147,9 +147,8 @@ struct CfgCost {
 // launch.  The constants are fitted (log-time error plus selection regret) to
 // the measured times of every configuration and split factor on 29 shapes --
 // the benchmark shapes, square, ragged, tall, wide, skinny, batched and
-// convolution GEMMs -- on one MI355X.  The efficiencies of the prefetching
-// configurations 4-6 come from same-box comparisons with configurations 0, 2
-// and 1, which have the same tiles.
+// convolution GEMMs -- on one MI355X; those of gemm_f32_sp, later, to 71
+// (kDlCost).
 constexpr CfgCost kRsCost[kNumCfg] = {      // register-staged kernel, any strides
     {TileCfg<0>::BM, TileCfg<0>::BN, 0.80, 1},
     {TileCfg<1>::BM, TileCfg<1>::BN, 0.75, 2},
@@ -332,7 +331,7 @@ double plan_cycles(const CostModel& cm, const CfgCost& cc, const Plan& pl, int64
 
 size_t scratch_rule_ws(int64_t M, int64_t N, int64_t K, int64_t batch, int cus);
 
-// wide: the prefetching direct-to-LDS configurations (is_dlp_cfg) may be
+// wide: configurations 4-6 (is_wide_cfg) may be
 // chosen (see wide_ok in launch_gemm); ksw: the wave-split kernel may be;
 // sp: gemm_f32_sp can take the operands (sp_fits, sp_layouts); imw: B is the
 // weight-gradient operand (priced by kDlCostImw); im16: the 112-column tile
@@ -446,9 +445,8 @@ thread_local ForcedConfig g_forced;
 
 // The plan of the forced configuration, when one is set and its family can
 // take these operands (dl_ok: both operands have direct-to-LDS layouts;
-// rs_ok: no implicit-im2col operand; wide_ok: the prefetching configurations
-// can take them too; im16_ok: B is L_IM, which the 16x16-block convolution
-// configurations take).
+// rs_ok: no implicit-im2col operand; wide_ok: configurations 4-6 can take them
+// too; im16_ok: B is L_IM, which configuration 7 takes).
 bool forced_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool dl_ok, bool rs_ok,
                  bool wide_ok, bool sp_ok, Plan* out, bool im16_ok = false) {
     const ForcedConfig f = g_forced;
@@ -1202,7 +1200,7 @@ int launch_gemm(GemmParams& p, bool dl, int la, int lb, void* workspace, size_t 
             skinny_plan(M, N, K, batch, la, lb, p.c_n_inner < N, device_cu_count());
         if (sp.kind != SK_NONE) return launch_skinny(p, sp, workspace, ws_bytes, stream);
     }
-    // The prefetching configurations' contract: vector layouts or the
+    // Configurations 4-6 take vector layouts or the
     // weight-gradient operand (not the implicit-im2col one), a non-empty K
     // range.
     const bool wide_ok = dl && lb != L_IM && lb != L_IMR && lb != L_IM4 && K > 0;
@@ -2472,7 +2470,7 @@ size_t implicit_gemm_ws(int64_t M, int64_t N, int64_t K, bool imw, bool im4 = fa
         const Plan pl = make_plan(M, N, K, 1, cus, true, true, imw, false, sp, imw);
         // (with the weight gradient's row sums: M floats per split)
         ws = std::max(ws, pl.ws_bytes + (imw && pl.splits > 1 ? (size_t)pl.splits * M * 4 : 0));
-        if (!imw && kOfferNarrow)   // the channels-last operand may take the 16x16-block kernel
+        if (!imw && kOfferNarrow)   // the channels-last operand may take configuration 7
             ws = std::max(ws,
                           make_plan(M, N, K, 1, cus, true, true, false, false, sp, false, true).ws_bytes);
     }
