@@ -157,6 +157,9 @@ template <int CFG> struct KswTile {
 
 // Configuration cfg of the wave-split kernel; va / vb: A / B is L_KV.
 GemmLaunchFn ksw_launcher(int cfg, bool va, bool vb);
+// ... with the row sums of A (GemmParams::rowsum): scalar loads of both operands,
+// no split; nullptr for the 32x32-block configurations 0-3.
+GemmLaunchFn ksw_rowsum_launcher(int cfg);
 void ksw_tile(int cfg, int* bm, int* bn);
 
 // Vector-ALU kernels of the HBM-bound shapes (gemm_skinny_kernel.hpp):

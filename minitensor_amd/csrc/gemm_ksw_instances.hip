@@ -1,6 +1,7 @@
 // gemm_ksw_instances.hip -- instantiates the wave-split kernels
-// (gemm_f32_ksw, gemm_f32_ksw16) for their tile configurations and the 2x2 choices of 16-byte or scalar
-// fragment loads for A and B.
+// (gemm_f32_ksw, gemm_f32_ksw16) for their tile configurations and the 2x2
+// choices of 16-byte or scalar fragment loads for A and B, and the 16x16-block
+// ones with the row sums of A for scalar loads of both.
 #include "gemm_configs.hpp"
 #include "gemm_ksw_kernel.hpp"
 
@@ -19,6 +20,15 @@ hipError_t launch_ksw(const GemmParams& p, unsigned nblocks, hipStream_t s) {
     return hipGetLastError();
 }
 
+template <int CFG>
+hipError_t launch_ksw_rows(const GemmParams& p, unsigned nblocks, hipStream_t s) {
+    using C = KswCfg<CFG>;
+    static_assert(C::R == 16, "row sums: 16x16 blocks");
+    hipLaunchKernelGGL((gemm_f32_ksw16<C::MB, C::NB, C::W, false, false, C::D, true>),
+                       dim3(nblocks), dim3(C::W * 64), 0, s, p);
+    return hipGetLastError();
+}
+
 #define MT_KSW_TABLE(CFG) \
     { { launch_ksw<CFG, false, false>, launch_ksw<CFG, false, true> }, \
       { launch_ksw<CFG, true, false>, launch_ksw<CFG, true, true> } }
@@ -30,6 +40,13 @@ GemmLaunchFn ksw_launcher(int cfg, bool va, bool vb) {
         MT_KSW_TABLE(0), MT_KSW_TABLE(1), MT_KSW_TABLE(2), MT_KSW_TABLE(3),
         MT_KSW_TABLE(4), MT_KSW_TABLE(5), MT_KSW_TABLE(6), MT_KSW_TABLE(7), MT_KSW_TABLE(8)};
     return table[cfg][va][vb];
+}
+
+GemmLaunchFn ksw_rowsum_launcher(int cfg) {
+    static const GemmLaunchFn table[kNumKswCfg] = {
+        nullptr, nullptr, nullptr, nullptr, launch_ksw_rows<4>, launch_ksw_rows<5>,
+        launch_ksw_rows<6>, launch_ksw_rows<7>, launch_ksw_rows<8>};
+    return table[cfg];
 }
 
 void ksw_tile(int cfg, int* bm, int* bn) {

@@ -1186,12 +1186,13 @@ int launch_gemm(GemmParams& p, bool dl, int la, int lb, void* workspace, size_t 
               (p.c_n_inner >= N || ((p.c_n_inner & 3) == 0 && (p.c_n_outer & 3) == 0 &&
                                     (p.c_n_inner2 <= 0 ||
                                      ((p.c_n_inner2 & 3) == 0 && (p.c_n_outer2 & 3) == 0))));
-    // Row sums of A are fused only into a direct-to-LDS launch of two
+    // Row sums of A are fused only into a direct-to-LDS (or, below, wave-split) launch of two
     // mn-contiguous operands without split-K (the caller sees p.rowsum cleared
     // and computes them separately).
     // A batch-summed product of two k-contiguous operands fuses them too, as
     // partials per (split, batch entry) that its reduction sums for csum.
     const bool rs_part = p.part && la == L_KV && lb == L_KV && p.csum != nullptr;
+    float* const rows_out = p.rowsum;
     if (!rs_part && lb != L_IMW && (batch != 1 || la != L_MV || lb != L_MV || p.part))
         p.rowsum = nullptr;
     // The HBM-bound shapes (few rows or columns, or K <= 16) on the vector ALUs.
@@ -1240,6 +1241,12 @@ int launch_gemm(GemmParams& p, bool dl, int la, int lb, void* workspace, size_t 
     if (lb == L_IMW && !rs_imw) p.rowsum = nullptr;
     if (!plan.dl || (plan.splits > 1 && !rs_part && !rs_imw) || plan.cfg == kNarrowCfg)
         p.rowsum = nullptr;
+    // ... and into the wave-split kernel on 16x16 blocks, where neither operand
+    // takes 16-byte loads (dYᵀ never does, an X of odd width does not).
+    const bool rs_ksw = rows_out != nullptr && plan.ksw && plan.splits == 1 && batch == 1 &&
+                        !p.part && !implicit && la != L_KV && lb != L_KV &&
+                        ksw_rowsum_launcher(plan.cfg) != nullptr;
+    if (rs_ksw) p.rowsum = rows_out;
     p.splits = plan.splits;
     p.k_per_split = plan.splits > 1 ? plan.kps : (int)std::max<int64_t>(K, 1);
     p.tiles_m = plan.tiles_m;
@@ -1277,6 +1284,7 @@ int launch_gemm(GemmParams& p, bool dl, int la, int lb, void* workspace, size_t 
 
     GemmLaunchFn fn = halo ? dlh_launcher(plan.cfg)
                       : lb == L_IM || lb == L_IMR || lb == L_IM4 ? conv_launcher(plan.cfg, lb)
+                      : rs_ksw                             ? ksw_rowsum_launcher(plan.cfg)
                       : lb == L_IMW && p.rowsum != nullptr ? sp_launcher(plan.cfg, la, lb, true)
                       : lb == L_IMW ? convw_launcher(plan.cfg, (K & 15) != 0, la == L_KVI)
                       : p.rowsum != nullptr ? rowsum_launcher(plan.cfg, (K & 15) != 0, la == L_KV)
