@@ -261,7 +261,12 @@ constexpr int kDlSmallCfg = 2;           // the 64x64 direct-to-LDS configuratio
 constexpr double kCoresidentPair = 0.75;
 constexpr int kAloneMinK = 1024;
 constexpr double kAlonePenalty = 1.3;
+// A gemm_f32_sp workgroup alone on its CU: 1.13 with the gathered operands and
+// over short K ranges, where the first loads weigh most; over 512 and more of a
+// matrix operand its MFMAs hide them (2048 x 2048 x 1024 on 128x128 tiles, one
+// per CU: 47.8 us, priced at 57 with the factor; two splits of 256x128 took 59).
 constexpr double kSpAlone = 1.13;
+constexpr int kSpAloneMinK = 512;
 constexpr int kMaxForcedSplits = 64;
 constexpr bool kOfferNarrow = true;
 
@@ -365,6 +370,8 @@ Plan make_plan_uncached(int64_t M, int64_t N, int64_t K, int64_t batch, int cus,
             if (pl.splits != s) continue;
             const int64_t wgs = (int64_t)pl.tiles_m * pl.tiles_n * batch * pl.splits;
             if (wgs * 512 >= ((int64_t)1 << 32)) continue;
+            if (dl && wide && !imw && cc.sp && cc.occ > 1)
+                cc.alone = pl.kps >= kSpAloneMinK ? 1.0 : kSpAlone;
             // The 64x112 tile of 16x16 blocks moves about twice the operand
             // bytes per flop of the 256x128 one; with one workgroup per CU
             // (nothing co-resident to hide the fetches) it lost everywhere it
