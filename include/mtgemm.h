@@ -93,8 +93,9 @@ size_t mt_gemm_workspace_f32(const mt_mat_f32* A, const mt_mat_f32* B, const mt_
  *   - Same plan and the same results, bit for bit, as mt_gemm_f32 with a
  *     workspace of mt_gemm_workspace_f32 bytes.
  *   - A problem that needs more scratch returns MT_ERR_SCRATCH_LIMIT and
- *     launches nothing: by a fixed rule on its sizes, under which every problem
- *     that is taken has a mt_gemm_workspace_f32 within the limit.
+ *     launches nothing: by a rule on its sizes that has prices of its own and
+ *     does not move with the kernels', and under which every problem that is
+ *     taken has a mt_gemm_workspace_f32 within the limit.
  *   - Allocates nothing and calls no allocating routine; the first call on
  *     each GPU looks up that GPU's copy of the buffer (hipGetSymbolAddress).
  *   - Every call on a GPU uses that GPU's one buffer: calls that may overlap

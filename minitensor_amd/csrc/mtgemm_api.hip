@@ -24,6 +24,7 @@
 
 #include "gemm_configs.hpp"
 #include "mtgemm.h"
+#include "noalloc_rule.hpp"
 
 using namespace mtk;
 
@@ -334,8 +335,6 @@ double plan_cycles(const CostModel& cm, const CfgCost& cc, const Plan& pl, int64
     return t;
 }
 
-size_t scratch_rule_ws(int64_t M, int64_t N, int64_t K, int64_t batch, int cus);
-
 // wide: configurations 4-6 (is_wide_cfg) may be
 // chosen (see wide_ok in launch_gemm); ksw: the wave-split kernel may be;
 // sp: gemm_f32_sp can take the operands (sp_fits, sp_layouts); imw: B is the
@@ -379,7 +378,8 @@ Plan make_plan_uncached(int64_t M, int64_t N, int64_t K, int64_t batch, int cus,
             if (dl && cfg == kNarrowCfg && wgs <= cus) continue;
             if (product && pl.ws_bytes > (size_t)MT_NOALLOC_SCRATCH_BYTES) {
                 if (!ruled)
-                    small_ws = scratch_rule_ws(M, N, K, batch, cus) <= MT_NOALLOC_SCRATCH_BYTES;
+                    small_ws =
+                        noalloc_rule::takes(M, N, K, batch, cus, MT_NOALLOC_SCRATCH_BYTES);
                 ruled = true;
                 if (small_ws) continue;
             }
@@ -716,50 +716,6 @@ size_t plan_ws_uncached(int64_t M, int64_t N, int64_t K, int64_t batch, int cus)
     return std::max(ws, skinny_ws(M, N, K, batch, cus));
 }
 
-// Which calls mt_gemm_noalloc_f32 takes: those whose sizes need at most its
-// scratch under this price table, the one of the fp32 matrix units' tiles.  It
-// is a rule of that entry point and no plan: it stays as it is when the kernels
-// and their prices change, so that a call that was taken is taken still and one
-// that was refused is refused.  (thresholds of K: the 128x128 tile of 8 waves)
-constexpr CfgCost kScratchRs[3] = {{256, 256, 0.86, 1}, {128, 128, 0.75, 2}, {64, 64, 0.57, 4}};
-constexpr CfgCost kScratchDl[7] = {{256, 256, 0.90, 1}, {128, 128, 0.86, 4}, {64, 64, 0.68, 8},
-                                   {256, 128, 0.87, 3}, {256, 256, 0.98, 1}, {64, 64, 0.72, 8},
-                                   {128, 128, 0.90, 3}};
-constexpr int kScratchMinK = 512, kScratchMinKOneRound = 256;
-
-size_t scratch_rule_ws(int64_t M, int64_t N, int64_t K, int64_t batch, int cus) {
-    static const CostModel cm;
-    const int64_t most = std::min<int64_t>(kMaxSplits, std::max<int64_t>(K / 48, 1));
-    if ((double)M * N * batch * 4 * most <= (double)MT_NOALLOC_SCRATCH_BYTES)
-        return skinny_ws(M, N, K, batch, cus);   // whatever the plan
-    size_t ws = 0;
-    for (int form = 0; form < 3; ++form) {   // register-staged, direct-to-LDS, prefetching too
-        const bool dl = form > 0;
-        const CfgCost* cfgs = dl ? kScratchDl : kScratchRs;
-        double best_t = 1e300;
-        size_t best_ws = 0;
-        for (int cfg = 0; cfg < (form == 0 ? 3 : form == 1 ? 4 : 7); ++cfg)
-            for (int s = 1; s <= kMaxSplits; ++s) {
-                const Plan pl = cfg_plan(cfgs[cfg], cfg, dl, M, N, K, batch, s);
-                if (s > 1 && pl.kps < 64) break;
-                if (s > kFittedSplits && pl.kps < kMinKpsBeyondFit) break;
-                const int64_t k6 = std::min<int64_t>(pl.kps, K);
-                if (dl && cfg == 6 && k6 < kScratchMinKOneRound) break;
-                if (pl.splits != s) continue;
-                const int64_t wgs = (int64_t)pl.tiles_m * pl.tiles_n * batch * pl.splits;
-                if (dl && cfg == 6 && k6 < kScratchMinK && wgs > cus) continue;
-                if (wgs * 512 >= ((int64_t)1 << 32)) continue;
-                const double t = plan_cycles(cm, cfgs[cfg], pl, M, N, batch, cus);
-                if (t < best_t) {
-                    best_t = t;
-                    best_ws = pl.ws_bytes;
-                }
-            }
-        ws = std::max(ws, best_ws);
-    }
-    return std::max(ws, skinny_ws(M, N, K, batch, cus));
-}
-
 size_t plan_ws(int64_t M, int64_t N, int64_t K, int64_t batch, int cus) {
     if (g_forced.family != MT_FAMILY_AUTO) {
         Plan forced;
@@ -779,19 +735,20 @@ size_t plan_ws(int64_t M, int64_t N, int64_t K, int64_t batch, int cus) {
     return e.ws;
 }
 
-// scratch_rule_ws, the last answers kept: a decode loop asks for the same sizes.
-size_t noalloc_rule_ws(int64_t M, int64_t N, int64_t K, int64_t batch, int cus) {
+// noalloc_rule::takes, the last answers kept: a decode loop asks for the same sizes.
+bool noalloc_takes(int64_t M, int64_t N, int64_t K, int64_t batch, int cus) {
     struct Entry {
         int64_t M = -1, N = -1, K = -1, batch = -1;
         int cus = 0;
-        size_t ws = 0;
+        bool taken = false;
     };
     constexpr int kBits = 7;
     thread_local Entry cache[1 << kBits];
     Entry& e = cache[hash_slot(kBits, M, N, K, batch)];
     if (e.M != M || e.N != N || e.K != K || e.batch != batch || e.cus != cus)
-        e = Entry{M, N, K, batch, cus, scratch_rule_ws(M, N, K, batch, cus)};
-    return e.ws;
+        e = Entry{M, N, K, batch, cus,
+                  noalloc_rule::takes(M, N, K, batch, cus, MT_NOALLOC_SCRATCH_BYTES)};
+    return e.taken;
 }
 
 // Contiguous layout of one operand for gemm_f32_sp, whatever its alignment, or
@@ -2668,7 +2625,7 @@ int mt_gemm_noalloc_f32(const mt_mat_f32* A, const mt_mat_f32* B, const mt_mat_f
     if (g_forced.family != MT_FAMILY_AUTO && need > MT_NOALLOC_SCRATCH_BYTES)
         return MT_ERR_SCRATCH_LIMIT;
     if (M > 0 && N > 0 && batch > 0 &&
-        noalloc_rule_ws(M, N, K, batch, device_cu_count()) > MT_NOALLOC_SCRATCH_BYTES)
+        !noalloc_takes(M, N, K, batch, device_cu_count()))
         return MT_ERR_SCRATCH_LIMIT;
     void* ws = nullptr;
     if (need > 0) {
