@@ -269,7 +269,6 @@ constexpr double kAlonePenalty = 1.3;
 constexpr double kSpAlone = 1.13;
 constexpr int kSpAloneMinK = 512;
 constexpr int kMaxForcedSplits = 64;
-constexpr bool kOfferNarrow = true;
 
 // Tile grid and K split of configuration `cfg` asked for `s` splits (the
 // split count can come out lower: every split takes whole 16-deep chunks).
@@ -294,6 +293,11 @@ Plan cfg_plan(const CfgCost& cc, int cfg, bool dl, int64_t M, int64_t N, int64_t
 // fused bias gradient's partials).
 size_t part_ws_bytes(const Plan& pl, int64_t M, int64_t N, int64_t batch) {
     return (size_t)std::max(pl.splits, 1) * batch * M * (N + 1) * sizeof(float);
+}
+
+// ... of a split's partials and their sum.
+double split_cycles(const CostModel& cm, int splits, int64_t M, int64_t N, int64_t batch) {
+    return (double)(2 * splits + 1) * M * N * batch * 4.0 / cm.bytes_per_cycle + cm.launch_cycles;
 }
 
 // Modelled cycles of one plan (see CostModel).
@@ -328,27 +332,23 @@ double plan_cycles(const CostModel& cm, const CfgCost& cc, const Plan& pl, int64
                                                              : 1.0;
     double t = per_cu * work * pair * alone + per_cu * epi / cc.occ +
                rounds * (cc.sp ? cm.sp_round_latency : cm.round_latency);
-    if (pl.splits > 1) {
-        const double bytes = (double)(2 * pl.splits + 1) * M * N * batch * 4.0;
-        t += bytes / (cm.bytes_per_cycle) + cm.launch_cycles;
-    }
+    if (pl.splits > 1) t += split_cycles(cm, pl.splits, M, N, batch);
     return t;
 }
 
-// wide: configurations 4-6 (is_wide_cfg) may be
-// chosen (see wide_ok in launch_gemm); ksw: the wave-split kernel may be;
-// sp: gemm_f32_sp can take the operands (sp_fits, sp_layouts); imw: B is the
+// wide: configurations 4-6 (is_wide_cfg) may be chosen (see wide_ok in
+// launch_gemm); sp: gemm_f32_sp can take the operands (sp_fits, sp_layouts); imw: B is the
 // weight-gradient operand (priced by kDlCostImw); im16: the 112-column tile
 // (kNarrowCfg, B = L_IM) may be; im4: B is L_IM4 (configurations 1, 3 and 7).
 Plan make_plan_uncached(int64_t M, int64_t N, int64_t K, int64_t batch, int cus,
-                        bool allow_split, bool dl, bool wide, bool ksw, bool sp, bool imw, bool im16,
+                        bool allow_split, bool dl, bool wide, bool sp, bool imw, bool im16,
                         bool im4) {
     static const CostModel cm;
     const CfgCost* cfgs = dl ? (imw ? kDlCostImw : kDlCost) : sp ? kRsSpCost : kRsCost;
     const int ncfg = dl ? kNumDlCfg : kNumCfg;
     Plan best;
     best.dl = dl;
-    double best_t = 1e300;
+    double best_t = best.cycles = 1e300;
     // A matrix product that mt_gemm_noalloc_f32 takes keeps its partials within
     // that entry point's scratch, so that both run the same plan.
     const bool product = !imw && (wide || !dl);
@@ -363,6 +363,8 @@ Plan make_plan_uncached(int64_t M, int64_t N, int64_t K, int64_t batch, int cus,
         if (dl && cfg == 0 && !wide && !im16 && !im4) cc.eff = kImrNarrowEff;   // L_IMR
         for (int s = 1; s <= (imw ? kMaxImwSplits : kMaxSplits); ++s) {
             if (s > 1 && !allow_split) break;
+            // this and every further split's partials cost more than the best plan
+            if (s > 1 && split_cycles(cm, s, M, N, batch) > best_t) break;
             const Plan pl = cfg_plan(cc, cfg, dl, M, N, K, batch, s);
             if (s > 1 && pl.kps < 64) break;
             if (s > kFittedSplits && pl.kps < kMinKpsBeyondFit) break;
@@ -391,20 +393,20 @@ Plan make_plan_uncached(int64_t M, int64_t N, int64_t K, int64_t batch, int cus,
             }
         }
     }
-    if (ksw) {
-        for (int cfg = 0; cfg < kNumKswCfg; ++cfg) {
-            if (K < (int64_t)kBK * kKswWaves[cfg]) continue;
-            Plan pl = cfg_plan(kKswCost[cfg], cfg, false, M, N, K, batch, 1);
-            pl.ksw = true;
-            const int64_t wgs = (int64_t)pl.tiles_m * pl.tiles_n * batch;
-            if (wgs * 512 >= ((int64_t)1 << 32)) continue;
-            const double t = plan_cycles(cm, kKswCost[cfg], pl, M, N, batch, cus);
-            if (t < best_t) {
-                best_t = t;
-                best = pl;
-                best.cycles = t;
-            }
-        }
+    return best;
+}
+
+// `best`, or the wave-split plan (one split, no workspace) where that is cheaper.
+Plan or_wave_split(Plan best, int64_t M, int64_t N, int64_t K, int64_t batch, int cus) {
+    static const CostModel cm;
+    for (int cfg = 0; cfg < kNumKswCfg; ++cfg) {
+        if (K < (int64_t)kBK * kKswWaves[cfg]) continue;
+        Plan pl = cfg_plan(kKswCost[cfg], cfg, false, M, N, K, batch, 1);
+        pl.ksw = true;
+        const int64_t wgs = (int64_t)pl.tiles_m * pl.tiles_n * batch;
+        if (wgs * 512 >= ((int64_t)1 << 32)) continue;
+        pl.cycles = plan_cycles(cm, kKswCost[cfg], pl, M, N, batch, cus);
+        if (pl.cycles < best.cycles) best = pl;
     }
     return best;
 }
@@ -417,29 +419,62 @@ size_t hash_slot(int bits, T... words) {
     return (size_t)(h >> (64 - bits));
 }
 
+// What a thread asked for last, by sizes and flags: 2^kBits sets of four entries,
+// the oldest of a set gives way.  (One entry a slot had shapes that share one
+// evict each other at every step: 100 distinct shapes a step took 24.7 us per
+// query and launch where 8 took 5.8.)
+template <class V, int kBits>
+class Recent {
+    struct Entry {
+        int64_t M, N, K, batch;
+        int cus, flags;
+        bool used;
+        V value;
+    };
+    Entry entry_[1 << kBits][4] = {};
+    uint8_t next_[1 << kBits] = {};
+
+   public:
+    // make() may ask this table for other keys.
+    template <class F>
+    V get(int64_t M, int64_t N, int64_t K, int64_t batch, int cus, int flags, F make) {
+        const size_t set = hash_slot(kBits, M, N, K, batch, flags);
+        for (const Entry& e : entry_[set])
+            if (e.used && e.M == M && e.N == N && e.K == K && e.batch == batch && e.cus == cus &&
+                e.flags == flags)
+                return e.value;
+        const V v = make();
+        entry_[set][next_[set]++ & 3] = Entry{M, N, K, batch, cus, flags, true, v};
+        return v;
+    }
+};
+
 // The cost model is a pure function of its arguments; a training loop asks
-// for the same few shapes again and again (workspace query, then launch), so
-// each thread keeps plans, one per slot of a table indexed by a hash of the
-// key.  A workspace query of one GEMM visits 12 keys, one convolution backward
-// query four such shapes: the table holds several layers' worth.
+// for the same shapes again and again (workspace query, then launch), so each
+// thread keeps plans.
 Plan make_plan(int64_t M, int64_t N, int64_t K, int64_t batch, int cus, bool allow_split,
                bool dl, bool wide, bool ksw, bool sp, bool imw = false, bool im16 = false,
                bool im4 = false) {
-    struct Entry {
-        int64_t M = -1, N = -1, K = -1, batch = -1;
-        int cus = 0, flags = 0;
-        Plan plan;
-    };
-    constexpr int kBits = 9;
-    thread_local Entry cache[1 << kBits];
+    thread_local Recent<Plan, 8> plans;
     const int flags = allow_split | dl << 1 | wide << 2 | ksw << 3 | sp << 4 | imw << 5 | im16 << 6 |
                       im4 << 7;
-    Entry& e = cache[hash_slot(kBits, M, N, K, batch, flags)];
-    if (e.M != M || e.N != N || e.K != K || e.batch != batch || e.cus != cus || e.flags != flags)
-        e = Entry{M, N, K, batch, cus, flags,
-                  make_plan_uncached(M, N, K, batch, cus, allow_split, dl, wide, ksw, sp, imw,
-                                     im16, im4)};
-    return e.plan;
+    return plans.get(M, N, K, batch, cus, flags, [&] {
+        if (ksw)
+            return or_wave_split(make_plan(M, N, K, batch, cus, allow_split, dl, wide, false, sp,
+                                           imw, im16, im4),
+                                 M, N, K, batch, cus);
+        return make_plan_uncached(M, N, K, batch, cus, allow_split, dl, wide, sp, imw, im16, im4);
+    });
+}
+
+// Workspace queries that visit several plans keep their answers too (no forced
+// configuration).  A plan without the wave-split kernel, which takes no
+// workspace, needs what any plan of the same operands does.
+enum WsKind { WS_PLAN, WS_PART, WS_IMPLICIT, WS_IMPLICIT_IM4, WS_IMW };
+template <class F>
+size_t recent_ws(WsKind kind, int64_t M, int64_t N, int64_t K, int64_t batch, int cus, F make) {
+    thread_local Recent<size_t, 7> sizes;
+    return sizes.get(M, N, K, batch, cus, kind, make);
 }
 
 // Configuration forced on this thread's launches by mt_gemm_force_config.
@@ -706,49 +741,27 @@ size_t skinny_ws(int64_t M, int64_t N, int64_t K, int64_t batch, int cus) {
 
 // Workspace that covers the plan of either kernel family (for sizes queried
 // before the operand pointers, and hence the layouts, are known).
-size_t plan_ws_uncached(int64_t M, int64_t N, int64_t K, int64_t batch, int cus) {
-    size_t ws = 0;
-    for (bool dl : {false, true})
-        for (bool ksw : {false, true})
+size_t plan_ws(int64_t M, int64_t N, int64_t K, int64_t batch, int cus) {
+    const auto plans = [&] {
+        size_t ws = 0;
+        for (bool dl : {false, true})
             for (bool sp : {false, true})
                 ws = std::max(ws,
-                              make_plan(M, N, K, batch, cus, true, dl, dl, ksw, sp).ws_bytes);
-    return std::max(ws, skinny_ws(M, N, K, batch, cus));
-}
-
-size_t plan_ws(int64_t M, int64_t N, int64_t K, int64_t batch, int cus) {
-    if (g_forced.family != MT_FAMILY_AUTO) {
-        Plan forced;
-        const bool f = forced_plan(M, N, K, batch, true, true, true, true, &forced);
-        return std::max(f ? forced.ws_bytes : 0, plan_ws_uncached(M, N, K, batch, cus));
-    }
-    struct Entry {
-        int64_t M = -1, N = -1, K = -1, batch = -1;
-        int cus = 0;
-        size_t ws = 0;
+                              make_plan(M, N, K, batch, cus, true, dl, dl, false, sp).ws_bytes);
+        return std::max(ws, skinny_ws(M, N, K, batch, cus));
     };
-    constexpr int kBits = 7;
-    thread_local Entry cache[1 << kBits];
-    Entry& e = cache[hash_slot(kBits, M, N, K, batch)];
-    if (e.M != M || e.N != N || e.K != K || e.batch != batch || e.cus != cus)
-        e = Entry{M, N, K, batch, cus, plan_ws_uncached(M, N, K, batch, cus)};
-    return e.ws;
+    if (g_forced.family == MT_FAMILY_AUTO) return recent_ws(WS_PLAN, M, N, K, batch, cus, plans);
+    Plan forced;
+    const bool f = forced_plan(M, N, K, batch, true, true, true, true, &forced);
+    return std::max(f ? forced.ws_bytes : 0, plans());
 }
 
 // noalloc_rule::takes, the last answers kept: a decode loop asks for the same sizes.
 bool noalloc_takes(int64_t M, int64_t N, int64_t K, int64_t batch, int cus) {
-    struct Entry {
-        int64_t M = -1, N = -1, K = -1, batch = -1;
-        int cus = 0;
-        bool taken = false;
-    };
-    constexpr int kBits = 7;
-    thread_local Entry cache[1 << kBits];
-    Entry& e = cache[hash_slot(kBits, M, N, K, batch)];
-    if (e.M != M || e.N != N || e.K != K || e.batch != batch || e.cus != cus)
-        e = Entry{M, N, K, batch, cus,
-                  noalloc_rule::takes(M, N, K, batch, cus, MT_NOALLOC_SCRATCH_BYTES)};
-    return e.taken;
+    thread_local Recent<bool, 5> taken;
+    return taken.get(M, N, K, batch, cus, 0, [&] {
+        return noalloc_rule::takes(M, N, K, batch, cus, MT_NOALLOC_SCRATCH_BYTES);
+    });
 }
 
 // Contiguous layout of one operand for gemm_f32_sp, whatever its alignment, or
@@ -1189,10 +1202,10 @@ int launch_gemm(GemmParams& p, bool dl, int la, int lb, void* workspace, size_t 
         // convolution operands and the fused row sums
         const bool ksw_ok = !implicit && p.rowsum == nullptr;
         plan = make_plan(M, N, K, batch, device_cu_count(), true, dl, wide_ok, ksw_ok, sp_ok,
-                         lb == L_IMW, im16_ok && kOfferNarrow, lb == L_IM4);
+                         lb == L_IMW, im16_ok, lb == L_IM4);
         if (need(plan) > 0 && (workspace == nullptr || ws_bytes < need(plan)))
             plan = make_plan(M, N, K, batch, device_cu_count(), false, dl, wide_ok, ksw_ok, sp_ok,
-                             lb == L_IMW, im16_ok && kOfferNarrow, lb == L_IM4);
+                             lb == L_IMW, im16_ok, lb == L_IM4);
         if (need(plan) > 0 && (workspace == nullptr || ws_bytes < need(plan)))
             return MT_ERR_WORKSPACE;
     }
@@ -2083,14 +2096,16 @@ bool pointwise(const mt_conv2d_desc* d) {
 // Workspace of a batch-summed product (GemmParams::part) under any plan the
 // launcher can take for it.
 size_t part_plan_ws(int64_t M, int64_t N, int64_t K, int64_t batch, int cus) {
-    size_t ws = 0;
-    for (bool dl : {false, true})
-        for (bool wide : {false, true})
-            for (bool ksw : {false, true})
+    size_t ws = recent_ws(WS_PART, M, N, K, batch, cus, [&] {
+        size_t w = 0;
+        for (bool dl : {false, true})
+            for (bool wide : {false, true})
                 for (bool sp : {false, true})
-                    ws = std::max(
-                        ws, part_ws_bytes(make_plan(M, N, K, batch, cus, true, dl, wide, ksw, sp),
-                                          M, N, batch));
+                    w = std::max(
+                        w, part_ws_bytes(make_plan(M, N, K, batch, cus, true, dl, wide, false, sp),
+                                         M, N, batch));
+        return w;
+    });
     Plan forced;
     if (forced_plan(M, N, K, batch, true, true, true, true, &forced))
         ws = std::max(ws, part_ws_bytes(forced, M, N, batch));
@@ -2437,18 +2452,22 @@ bool dx_prefer_phased(const mt_conv2d_desc* d, int64_t Ho, int64_t Wo, bool cl) 
 size_t implicit_gemm_ws(int64_t M, int64_t N, int64_t K, bool imw, bool im4 = false) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     const int cus = device_cu_count();
-    size_t ws = 0;
-    for (bool sp : {false, true}) {
-        const Plan pl = make_plan(M, N, K, 1, cus, true, true, imw, false, sp, imw);
-        // (with the weight gradient's row sums: M floats per split)
-        ws = std::max(ws, pl.ws_bytes + (imw && pl.splits > 1 ? (size_t)pl.splits * M * 4 : 0));
-        if (!imw && kOfferNarrow)   // the channels-last operand may take configuration 7
-            ws = std::max(ws,
-                          make_plan(M, N, K, 1, cus, true, true, false, false, sp, false, true).ws_bytes);
-    }
-    if (im4)
-        ws = std::max(ws, make_plan(M, N, K, 1, cus, true, true, false, false, true, false, false,
-                                    true).ws_bytes);
+    const WsKind kind = imw ? WS_IMW : im4 ? WS_IMPLICIT_IM4 : WS_IMPLICIT;
+    size_t ws = recent_ws(kind, M, N, K, 1, cus, [&] {
+        size_t w = 0;
+        for (bool sp : {false, true}) {
+            const Plan pl = make_plan(M, N, K, 1, cus, true, true, imw, false, sp, imw);
+            // (with the weight gradient's row sums: M floats per split)
+            w = std::max(w, pl.ws_bytes + (imw && pl.splits > 1 ? (size_t)pl.splits * M * 4 : 0));
+            if (!imw)   // the channels-last operand may take configuration 7
+                w = std::max(w, make_plan(M, N, K, 1, cus, true, true, false, false, sp, false,
+                                          true).ws_bytes);
+        }
+        if (im4)
+            w = std::max(w, make_plan(M, N, K, 1, cus, true, true, false, false, true, false,
+                                      false, true).ws_bytes);
+        return w;
+    });
     Plan f;
     if (forced_plan(M, N, K, 1, true, false, imw, true, &f, !imw)) ws = std::max(ws, f.ws_bytes);
     return ws;

@@ -39,7 +39,12 @@ inline Split split_of(const Tile& t, int64_t M, int64_t N, int64_t K, int64_t ba
             splits > 1 ? (size_t)splits * batch * M * N * sizeof(float) : 0};
 }
 
-// Modelled cycles; `small`: a direct-to-LDS tile of 64 x 64, `prefetching`: the
+// Modelled cycles of the partials and their sum.
+inline double split_cycles(int64_t splits, int64_t M, int64_t N, int64_t batch) {
+    return (double)(2 * splits + 1) * M * N * batch * 4.0 / 6400.0 + 17700.0;
+}
+
+// ... of the whole; `small`: a direct-to-LDS tile of 64 x 64, `prefetching`: the
 // one of the two with fragment prefetch.
 inline double cycles(const Tile& t, const Split& p, bool small, bool prefetching, int64_t M,
                      int64_t N, int64_t batch, int cus) {
@@ -51,7 +56,7 @@ inline double cycles(const Tile& t, const Split& p, bool small, bool prefetching
     const double pair = prefetching && p.tiles_m == 1 && per_cu == 2 ? 0.75 : 1.0;
     const double alone = per_cu <= 1 && small && p.kps >= 1024 ? 1.3 : 1.0;
     double c = per_cu * work * pair * alone + per_cu * epilogue / t.occ + rounds * 6200.0;
-    if (p.splits > 1) c += (double)(2 * p.splits + 1) * M * N * batch * 4.0 / 6400.0 + 17700.0;
+    if (p.splits > 1) c += split_cycles(p.splits, M, N, batch);
     return c;
 }
 
@@ -87,6 +92,7 @@ inline bool takes(int64_t M, int64_t N, int64_t K, int64_t batch, int cus, size_
         for (int i = 0; i < (form == 0 ? 3 : form == 1 ? 4 : 7); ++i) {
             const Tile& t = direct ? kDirect[i] : kStaged[i];
             for (int64_t s = 1; s <= 256; ++s) {
+                if (s > 1 && split_cycles(s, M, N, batch) > best) break;   // nor any further split
                 const Split p = split_of(t, M, N, K, batch, s);
                 if (s > 1 && p.kps < 64) break;
                 if (s > 16 && p.kps < 256) break;
