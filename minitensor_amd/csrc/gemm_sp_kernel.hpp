@@ -574,8 +574,15 @@ gemm_f32_sp(GemmParams p) {
 
     f32x16 acc[MB][NB];
     // Row sums: every thread adds up the items of A that it loads; those of a
-    // row meet after the loop, in a fixed order.
-    float rsum[IA::NI];
+    // row meet after the loop, in a fixed order.  Those of a weight gradient's dY
+    // would be one chain per thread, where a launch of their own
+    // (block_channel_sum) has eight: every four chunks the sum goes to rtot, and
+    // what that addition rounds off to rlow (Knuth's two-sum).  Error against 64
+    // bits of 32 x 12544 normal values in 512 splits: 1.58e-7 plain, 1.17e-7 so,
+    // 1.26e-7 the launch of their own; 32 x 196 in 8: 1.55e-7, 0.88e-7, 0.97e-7.
+    constexpr bool kTwoSum = RS && LB == L_IMQ;
+    constexpr int kLow = kTwoSum ? IA::NI : 1;
+    float rsum[IA::NI], rtot[kLow], rlow[kLow];
     SpLoader<LA, BM, NT> la;
     SpLoader<LB, BN, NT> lb;
     auto seek = [&](int k) {
@@ -586,12 +593,24 @@ gemm_f32_sp(GemmParams p) {
         zero_blocks<MB, NB>(acc);
 #pragma unroll
         for (int i = 0; i < IA::NI; ++i) rsum[i] = 0.f;
+#pragma unroll
+        for (int i = 0; i < kLow; ++i) rtot[i] = rlow[i] = 0.f;
     };
     auto add_rows = [&](const f32x4 (&xa)[IA::NI]) {
         if constexpr (RS)
 #pragma unroll
             for (int i = 0; i < IA::NI; ++i)
                 rsum[i] += (xa[i][0] + xa[i][1]) + (xa[i][2] + xa[i][3]);
+    };
+    auto fold_rows = [&] {
+        if constexpr (kTwoSum)
+#pragma unroll
+            for (int i = 0; i < IA::NI; ++i) {
+                const float s = rtot[i] + rsum[i], u = s - rtot[i];
+                rlow[i] += (rtot[i] - (s - u)) + (rsum[i] - u);
+                rtot[i] = s;
+                rsum[i] = 0.f;
+            }
     };
 
     __shared__ int bad;
@@ -693,6 +712,7 @@ gemm_f32_sp(GemmParams p) {
             for (; kt + 2 < nk; kt += 2) {
                 step(kt, ya, yb, xa, xb);
                 step(kt + 1, xa, xb, ya, yb);
+                if (kTwoSum && (kt & 2)) fold_rows();
             }
             if (kt + 1 < nk) step(kt, ya, yb, xa, xb);
             sp_barrier();
@@ -739,6 +759,9 @@ gemm_f32_sp(GemmParams p) {
     }
 
     if constexpr (RS) {
+        if constexpr (kTwoSum)
+#pragma unroll
+            for (int i = 0; i < IA::NI; ++i) rsum[i] = rtot[i] + (rlow[i] + rsum[i]);
         // The four items of a row: on consecutive lanes (k-contiguous A), or
         // on threads BM apart, through LDS.
         if (id.tn == 0) {

@@ -1257,7 +1257,9 @@ int launch_gemm(GemmParams& p, bool dl, int la, int lb, void* workspace, size_t 
                   plan.ksw ? "ksw" : plan.dl ? "dl" : "rs", plan.bm,
                   plan.bn, layout_name(la), layout_name(halo ? L_IMH : lb), plan.splits,
                   (long long)nblocks, plan.cfg,
-                  p.part ? (p.csum_rows ? " batch-summed rows" : " batch-summed") : "");
+                  p.part ? (p.csum_rows ? " batch-summed rows" : " batch-summed")
+                  : p.rowsum != nullptr ? " rows"   // of A, out of this launch
+                                        : "");
 
     GemmLaunchFn fn = halo ? dlh_launcher(plan.cfg)
                       : lb == L_IM || lb == L_IMR || lb == L_IM4 ? conv_launcher(plan.cfg, lb)
