@@ -4,6 +4,10 @@
 // Python form of the same steps (three ctypes descriptors, two allocations, two
 // foreign calls) took 13 us for a 256x512x512 product whose kernel takes 4.5.
 //
+// The interpreter lock is not held from the first allocation to the last launch,
+// as it was not through the ctypes calls: a launch may wait for a full queue, and
+// what it waits for (a host callback on the stream) may wait for the lock.
+//
 // Every function returns None where a call is not the plain case (an operand
 // that is no fp32 tensor on a GPU, a wrapped or mismatched one): the caller then
 // takes its own path, whose checks and errors are the contract.
@@ -58,9 +62,9 @@ struct Workspace {
     void* p = nullptr;
     size_t n = 0;
     template <class Need>
-    Workspace(py::handle given, const at::Tensor& like, Need need) {
-        if (!given.is_none()) {
-            own = THPVariable_Unpack(given.ptr());
+    Workspace(const at::Tensor& given, const at::Tensor& like, Need need) {
+        if (given.defined()) {
+            own = given;
             n = (size_t)own.numel();
         } else if ((n = need()) > 0) {
             own = at::empty({(int64_t)n}, at::TensorOptions().dtype(at::kByte).device(like.device()));
@@ -69,7 +73,13 @@ struct Workspace {
     }
 };
 
-bool usable_ws(py::handle h) { return h.is_none() || THPVariable_Check(h.ptr()); }
+// The caller's workspace (nothing for None); `ok` is cleared for no tensor.
+at::Tensor given_ws(py::handle h, bool* ok) {
+    if (h.is_none()) return {};
+    if (THPVariable_Check(h.ptr())) return THPVariable_Unpack(h.ptr());
+    *ok = false;
+    return {};
+}
 
 void check(int rc, const char* what) {
     if (rc == MT_OK) return;
@@ -91,7 +101,8 @@ py::object tensor(const at::Tensor& t) {
 
 py::object gemm(py::handle pa, py::handle pb, py::handle pout, py::handle pbias, int axis,
                 float beta, py::handle pws, py::handle stream) {
-    bool ok = usable_ws(pws);
+    bool ok = true;
+    const at::Tensor gws = given_ws(pws, &ok);
     const at::Tensor a = arg(pa, &ok), b = arg(pb, &ok), bias = arg(pbias, &ok);
     at::Tensor out = arg(pout, &ok);
     if (!ok || !a.defined() || !b.defined()) return py::none();
@@ -101,39 +112,46 @@ py::object gemm(py::handle pa, py::handle pb, py::handle pout, py::handle pbias,
         return py::none();
     const int64_t m = a.size(d - 2), n = b.size(d - 1);
     const int64_t batch = d == 3 ? std::max(a.size(0), b.size(0)) : 1;
-    if (!out.defined()) {
-        out = d == 3 ? empty({batch, m, n}, a) : empty({m, n}, a);
-    } else if (out.dim() != d || out.size(d - 2) != m || out.size(d - 1) != n ||
-               (d == 3 && out.size(0) != batch)) {
+    if (out.defined() && (out.dim() != d || out.size(d - 2) != m || out.size(d - 1) != n ||
+                          (d == 3 && out.size(0) != batch)))
         return py::none();
+    void* const s = stream_of(stream);
+    {
+        const py::gil_scoped_release nogil;
+        if (!out.defined()) out = d == 3 ? empty({batch, m, n}, a) : empty({m, n}, a);
+        const mt_mat_f32 ma = mat(a), mb = mat(b), mc = mat(out);
+        mt_epilogue_f32 ep{ptr(bias), bias.defined() ? bias.stride(-1) : 0,
+                           bias.defined() ? axis : MT_BIAS_NONE, beta};
+        const Workspace ws(gws, a, [&] { return mt_gemm_workspace_f32(&ma, &mb, &mc); });
+        check(mt_gemm_f32(&ma, &mb, &mc, bias.defined() || beta != 0.f ? &ep : nullptr, ws.p, ws.n,
+                          s),
+              "mt_gemm_f32");
     }
-    const mt_mat_f32 ma = mat(a), mb = mat(b), mc = mat(out);
-    mt_epilogue_f32 ep{ptr(bias), bias.defined() ? bias.stride(-1) : 0,
-                       bias.defined() ? axis : MT_BIAS_NONE, beta};
-    const Workspace ws(pws, a, [&] { return mt_gemm_workspace_f32(&ma, &mb, &mc); });
-    check(mt_gemm_f32(&ma, &mb, &mc, bias.defined() || beta != 0.f ? &ep : nullptr, ws.p, ws.n,
-                      stream_of(stream)),
-          "mt_gemm_f32");
     return pout.is_none() ? tensor(out) : py::reinterpret_borrow<py::object>(pout);
 }
 
 py::object linear(py::handle px, py::handle pw, py::handle pb, py::handle pout, py::handle pws,
                   py::handle stream) {
-    bool ok = usable_ws(pws);
+    bool ok = true;
+    const at::Tensor gws = given_ws(pws, &ok);
     const at::Tensor x = arg(px, &ok), w = arg(pw, &ok), b = arg(pb, &ok);
     at::Tensor out = arg(pout, &ok);
     if (!ok || !x.defined() || !w.defined() || x.dim() != 2 || w.dim() != 2 ||
         x.size(1) != w.size(1) || (b.defined() && (b.dim() != 1 || b.size(0) != w.size(0))) ||
         (out.defined() && out.dim() != 2))
         return py::none();
-    if (!out.defined()) out = empty({x.size(0), w.size(0)}, x);
-    const mt_mat_f32 mx = mat(x), mw = mat(w), my = mat(out);
-    const Workspace ws(pws, x, [&] {
-        return mt_linear_workspace_f32(x.size(0), x.size(1), w.size(0));
-    });
-    check(mt_linear_forward_f32(&mx, &mw, ptr(b), b.defined() ? b.stride(0) : 0, &my, ws.p, ws.n,
-                                stream_of(stream)),
-          "mt_linear_forward_f32");
+    void* const s = stream_of(stream);
+    {
+        const py::gil_scoped_release nogil;
+        if (!out.defined()) out = empty({x.size(0), w.size(0)}, x);
+        const mt_mat_f32 mx = mat(x), mw = mat(w), my = mat(out);
+        const Workspace ws(gws, x, [&] {
+            return mt_linear_workspace_f32(x.size(0), x.size(1), w.size(0));
+        });
+        check(mt_linear_forward_f32(&mx, &mw, ptr(b), b.defined() ? b.stride(0) : 0, &my, ws.p,
+                                    ws.n, s),
+              "mt_linear_forward_f32");
+    }
     return pout.is_none() ? tensor(out) : py::reinterpret_borrow<py::object>(pout);
 }
 
@@ -141,7 +159,8 @@ py::object linear_backward(py::handle pdy, py::handle px, py::handle pw, bool ne
                            bool need_dw, bool need_db, py::handle pdx, py::handle pdw,
                            py::handle pdb, float beta_w, float beta_b, py::handle pws,
                            py::handle stream) {
-    bool ok = usable_ws(pws);
+    bool ok = true;
+    const at::Tensor gws = given_ws(pws, &ok);
     const at::Tensor dy = arg(pdy, &ok), x = arg(px, &ok), w = arg(pw, &ok);
     at::Tensor dx = arg(pdx, &ok), dw = arg(pdw, &ok), db = arg(pdb, &ok);
     if (!ok || !dy.defined() || !x.defined() || !w.defined() || dy.dim() != 2 || x.dim() != 2 ||
@@ -149,20 +168,23 @@ py::object linear_backward(py::handle pdy, py::handle px, py::handle pw, bool ne
         (db.defined() && db.dim() != 1))
         return py::none();
     const int64_t rows = x.size(0), fin = x.size(1), fout = w.size(0);
-    if (need_dx && !dx.defined()) dx = empty({rows, fin}, x);
-    if (need_dw && !dw.defined()) dw = empty({fout, fin}, x);
-    if (need_db && !db.defined()) db = empty({fout}, x);
-    const mt_mat_f32 mdy = mat(dy), mx = mat(x), mw = mat(w);
-    mt_mat_f32 mdx{}, mdw{};
-    if (need_dx) mdx = mat(dx);
-    if (need_dw) mdw = mat(dw);
-    const Workspace ws(pws, x, [&] { return mt_linear_workspace_f32(rows, fin, fout); });
-    check(mt_linear_backward_f32(&mdy, &mx, &mw, need_dx ? &mdx : nullptr,
-                                 need_dw ? &mdw : nullptr, beta_w,
-                                 need_db ? const_cast<float*>(ptr(db)) : nullptr,
-                                 need_db ? db.stride(0) : 0, beta_b, ws.p, ws.n,
-                                 stream_of(stream)),
-          "mt_linear_backward_f32");
+    void* const s = stream_of(stream);
+    {
+        const py::gil_scoped_release nogil;
+        if (need_dx && !dx.defined()) dx = empty({rows, fin}, x);
+        if (need_dw && !dw.defined()) dw = empty({fout, fin}, x);
+        if (need_db && !db.defined()) db = empty({fout}, x);
+        const mt_mat_f32 mdy = mat(dy), mx = mat(x), mw = mat(w);
+        mt_mat_f32 mdx{}, mdw{};
+        if (need_dx) mdx = mat(dx);
+        if (need_dw) mdw = mat(dw);
+        const Workspace ws(gws, x, [&] { return mt_linear_workspace_f32(rows, fin, fout); });
+        check(mt_linear_backward_f32(&mdy, &mx, &mw, need_dx ? &mdx : nullptr,
+                                     need_dw ? &mdw : nullptr, beta_w,
+                                     need_db ? const_cast<float*>(ptr(db)) : nullptr,
+                                     need_db ? db.stride(0) : 0, beta_b, ws.p, ws.n, s),
+              "mt_linear_backward_f32");
+    }
     const auto back = [](py::handle given, const at::Tensor& t) {
         return given.is_none() ? tensor(t) : py::reinterpret_borrow<py::object>(given);
     };
@@ -171,7 +193,8 @@ py::object linear_backward(py::handle pdy, py::handle px, py::handle pw, bool ne
 
 py::object conv2d(py::handle px, py::handle pw, py::handle pb, int64_t stride, int64_t pad,
                   py::handle pws, py::handle stream) {
-    bool ok = usable_ws(pws);
+    bool ok = true;
+    const at::Tensor gws = given_ws(pws, &ok);
     const at::Tensor x = arg(px, &ok);
     at::Tensor w = arg(pw, &ok), b = arg(pb, &ok);
     if (!ok || !x.defined() || !w.defined() || x.dim() != 4 || w.dim() != 4 ||
@@ -184,19 +207,25 @@ py::object conv2d(py::handle px, py::handle pw, py::handle pb, int64_t stride, i
     const auto extent = [&](int64_t in, int64_t k) {
         return in + 2 * pad < k ? 0 : (in + 2 * pad - k) / stride + 1;
     };
-    at::Tensor out = empty({d.n, d.c_out, extent(d.h, d.kh), extent(d.w, d.kw)}, x);
-    const Workspace ws(pws, x, [&] { return mt_conv2d_workspace_f32(&d); });
-    const int64_t st[4] = {x.stride(0), x.stride(1), x.stride(2), x.stride(3)};
-    check(mt_conv2d_fwd_strided_f32(&d, ptr(x), st, ptr(w), ptr(b), const_cast<float*>(ptr(out)),
-                                    ws.p, ws.n, stream_of(stream)),
-          "mt_conv2d_fwd_strided_f32");
+    void* const s = stream_of(stream);
+    at::Tensor out;
+    {
+        const py::gil_scoped_release nogil;
+        out = empty({d.n, d.c_out, extent(d.h, d.kh), extent(d.w, d.kw)}, x);
+        const Workspace ws(gws, x, [&] { return mt_conv2d_workspace_f32(&d); });
+        const int64_t st[4] = {x.stride(0), x.stride(1), x.stride(2), x.stride(3)};
+        check(mt_conv2d_fwd_strided_f32(&d, ptr(x), st, ptr(w), ptr(b),
+                                        const_cast<float*>(ptr(out)), ws.p, ws.n, s),
+              "mt_conv2d_fwd_strided_f32");
+    }
     return tensor(out);
 }
 
 py::object conv2d_backward(py::handle px, py::handle pw, py::handle pdy, int64_t stride,
                            int64_t pad, bool need_dx, bool need_dw, bool need_db,
                            py::handle pws, py::handle pdw, float beta_w, py::handle stream) {
-    bool ok = usable_ws(pws);
+    bool ok = true;
+    const at::Tensor gws = given_ws(pws, &ok);
     const at::Tensor x = arg(px, &ok), w = arg(pw, &ok), dy = arg(pdy, &ok);
     at::Tensor dw = arg(pdw, &ok);
     if (!ok || !x.defined() || !w.defined() || !dy.defined() || x.dim() != 4 || w.dim() != 4 ||
@@ -212,23 +241,26 @@ py::object conv2d_backward(py::handle px, py::handle pw, py::handle pdy, int64_t
         dy.size(3) != extent(d.w, d.kw) ||
         (need_dw && dw.defined() && (dw.sizes() != w.sizes() || !dw.is_contiguous())))
         return py::none();
-    const Workspace ws(pws, x, [&] { return mt_conv2d_bwd_workspace_f32(&d); });
     void* const s = stream_of(stream);
     const auto out = [](const at::Tensor& t) { return const_cast<float*>(ptr(t)); };
     at::Tensor dx, db;
-    if (need_dx) {
-        dx = empty(x.sizes(), x);
-        check(mt_conv2d_bwd_input_f32(&d, ptr(dy), ptr(w), out(dx), ws.p, ws.n, s),
-              "mt_conv2d_bwd_input_f32");
-    }
-    if (need_db) db = empty({d.c_out}, x);
-    if (need_dw) {
-        if (!dw.defined()) dw = empty(w.sizes(), x);
-        check(mt_conv2d_bwd_weight_bias_f32(&d, ptr(x), ptr(dy), out(dw), beta_w, out(db), 0.f,
-                                            ws.p, ws.n, s),
-              "mt_conv2d_bwd_weight_bias_f32");
-    } else if (need_db) {
-        check(mt_conv2d_bwd_bias_f32(&d, ptr(dy), out(db), 0.f, s), "mt_conv2d_bwd_bias_f32");
+    {
+        const py::gil_scoped_release nogil;
+        const Workspace ws(gws, x, [&] { return mt_conv2d_bwd_workspace_f32(&d); });
+        if (need_dx) {
+            dx = empty(x.sizes(), x);
+            check(mt_conv2d_bwd_input_f32(&d, ptr(dy), ptr(w), out(dx), ws.p, ws.n, s),
+                  "mt_conv2d_bwd_input_f32");
+        }
+        if (need_db) db = empty({d.c_out}, x);
+        if (need_dw) {
+            if (!dw.defined()) dw = empty(w.sizes(), x);
+            check(mt_conv2d_bwd_weight_bias_f32(&d, ptr(x), ptr(dy), out(dw), beta_w, out(db), 0.f,
+                                                ws.p, ws.n, s),
+                  "mt_conv2d_bwd_weight_bias_f32");
+        } else if (need_db) {
+            check(mt_conv2d_bwd_bias_f32(&d, ptr(dy), out(db), 0.f, s), "mt_conv2d_bwd_bias_f32");
+        }
     }
     const py::object rdw = !need_dw          ? py::object(py::none())
                            : !pdw.is_none() ? py::reinterpret_borrow<py::object>(pdw)
