@@ -1253,13 +1253,13 @@ int launch_gemm(GemmParams& p, bool dl, int la, int lb, void* workspace, size_t 
                       halo_fits(p.cv, (int)(N / ((int64_t)p.cv.ho * p.cv.wo)), plan.cfg,
                                 p.k_per_split, !forced);
     std::snprintf(g_last_config, sizeof g_last_config,
-                  "%s %dx%d a=%s b=%s split=%d wgs=%lld cfg=%d%s",
+                  "%s %dx%d a=%s b=%s split=%d wgs=%lld%s cfg=%d%s",
                   plan.ksw ? "ksw" : plan.dl ? "dl" : "rs", plan.bm,
                   plan.bn, layout_name(la), layout_name(halo ? L_IMH : lb), plan.splits,
-                  (long long)nblocks, plan.cfg,
-                  p.part ? (p.csum_rows ? " batch-summed rows" : " batch-summed")
-                  : p.rowsum != nullptr ? " rows"   // of A, out of this launch
-                                        : "");
+                  (long long)nblocks,
+                  p.rowsum != nullptr && !p.part ? " rows" : "",   // of A, out of this launch
+                  plan.cfg,
+                  p.part ? (p.csum_rows ? " batch-summed rows" : " batch-summed") : "");
 
     GemmLaunchFn fn = halo ? dlh_launcher(plan.cfg)
                       : lb == L_IM || lb == L_IMR || lb == L_IM4 ? conv_launcher(plan.cfg, lb)

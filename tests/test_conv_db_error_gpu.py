@@ -23,7 +23,7 @@ def test_db_error(dev, layer):
         want = dy.double().sum((0, 2, 3))
         with mt.forced_config(mt.FAMILY_DL, 0, 64):
             db = mt.conv2d_backward(x, w, dy, s, p, need_dx=False)[2]
-        assert mt.last_config().endswith(" rows"), mt.last_config()   # db came out of the dW launch
+        assert " rows " in mt.last_config(), mt.last_config()   # db came out of the dW launch
         fused += float((db.double() - want).pow(2).sum())
         db = mt.conv2d_backward(x, w, dy, s, p, need_dx=False, need_dw=False)[2]
         alone += float((db.double() - want).pow(2).sum())
