@@ -137,6 +137,7 @@ struct CfgCost {
     int occ;      // resident workgroups per CU
     bool sp = false;   // gemm_f32_sp
     double alone = 0;  // factor of a workgroup alone on its CU (0: the model's own rules)
+    bool lone_store = false;   // its store, alone on its CU, runs beside nothing
 };
 
 // Cost model (in CU cycles) used to pick the tile configuration and split-K
@@ -166,10 +167,13 @@ constexpr CfgCost kRsSpCost[kNumCfg] = {
     {TileCfg<2>::BM, TileCfg<2>::BN, 0.80, 4, true}};
 // Vector layouts.  The efficiencies of gemm_f32_sp's configurations (above 1:
 // bf16 units), its round latency and the factor of a workgroup alone on its CU
-// (kSpAlone) are fitted to graph timings of every configuration at 1-16 splits
-// on 71 shapes (35 GEMMs, 8 batched, 10 of unaligned operands, 18 convolution
-// layers; one MI355X), for the least regret of the pick: 4.4 % on average
-// against the fastest measured plan.
+// (kSpAlone) were fitted to graph timings of every configuration at 1-16 splits
+// on 71 shapes, then held against 1700 drawn calls of this and of the fp32
+// units' plans, every configuration at 1-64 splits timed on each.  Of 496
+// products the picks were 2.6 % above the fastest on average, and 9 more than 5 %
+// slower than the fp32 plans had been; with kProduct64x256, lone_store and
+// kSpBothMn* 2.3 % and 4.  Of 100 layers 6.3 % and 4; with kNarrowShort 5.9 % and
+// none.
 constexpr CfgCost kDlCost[kNumDlCfg] = {
     {DlCfg<0>::BM, DlCfg<0>::BN, 1.08, 2, true},
     {DlCfg<1>::BM, DlCfg<1>::BN, 1.18, 2, true},
@@ -266,8 +270,29 @@ constexpr double kAlonePenalty = 1.3;
 // over short K ranges, where the first loads weigh most; over 512 and more of a
 // matrix operand its MFMAs hide them (2048 x 2048 x 1024 on 128x128 tiles, one
 // per CU: 47.8 us, priced at 57 with the factor; two splits of 256x128 took 59).
+// Below 256 of a matrix operand it is the store of configurations 0 and 1 that
+// runs beside nothing, and costs more than the factor (19 images of 32x32, 112 -> 144
+// channels 1x1: 64x256 tiles, one a CU, 19.5 us; 64x64 now 15.0).
 constexpr double kSpAlone = 1.13;
-constexpr int kSpAloneMinK = 512;
+constexpr int kSpAloneMinK = 512, kLoneStoreMaxK = 256;
+constexpr double kProduct64x256 = 1.04;   // efficiency of configuration 0 with matrix operands
+// The 64x112 tile over short ranges of a split K, where its fill and drain weigh
+// more than the price of a round says (1 image of 28x28, 3x3, 96 -> 416 in 9
+// splits of 96: 25.0 us, 64x64 in 5 of 176: 21.5).
+constexpr double kNarrowShort = 1.03;
+constexpr int kNarrowShortK = 160;
+// Both operands mn-contiguous: 4-byte loads of each, and the tiles of fewer MFMAs
+// a chunk wait for them (256-row and 256-column ones do not).  Measured over
+// predicted at 64-256 of K: 1.27-1.5 on 128x128, 1.3-1.4 on 128x64, 1.0 on
+// 256x128; 144 x 2656 x 2656: 31.6 us on 128x128, 29.5 on 256x128.  (Not over long
+// ranges: 2832 x 3904 x 864 128x128 138 us, 256x128 155.)
+constexpr double kSpBothMn128x128 = 1.10, kSpBothMn128x64 = 1.15;
+constexpr int kSpBothMnMaxK = 512;
+// Operands off 16-byte alignment over at most two chunks of K: the 64x64 tile is
+// the fastest up to 2000^2 and the 128x128 one priced too low for it (3904 x 1120 x 17
+// accumulating: 21.6 us, 12.5 on 64x64).
+constexpr int kRsShortK = 32;
+constexpr double kRsShortEff128 = 0.90;
 constexpr int kMaxForcedSplits = 64;
 
 // Tile grid and K split of configuration `cfg` asked for `s` splits (the
@@ -330,7 +355,8 @@ double plan_cycles(const CostModel& cm, const CfgCost& cc, const Plan& pl, int64
                          : small && pl.kps >= kAloneMinK     ? kAlonePenalty
                          : cc.sp && cc.occ > 1               ? kSpAlone
                                                              : 1.0;
-    double t = per_cu * work * pair * alone + per_cu * epi / cc.occ +
+    const double store = per_cu <= 1 && cc.lone_store ? epi : per_cu * epi / cc.occ;
+    double t = per_cu * work * pair * alone + store +
                rounds * (cc.sp ? cm.sp_round_latency : cm.round_latency);
     if (pl.splits > 1) t += split_cycles(cm, pl.splits, M, N, batch);
     return t;
@@ -339,10 +365,11 @@ double plan_cycles(const CostModel& cm, const CfgCost& cc, const Plan& pl, int64
 // wide: configurations 4-6 (is_wide_cfg) may be chosen (see wide_ok in
 // launch_gemm); sp: gemm_f32_sp can take the operands (sp_fits, sp_layouts); imw: B is the
 // weight-gradient operand (priced by kDlCostImw); im16: the 112-column tile
-// (kNarrowCfg, B = L_IM) may be; im4: B is L_IM4 (configurations 1, 3 and 7).
+// (kNarrowCfg, B = L_IM) may be; im4: B is L_IM4 (configurations 1, 3 and 7);
+// mm: both operands L_MV.
 Plan make_plan_uncached(int64_t M, int64_t N, int64_t K, int64_t batch, int cus,
                         bool allow_split, bool dl, bool wide, bool sp, bool imw, bool im16,
-                        bool im4) {
+                        bool im4, bool mm) {
     static const CostModel cm;
     const CfgCost* cfgs = dl ? (imw ? kDlCostImw : kDlCost) : sp ? kRsSpCost : kRsCost;
     const int ncfg = dl ? kNumDlCfg : kNumCfg;
@@ -361,6 +388,9 @@ Plan make_plan_uncached(int64_t M, int64_t N, int64_t K, int64_t batch, int cus,
         if (im4 && cfg != 1 && cfg != 3 && cfg != kNarrowCfg) continue;
         CfgCost cc = cfgs[cfg];
         if (dl && cfg == 0 && !wide && !im16 && !im4) cc.eff = kImrNarrowEff;   // L_IMR
+        const bool sp_product = dl && wide && !imw && cc.sp;   // matrix operands
+        if (sp_product && cfg == 0) cc.eff = kProduct64x256;
+        if (!dl && sp && cfg == 1 && K <= kRsShortK) cc.eff = kRsShortEff128;
         for (int s = 1; s <= (imw ? kMaxImwSplits : kMaxSplits); ++s) {
             if (s > 1 && !allow_split) break;
             // this and every further split's partials cost more than the best plan
@@ -371,9 +401,14 @@ Plan make_plan_uncached(int64_t M, int64_t N, int64_t K, int64_t batch, int cus,
             if (pl.splits != s) continue;
             const int64_t wgs = (int64_t)pl.tiles_m * pl.tiles_n * batch * pl.splits;
             if (wgs * 512 >= ((int64_t)1 << 32)) continue;
-            if (dl && wide && !imw && cc.sp && cc.occ > 1)
-                cc.alone = pl.kps >= kSpAloneMinK ? 1.0 : kSpAlone;
-            // The 64x112 tile of 16x16 blocks moves about twice the operand
+            CfgCost pc = cc;
+            if (sp_product) {
+                pc.lone_store = cfg <= 1 && pl.kps < kLoneStoreMaxK;
+                pc.alone = pc.lone_store || pl.kps >= kSpAloneMinK ? 1.0 : cc.occ > 1 ? kSpAlone : 0;
+                if (mm && pl.kps < kSpBothMnMaxK)
+                    pc.eff /= cfg == 1 ? kSpBothMn128x128 : cfg == 6 ? kSpBothMn128x64 : 1.0;
+            }
+            // The 64x112 tile moves about twice the operand
             // bytes per flop of the 256x128 one; with one workgroup per CU
             // (nothing co-resident to hide the fetches) it lost everywhere it
             // was measured (the 5a layer: 93.2 us against 80.2 at split 5).
@@ -385,7 +420,8 @@ Plan make_plan_uncached(int64_t M, int64_t N, int64_t K, int64_t batch, int cus,
                 ruled = true;
                 if (small_ws) continue;
             }
-            const double t = plan_cycles(cm, cc, pl, M, N, batch, cus);
+            double t = plan_cycles(cm, pc, pl, M, N, batch, cus);
+            if (im16 && cfg == kNarrowCfg && s > 1 && pl.kps < kNarrowShortK) t *= kNarrowShort;
             if (t < best_t) {
                 best_t = t;
                 best = pl;
@@ -454,16 +490,17 @@ class Recent {
 // thread keeps plans.
 Plan make_plan(int64_t M, int64_t N, int64_t K, int64_t batch, int cus, bool allow_split,
                bool dl, bool wide, bool ksw, bool sp, bool imw = false, bool im16 = false,
-               bool im4 = false) {
+               bool im4 = false, bool mm = false) {
     thread_local Recent<Plan, 8> plans;
     const int flags = allow_split | dl << 1 | wide << 2 | ksw << 3 | sp << 4 | imw << 5 | im16 << 6 |
-                      im4 << 7;
+                      im4 << 7 | mm << 8;
     return plans.get(M, N, K, batch, cus, flags, [&] {
         if (ksw)
             return or_wave_split(make_plan(M, N, K, batch, cus, allow_split, dl, wide, false, sp,
-                                           imw, im16, im4),
+                                           imw, im16, im4, mm),
                                  M, N, K, batch, cus);
-        return make_plan_uncached(M, N, K, batch, cus, allow_split, dl, wide, sp, imw, im16, im4);
+        return make_plan_uncached(M, N, K, batch, cus, allow_split, dl, wide, sp, imw, im16, im4,
+                                  mm);
     });
 }
 
@@ -746,8 +783,10 @@ size_t plan_ws(int64_t M, int64_t N, int64_t K, int64_t batch, int cus) {
         size_t ws = 0;
         for (bool dl : {false, true})
             for (bool sp : {false, true})
-                ws = std::max(ws,
-                              make_plan(M, N, K, batch, cus, true, dl, dl, false, sp).ws_bytes);
+                for (bool mm : {false, true})
+                    if (!mm || (dl && sp))
+                        ws = std::max(ws, make_plan(M, N, K, batch, cus, true, dl, dl, false, sp,
+                                                    false, false, false, mm).ws_bytes);
         return std::max(ws, skinny_ws(M, N, K, batch, cus));
     };
     if (g_forced.family == MT_FAMILY_AUTO) return recent_ws(WS_PLAN, M, N, K, batch, cus, plans);
@@ -1201,11 +1240,12 @@ int launch_gemm(GemmParams& p, bool dl, int la, int lb, void* workspace, size_t 
         // the wave-split kernel takes every operand form but the implicit
         // convolution operands and the fused row sums
         const bool ksw_ok = !implicit && p.rowsum == nullptr;
+        const bool mm = la == L_MV && lb == L_MV;
         plan = make_plan(M, N, K, batch, device_cu_count(), true, dl, wide_ok, ksw_ok, sp_ok,
-                         lb == L_IMW, im16_ok, lb == L_IM4);
+                         lb == L_IMW, im16_ok, lb == L_IM4, mm);
         if (need(plan) > 0 && (workspace == nullptr || ws_bytes < need(plan)))
             plan = make_plan(M, N, K, batch, device_cu_count(), false, dl, wide_ok, ksw_ok, sp_ok,
-                             lb == L_IMW, im16_ok, lb == L_IM4);
+                             lb == L_IMW, im16_ok, lb == L_IM4, mm);
         if (need(plan) > 0 && (workspace == nullptr || ws_bytes < need(plan)))
             return MT_ERR_WORKSPACE;
     }
@@ -2103,9 +2143,12 @@ size_t part_plan_ws(int64_t M, int64_t N, int64_t K, int64_t batch, int cus) {
         for (bool dl : {false, true})
             for (bool wide : {false, true})
                 for (bool sp : {false, true})
-                    w = std::max(
-                        w, part_ws_bytes(make_plan(M, N, K, batch, cus, true, dl, wide, false, sp),
-                                         M, N, batch));
+                    for (bool mm : {false, true})
+                        if (!mm || (wide && sp))
+                            w = std::max(w, part_ws_bytes(make_plan(M, N, K, batch, cus, true, dl,
+                                                                    wide, false, sp, false, false,
+                                                                    false, mm),
+                                                          M, N, batch));
         return w;
     });
     Plan forced;
