@@ -186,9 +186,12 @@ constexpr CfgCost kDlCost[kNumDlCfg] = {
 // The same configurations with the convolution weight gradient's gathered B
 // operand (L_IMW); 0: not offered.  Its gather costs every tile more than a
 // contiguous operand does, the 64x64 ones the most, and a workgroup alone on
-// its CU has nothing to hide it behind.  Fitted to graph timings of the
-// configurations at 1-64 splits on 16 layers (mean error of a time 6 %; the
-// pick is 0.9 % above the fastest measured plan on average).
+// its CU has nothing to hide it behind: not so over short ranges of K on the
+// 64x64 prefetching tile, which has the next fragments read already (n 20,
+// 80 channels 7x7, 3x3 -> 240: 5 splits of 208, one a CU, 20.0 us, 16 of 64
+// 22.7).  Fitted to graph timings of the configurations at 1-64 splits on 16
+// layers, then held against 154 drawn ones and the fp32 units' plans: 29 picks
+// were more than 2 % slower than those, now 7.
 constexpr CfgCost kDlCostImw[kNumDlCfg] = {
     {DlCfg<0>::BM, DlCfg<0>::BN, 0.86, 2, true, 1.11},
     {DlCfg<1>::BM, DlCfg<1>::BN, 0.64, 4, false, 1.0},
@@ -198,6 +201,8 @@ constexpr CfgCost kDlCostImw[kNumDlCfg] = {
     {DlCfg<5>::BM, DlCfg<5>::BN, 0.52, 8, false, 1.47},
     {DlCfg<6>::BM, DlCfg<6>::BN, 0, 3},
     {DlCfg<7>::BM, DlCfg<7>::BN, 0, 2}};   // (configuration 7: L_IM, L_IM4)
+constexpr double kImwShortAlone = 1.05;   // of configuration 5
+constexpr int kImwShortK = 250;
 // And with the 4-byte gathers of an NCHW view (L_IMR), of which a tile of 256
 // columns on 256 threads makes the most per thread: the 7x7 stem at batch 32
 // took 188 us on configuration 0 against 178 on 2.
@@ -408,6 +413,7 @@ Plan make_plan_uncached(int64_t M, int64_t N, int64_t K, int64_t batch, int cus,
                 if (mm && pl.kps < kSpBothMnMaxK)
                     pc.eff /= cfg == 1 ? kSpBothMn128x128 : cfg == 6 ? kSpBothMn128x64 : 1.0;
             }
+            if (imw && cfg == 5 && pl.kps < kImwShortK) pc.alone = kImwShortAlone;
             // The 64x112 tile moves about twice the operand
             // bytes per flop of the 256x128 one; with one workgroup per CU
             // (nothing co-resident to hide the fetches) it lost everywhere it
@@ -1248,6 +1254,15 @@ int launch_gemm(GemmParams& p, bool dl, int la, int lb, void* workspace, size_t 
                              lb == L_IMW, im16_ok, lb == L_IM4, mm);
         if (need(plan) > 0 && (workspace == nullptr || ws_bytes < need(plan)))
             return MT_ERR_WORKSPACE;
+        // The weight gradient on 64x64 tiles: the prefetching kernel, but for a
+        // dY read in NCHW with one workgroup a CU, where the plain one is 1 % faster
+        // (median over 794 timed pairs; with dY copied it is 1-2 % slower at all
+        // ranges of K, and up to 6 at 196 pixels).
+        if (lb == L_IMW && plan.dl && (plan.cfg == kDlSmallCfg || plan.cfg == kDlpSmallCfg))
+            plan.cfg = la == L_KVI && (int64_t)plan.tiles_m * plan.tiles_n * plan.splits <=
+                                          device_cu_count()
+                           ? kDlSmallCfg
+                           : kDlpSmallCfg;
     }
     // The weight gradient's row sums (db from the dY that it reads anyway):
     // partials per split, where configuration 0 splits K and the workspace has

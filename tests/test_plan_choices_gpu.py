@@ -1,4 +1,4 @@
-"""Tiles of calls that lost time when the larger ones moved to the bf16 units:
+"""Tiles and splits of calls that lost time when the larger ones moved to the bf16 units:
 too few workgroups for the first loads or the store to run beside anything, short
 ranges of K, both operands across rows.  (Times of the plan that each had taken,
 and of the one it takes, stand beside the planner's prices.)"""
@@ -38,11 +38,14 @@ PLANS = [
     (lambda d: gemm(d, 709, 2374, 396, tb=True), "64x64"),            # (128x64 would not hide)
     (lambda d: conv(d, 1, 96, 28, 416, 3, 1, 1, "fwd"), "64x64"),      # 64x112 in nine splits
     (lambda d: conv(d, 9, 8, 28, 80, 3, 1, 1, "dx"), "64x112"),        # ... stays where it won
+    (lambda d: conv(d, 20, 80, 7, 240, 3, 1, 1, "dw"), "split=5"),     # 16, three per CU
+    (lambda d: conv(d, 1, 32, 14, 112, 3, 1, 1, "dw"), "cfg=5"),       # the kernel without prefetch
+    (lambda d: conv(d, 4, 16, 32, 48, 3, 1, 1, "dw"), "cfg=2"),        # ... with dY in NCHW stays
 ]
 
 
 @pytest.mark.parametrize("case", range(len(PLANS)))
 def test_tile(dev, case):
     call, tile = PLANS[case]
-    got = call(dev)
+    got = call(dev) + " "
     assert f" {tile} " in got, got
