@@ -576,13 +576,15 @@ gemm_f32_sp(GemmParams p) {
     // Row sums: every thread adds up the items of A that it loads; those of a
     // row meet after the loop, in a fixed order.  Those of a weight gradient's dY
     // would be one chain per thread, where a launch of their own
-    // (block_channel_sum) has eight: every four chunks the sum goes to rtot, and
-    // what that addition rounds off to rlow (Knuth's two-sum).  Error against 64
-    // bits of 32 x 12544 normal values in 512 splits: 1.58e-7 plain, 1.17e-7 so,
-    // 1.26e-7 the launch of their own; 32 x 196 in 8: 1.55e-7, 0.88e-7, 0.97e-7.
-    constexpr bool kTwoSum = RS && LB == L_IMQ;
-    constexpr int kLow = kTwoSum ? IA::NI : 1;
-    float rsum[IA::NI], rtot[kLow], rlow[kLow];
+    // (block_channel_sum) has eight: every two chunks the sum goes to rtot, and
+    // what that addition rounds off (but for an early rtot below rsum) starts the
+    // next sum (Kahan).  Error against 64 bits of normal values, plain / so / the
+    // launch of their own: 32 x 12544 in 512 splits 1.58e-7 / 1.04e-7 / 1.16e-7,
+    // 32 x 196 in 8 1.55e-7 / 0.81e-7 / 0.97e-7; 8 x 784 in 2 0.73e-7 / 0.99e-7.
+    // Its three additions beside the MFMAs cost at most 1 % of a dW (Knuth's
+    // two-sum between the steps had cost 1-5).
+    constexpr bool kFold = RS && LB == L_IMQ;
+    float rsum[IA::NI], rtot[kFold ? IA::NI : 1];
     SpLoader<LA, BM, NT> la;
     SpLoader<LB, BN, NT> lb;
     auto seek = [&](int k) {
@@ -594,7 +596,7 @@ gemm_f32_sp(GemmParams p) {
 #pragma unroll
         for (int i = 0; i < IA::NI; ++i) rsum[i] = 0.f;
 #pragma unroll
-        for (int i = 0; i < kLow; ++i) rtot[i] = rlow[i] = 0.f;
+        for (float& r : rtot) r = 0.f;
     };
     auto add_rows = [&](const f32x4 (&xa)[IA::NI]) {
         if constexpr (RS)
@@ -603,13 +605,12 @@ gemm_f32_sp(GemmParams p) {
                 rsum[i] += (xa[i][0] + xa[i][1]) + (xa[i][2] + xa[i][3]);
     };
     auto fold_rows = [&] {
-        if constexpr (kTwoSum)
+        if constexpr (kFold)
 #pragma unroll
             for (int i = 0; i < IA::NI; ++i) {
-                const float s = rtot[i] + rsum[i], u = s - rtot[i];
-                rlow[i] += (rtot[i] - (s - u)) + (rsum[i] - u);
+                const float s = rtot[i] + rsum[i];
+                rsum[i] -= s - rtot[i];
                 rtot[i] = s;
-                rsum[i] = 0.f;
             }
     };
 
@@ -672,11 +673,12 @@ gemm_f32_sp(GemmParams p) {
             lb.template load<false>(xb, 16, adv);
         };
         auto step = [&](int kt, f32x4 (&xa)[IA::NI], f32x4 (&xb)[IB::NI], f32x4 (&ya)[IA::NI],
-                        f32x4 (&yb)[IB::NI]) {
+                        f32x4 (&yb)[IB::NI], auto fold) {
             sp_barrier();
             fetch(ya, yb);   // (past the last chunk: that chunk again)
             __builtin_amdgcn_sched_barrier(0);   // not behind the MFMAs
             multiply(kt);
+            if constexpr (fold) fold_rows();
             cut(kt + 1, xa, xb);
             // The fragment reads under the first MFMAs (read where they are used,
             // as the compiler had it, each exposed its latency: 3-4 % of the
@@ -710,11 +712,10 @@ gemm_f32_sp(GemmParams p) {
             cut(0, xa, xb);
             int kt = 0;
             for (; kt + 2 < nk; kt += 2) {
-                step(kt, ya, yb, xa, xb);
-                step(kt + 1, xa, xb, ya, yb);
-                if (kTwoSum && (kt & 2)) fold_rows();
+                step(kt, ya, yb, xa, xb, std::false_type{});
+                step(kt + 1, xa, xb, ya, yb, std::true_type{});
             }
-            if (kt + 1 < nk) step(kt, ya, yb, xa, xb);
+            if (kt + 1 < nk) step(kt, ya, yb, xa, xb, std::false_type{});
             sp_barrier();
             multiply(nk - 1);
             mfma_split<MB, NB, 5, 6>(acc, sml, fa, fb);
@@ -759,9 +760,9 @@ gemm_f32_sp(GemmParams p) {
     }
 
     if constexpr (RS) {
-        if constexpr (kTwoSum)
+        if constexpr (kFold)
 #pragma unroll
-            for (int i = 0; i < IA::NI; ++i) rsum[i] = rtot[i] + (rlow[i] + rsum[i]);
+            for (int i = 0; i < IA::NI; ++i) rsum[i] += rtot[i];
         // The four items of a row: on consecutive lanes (k-contiguous A), or
         // on threads BM apart, through LDS.
         if (id.tn == 0) {
