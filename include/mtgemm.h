@@ -264,7 +264,10 @@ const char* mt_last_config(void);
  * fixed kernel per case, src/gpu_ops.cpp:1103-1144).  Kernel families: */
 enum {
     MT_FAMILY_AUTO = 0,  /* the cost model chooses (default)                   */
-    MT_FAMILY_RS = 1,    /* register-staged kernel: any operand layout          */
+    MT_FAMILY_RS = 1,    /* any operand layout: contiguous operands of any
+                            alignment on the bf16 matrix units, other strides on
+                            the register-staged fp32 kernel, both in tiles of
+                            256x128, 128x128 and 64x64                         */
     MT_FAMILY_DL = 2,    /* k- or mn-contiguous operands of 16-byte alignment:
                             configurations 0 (64x256), 1 (128x128), 3 (256x128),
                             4 (128x256) and 6 (128x64) on the bf16 matrix units,

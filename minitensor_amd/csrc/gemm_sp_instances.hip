@@ -1,6 +1,7 @@
 // gemm_sp_instances.hip -- instantiates gemm_f32_sp for one configuration
-// (selected with -DMT_CFG=<n>): the 2x2 contiguous operand layouts with and
-// without the row sums of A, the forward convolution operands (L_IM and L_IMR:
+// (selected with -DMT_CFG=<n>): the 2x2 contiguous operand layouts, two alike
+// also with the row sums of A (not 2, whose operands are off 16-byte alignment:
+// their sums are a launch of its own), the forward convolution operands (L_IM and L_IMR:
 // configurations 0, 1, 3; L_IM4: 1, 3) and the weight gradient's (L_IMW, with dY copied or
 // read in NCHW; not 1 and 2).  Configuration 7: L_IM and
 // L_IM4 only.
@@ -35,8 +36,10 @@ GemmLaunchFn launcher(int la, int lb, bool rs) {
         if (la == L_KV && lb == L_IMW) return launch_sp<L_KV, L_IMQ, true>;
         if (la == L_KVI && lb == L_IMW) return launch_sp<L_KVI, L_IMQ, true>;
 #endif
+#if MT_CFG != 2
         if (la == L_KV && lb == L_KV) return launch_sp<L_KV, L_KV, true>;
         if (la == L_MV && lb == L_MV) return launch_sp<L_MV, L_MV, true>;
+#endif
         return nullptr;
     }
     if (la == L_KV && lb == L_KV) return launch_sp<L_KV, L_KV>;

@@ -7,9 +7,13 @@
 //     h = bf16(x), m = bf16(x - h), l = x - h - m, each rounded to nearest.
 //     8 bits each and a sign hold all 24 bits, and both differences are exact.
 //   * a·b is the sum of six of the nine bf16 products: h·h, and h·m, m·h, m·m,
-//     h·l, l·h, which are 2^-8 of it and less.  The three left out (m·l, l·m,
-//     l·l) are below 2^-26 of a·b, with either sign; a rounding of the fp32 sum
-//     is 2^-25.
+//     h·l, l·h, which are 2^-8 of it and less.  |m| <= 2^-8 |x| and |l| <= 2^-17
+//     |x|, so the three left out (m·l, l·m, l·l) come to at most 2^-24 of a·b,
+//     as much as one rounding of the fp32 sum.  That is reached where both
+//     operands sit just below half an ulp of bf16 (0x1.00ff8p+0, 2^-24.01), and
+//     a sum of such products of one sign is off by as much; normal values: rms
+//     2^-27.4, 3 % of the products beyond 2^-26, either sign (a sum of one or two
+//     products is no better than fp32's, longer ones are).
 //   * Every bf16 product is exact in fp32, and the matrix unit accumulates in
 //     fp32.  h·h has an accumulator of its own, and the five small products
 //     share a second one: the large sum is then rounded once per instruction

@@ -21,6 +21,7 @@
 #include <algorithm>
 #include <cstdio>
 #include <cstring>
+#include <limits>
 
 #include "gemm_configs.hpp"
 #include "mtgemm.h"
@@ -138,6 +139,7 @@ struct CfgCost {
     bool sp = false;   // gemm_f32_sp
     double alone = 0;  // factor of a workgroup alone on its CU (0: the model's own rules)
     bool lone_store = false;   // its store, alone on its CU, runs beside nothing
+    double fixed = 0;     // cycles of a workgroup beside its MFMAs
 };
 
 // Cost model (in CU cycles) used to pick the tile configuration and split-K
@@ -203,10 +205,31 @@ constexpr CfgCost kDlCostImw[kNumDlCfg] = {
     {DlCfg<7>::BM, DlCfg<7>::BN, 0, 2}};   // (configuration 7: L_IM, L_IM4)
 constexpr double kImwShortAlone = 1.05;   // of configuration 5
 constexpr int kImwShortK = 250;
-// And with the 4-byte gathers of an NCHW view (L_IMR), of which a tile of 256
-// columns on 256 threads makes the most per thread: the 7x7 stem at batch 32
-// took 188 us on configuration 0 against 178 on 2.
-constexpr double kImrNarrowEff = 0.80;
+// And with an NCHW view (L_IMR): the 4-byte gathers of gemm_f32_sp (of
+// gemm_f32_dl on 64x64), or the halo patches of gemm_f32_dlh where they fit and
+// pay (imr_price); a workgroup of either has a fixed price, its first gather or
+// patch, which two on a CU do not hide, and the sum of the splits costs what it
+// does in a graph.  Fitted to graph timings of configurations 0-3 at 1-24 splits
+// on 485 stride-1 layers (profiles/nchw_view_plans.md): the picks are 0.7 % above
+// the fastest on average and 7 more than 10 %; with the prices of matrix
+// operands, as if patches were gathered on the bf16 units, 8.1 % and 127.
+constexpr CfgCost kImrCost[4] = {
+    {DlCfg<0>::BM, DlCfg<0>::BN, 0.35, 2, true, 1.10, false, 7600},
+    {DlCfg<1>::BM, DlCfg<1>::BN, 0.85, 2, true, 1.31, false, 2000},
+    {DlCfg<2>::BM, DlCfg<2>::BN, 0.54, 8, false, 1.18, false, 1100},
+    {DlCfg<3>::BM, DlCfg<3>::BN, 1.90, 1, true, 1.18, false, 2600}};
+constexpr CfgCost kHaloCost[4] = {
+    {DlCfg<0>::BM, DlCfg<0>::BN, 0.80, 1, false, 1.20, false, 6000},
+    {DlCfg<1>::BM, DlCfg<1>::BN, 1.01, 4, false, 1.13, false, 7700},
+    {DlCfg<2>::BM, DlCfg<2>::BN, 0.50, 8, false, 1.04, false, 1500},
+    {DlCfg<3>::BM, DlCfg<3>::BN, 0.91, 3, false, 1.35, false, 350}};
+constexpr double kImrLaunchCycles = 2400.0, kImrSplitCycles = 140.0;
+// Sums of less than 256 keep 96 a split (others 64): up to 20 % faster at 64, for
+// outputs whose partials are then many times the output.
+constexpr int kImrShortK = 256, kImrShortMinKps = 96;
+// Configuration 0 where a strided dX's phases are priced against the column
+// buffer (dx_prefer_phased), whatever their operand.
+constexpr double kPhaseNarrowEff = 0.80;
 // Wave-split kernel (configurations of KswCfg): efficiencies from
 // graph-replay timings of every configuration at 1, 2 and 4 K splits on the
 // benchmark's small GEMMs and four neighbouring shapes (one MI355X).  It is
@@ -281,6 +304,11 @@ constexpr double kAlonePenalty = 1.3;
 constexpr double kSpAlone = 1.13;
 constexpr int kSpAloneMinK = 512, kLoneStoreMaxK = 256;
 constexpr double kProduct64x256 = 1.04;   // efficiency of configuration 0 with matrix operands
+// Three chunks of K on outputs of many tiles: 64 of 512 x 512 x 48 25.1 us on
+// 128x128, 26.1 on the 64x64 fp32 tile, which the price of longer sums put first;
+// 4096 x 4096 x 40 25.9, 26.4.  (Two chunks: 22.4, 21.2; the 64x64 one stays.)
+constexpr int kThreeChunks = 48;
+constexpr double kShort128x128 = 1.30;
 // The 64x112 tile over short ranges of a split K, where its fill and drain weigh
 // more than the price of a round says (1 image of 28x28, 3x3, 96 -> 416 in 9
 // splits of 96: 25.0 us, 64x64 in 5 of 176: 21.5).
@@ -293,11 +321,13 @@ constexpr int kNarrowShortK = 160;
 // ranges: 2832 x 3904 x 864 128x128 138 us, 256x128 155.)
 constexpr double kSpBothMn128x128 = 1.10, kSpBothMn128x64 = 1.15;
 constexpr int kSpBothMnMaxK = 512;
-// Operands off 16-byte alignment over at most two chunks of K: the 64x64 tile is
-// the fastest up to 2000^2 and the 128x128 one priced too low for it (3904 x 1120 x 17
-// accumulating: 21.6 us, 12.5 on 64x64).
+// Operands off 16-byte alignment over at most two chunks of K: the 64x64 tile,
+// at any size (256 x 65856 x 7: 32.2 us, 45.3 on 128x128, where the fp32 kernel of
+// that tile took 36.2; 432 x 24304 x 9: 26.8, 35.3, 26.7; 43 of 632 x 376 x 31:
+// 18.7, 21.9, 18.1; the largest loss 416 x 12544 x 31: 30.5, 29.4), which the
+// price of the 128x128 one at its other lengths does not say.
 constexpr int kRsShortK = 32;
-constexpr double kRsShortEff128 = 0.90;
+constexpr double kRsShortEff128 = 0.60;
 constexpr int kMaxForcedSplits = 64;
 
 // Tile grid and K split of configuration `cfg` asked for `s` splits (the
@@ -361,21 +391,30 @@ double plan_cycles(const CostModel& cm, const CfgCost& cc, const Plan& pl, int64
                          : cc.sp && cc.occ > 1               ? kSpAlone
                                                              : 1.0;
     const double store = per_cu <= 1 && cc.lone_store ? epi : per_cu * epi / cc.occ;
-    double t = per_cu * work * pair * alone + store +
+    double t = per_cu * (work * pair * alone + cc.fixed) + store +
                rounds * (cc.sp ? cm.sp_round_latency : cm.round_latency);
     if (pl.splits > 1) t += split_cycles(cm, pl.splits, M, N, batch);
     return t;
+}
+
+// The price of an NCHW view: 1, a bit for each of configurations 0-3 whose halo
+// patches fit and are small enough to pay, and above them the taps, of which a K
+// range must hold 16 times as many for them to be taken (halo_fits).
+int imr_price(const ConvGeom& g, int64_t n_img);
+bool imr_halo(int imr, int cfg, int64_t kps) {
+    return (imr >> (1 + cfg) & 1) != 0 && kps >= 16 * (int64_t)(imr >> 5);
 }
 
 // wide: configurations 4-6 (is_wide_cfg) may be chosen (see wide_ok in
 // launch_gemm); sp: gemm_f32_sp can take the operands (sp_fits, sp_layouts); imw: B is the
 // weight-gradient operand (priced by kDlCostImw); im16: the 112-column tile
 // (kNarrowCfg, B = L_IM) may be; im4: B is L_IM4 (configurations 1, 3 and 7);
-// mm: both operands L_MV.
+// mm: both operands L_MV; imr: B is L_IMR (imr_price).
 Plan make_plan_uncached(int64_t M, int64_t N, int64_t K, int64_t batch, int cus,
                         bool allow_split, bool dl, bool wide, bool sp, bool imw, bool im16,
-                        bool im4, bool mm) {
-    static const CostModel cm;
+                        bool im4, bool mm, int imr) {
+    static const CostModel matrix_cm, imr_cm{.launch_cycles = kImrLaunchCycles};
+    const CostModel& cm = imr ? imr_cm : matrix_cm;
     const CfgCost* cfgs = dl ? (imw ? kDlCostImw : kDlCost) : sp ? kRsSpCost : kRsCost;
     const int ncfg = dl ? kNumDlCfg : kNumCfg;
     Plan best;
@@ -392,21 +431,23 @@ Plan make_plan_uncached(int64_t M, int64_t N, int64_t K, int64_t batch, int cus,
         if (dl && cfg == kNarrowCfg && !im16 && !im4) continue;
         if (im4 && cfg != 1 && cfg != 3 && cfg != kNarrowCfg) continue;
         CfgCost cc = cfgs[cfg];
-        if (dl && cfg == 0 && !wide && !im16 && !im4) cc.eff = kImrNarrowEff;   // L_IMR
+        if (dl && cfg == 0 && !wide && !im16 && !im4) cc.eff = kPhaseNarrowEff;
         const bool sp_product = dl && wide && !imw && cc.sp;   // matrix operands
         if (sp_product && cfg == 0) cc.eff = kProduct64x256;
+        if (sp_product && cfg == 1 && K <= kThreeChunks) cc.eff = kShort128x128;
         if (!dl && sp && cfg == 1 && K <= kRsShortK) cc.eff = kRsShortEff128;
         for (int s = 1; s <= (imw ? kMaxImwSplits : kMaxSplits); ++s) {
             if (s > 1 && !allow_split) break;
             // this and every further split's partials cost more than the best plan
             if (s > 1 && split_cycles(cm, s, M, N, batch) > best_t) break;
             const Plan pl = cfg_plan(cc, cfg, dl, M, N, K, batch, s);
-            if (s > 1 && pl.kps < 64) break;
+            if (s > 1 && pl.kps < (imr && K < kImrShortK ? kImrShortMinKps : 64)) break;
             if (s > kFittedSplits && pl.kps < kMinKpsBeyondFit) break;
             if (pl.splits != s) continue;
             const int64_t wgs = (int64_t)pl.tiles_m * pl.tiles_n * batch * pl.splits;
             if (wgs * 512 >= ((int64_t)1 << 32)) continue;
             CfgCost pc = cc;
+            if (imr) pc = (imr_halo(imr, cfg, s > 1 ? pl.kps : K) ? kHaloCost : kImrCost)[cfg];
             if (sp_product) {
                 pc.lone_store = cfg <= 1 && pl.kps < kLoneStoreMaxK;
                 pc.alone = pc.lone_store || pl.kps >= kSpAloneMinK ? 1.0 : cc.occ > 1 ? kSpAlone : 0;
@@ -427,6 +468,7 @@ Plan make_plan_uncached(int64_t M, int64_t N, int64_t K, int64_t batch, int cus,
                 if (small_ws) continue;
             }
             double t = plan_cycles(cm, pc, pl, M, N, batch, cus);
+            if (imr && s > 1) t += kImrSplitCycles * s;
             if (im16 && cfg == kNarrowCfg && s > 1 && pl.kps < kNarrowShortK) t *= kNarrowShort;
             if (t < best_t) {
                 best_t = t;
@@ -496,17 +538,17 @@ class Recent {
 // thread keeps plans.
 Plan make_plan(int64_t M, int64_t N, int64_t K, int64_t batch, int cus, bool allow_split,
                bool dl, bool wide, bool ksw, bool sp, bool imw = false, bool im16 = false,
-               bool im4 = false, bool mm = false) {
+               bool im4 = false, bool mm = false, int imr = 0) {
     thread_local Recent<Plan, 8> plans;
     const int flags = allow_split | dl << 1 | wide << 2 | ksw << 3 | sp << 4 | imw << 5 | im16 << 6 |
-                      im4 << 7 | mm << 8;
+                      im4 << 7 | mm << 8 | imr << 9;
     return plans.get(M, N, K, batch, cus, flags, [&] {
         if (ksw)
             return or_wave_split(make_plan(M, N, K, batch, cus, allow_split, dl, wide, false, sp,
-                                           imw, im16, im4, mm),
+                                           imw, im16, im4, mm, imr),
                                  M, N, K, batch, cus);
         return make_plan_uncached(M, N, K, batch, cus, allow_split, dl, wide, sp, imw, im16, im4,
-                                  mm);
+                                  mm, imr);
     });
 }
 
@@ -515,9 +557,10 @@ Plan make_plan(int64_t M, int64_t N, int64_t K, int64_t batch, int cus, bool all
 // workspace, needs what any plan of the same operands does.
 enum WsKind { WS_PLAN, WS_PART, WS_IMPLICIT, WS_IMPLICIT_IM4, WS_IMW };
 template <class F>
-size_t recent_ws(WsKind kind, int64_t M, int64_t N, int64_t K, int64_t batch, int cus, F make) {
+size_t recent_ws(WsKind kind, int64_t M, int64_t N, int64_t K, int64_t batch, int cus, F make,
+                 int imr = 0) {
     thread_local Recent<size_t, 7> sizes;
-    return sizes.get(M, N, K, batch, cus, kind, make);
+    return sizes.get(M, N, K, batch, cus, kind | imr << 3, make);
 }
 
 // Configuration forced on this thread's launches by mt_gemm_force_config.
@@ -641,6 +684,27 @@ bool halo_fits(const ConvGeom& g, int n_img, int cfg, int kps, bool cost) {
 void set_halo_geometry(ConvGeom& g) {
     g.hp = (g.ho - 1) * g.stride + g.kh;
     g.pw = (g.wo - 1) * g.stride + g.kw;
+}
+
+// (By the shape alone, as if the view were dense: a workspace query knows no
+// strides.)
+int imr_price(const ConvGeom& view, int64_t n_img) {
+    ConvGeom g = view;
+    g.sw = 1; g.sh = g.w; g.sc = (int64_t)g.h * g.w; g.img_stride = g.c * g.sc;
+    int fits = 0;
+    for (int cfg = 0; cfg < 4; ++cfg)
+        if (halo_fits(g, (int)n_img, cfg, std::numeric_limits<int>::max(), true)) fits |= 1 << cfg;
+    return 1 | fits << 1 | (fits ? g.kh * g.kw : 0) << 5;
+}
+
+// The extents of a convolution over an NCHW view.
+ConvGeom nchw_geometry(const mt_conv2d_desc* d, int64_t Ho, int64_t Wo) {
+    ConvGeom g{};
+    g.c = (int)d->c_in; g.h = (int)d->h; g.w = (int)d->w;
+    g.kh = (int)d->kh; g.kw = (int)d->kw; g.stride = (int)d->stride; g.pad = g.pad_w = (int)d->pad;
+    g.ho = (int)Ho; g.wo = (int)Wo;
+    set_halo_geometry(g);
+    return g;
 }
 
 GemmLaunchFn conv_launcher(int cfg, int lb) {
@@ -1247,11 +1311,14 @@ int launch_gemm(GemmParams& p, bool dl, int la, int lb, void* workspace, size_t 
         // convolution operands and the fused row sums
         const bool ksw_ok = !implicit && p.rowsum == nullptr;
         const bool mm = la == L_MV && lb == L_MV;
+        const int imr = lb == L_IMR && p.cv.hp > 0
+                            ? imr_price(p.cv, N / ((int64_t)p.cv.ho * p.cv.wo))
+                            : 0;
         plan = make_plan(M, N, K, batch, device_cu_count(), true, dl, wide_ok, ksw_ok, sp_ok,
-                         lb == L_IMW, im16_ok, lb == L_IM4, mm);
+                         lb == L_IMW, im16_ok, lb == L_IM4, mm, imr);
         if (need(plan) > 0 && (workspace == nullptr || ws_bytes < need(plan)))
             plan = make_plan(M, N, K, batch, device_cu_count(), false, dl, wide_ok, ksw_ok, sp_ok,
-                             lb == L_IMW, im16_ok, lb == L_IM4, mm);
+                             lb == L_IMW, im16_ok, lb == L_IM4, mm, imr);
         if (need(plan) > 0 && (workspace == nullptr || ws_bytes < need(plan)))
             return MT_ERR_WORKSPACE;
         // The weight gradient on 64x64 tiles: the prefetching kernel, but for a
@@ -2200,12 +2267,9 @@ int run_conv_nchw(const mt_conv2d_desc* d, int64_t Ho, int64_t Wo, const float* 
     p.beta = 0.f;
     p.M = (int)d->c_out; p.N = (int)np; p.K = (int)kg; p.batch = 1;
     ConvGeom& g = p.cv;
+    g = nchw_geometry(d, Ho, Wo);
     g.img_stride = in_strides[0];
     g.sc = in_strides[1]; g.sh = in_strides[2]; g.sw = in_strides[3];
-    g.c = (int)d->c_in; g.h = (int)d->h; g.w = (int)d->w;
-    g.kh = (int)d->kh; g.kw = (int)d->kw; g.stride = (int)d->stride; g.pad = g.pad_w = (int)d->pad;
-    g.ho = (int)Ho; g.wo = (int)Wo;
-    set_halo_geometry(g);
     return launch_gemm(p, true, L_KV, L_IMR, workspace, ws_bytes, s);
 }
 
@@ -2507,19 +2571,20 @@ bool dx_prefer_phased(const mt_conv2d_desc* d, int64_t Ho, int64_t Wo, bool cl) 
 }
 
 // Workspace of one implicit-operand GEMM (L_IM / L_IMR: the direct-to-LDS
-// configurations 0-3 and 7; L_IMW, imw: 0-6),
+// configurations 0-3 and 7; L_IMW, imw: 0-6; L_IMR: its imr_price),
 // including a forced configuration's partials: what launch_gemm may use.
-size_t implicit_gemm_ws(int64_t M, int64_t N, int64_t K, bool imw, bool im4 = false) {
+size_t implicit_gemm_ws(int64_t M, int64_t N, int64_t K, bool imw, bool im4 = false, int imr = 0) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     const int cus = device_cu_count();
     const WsKind kind = imw ? WS_IMW : im4 ? WS_IMPLICIT_IM4 : WS_IMPLICIT;
     size_t ws = recent_ws(kind, M, N, K, 1, cus, [&] {
         size_t w = 0;
         for (bool sp : {false, true}) {
-            const Plan pl = make_plan(M, N, K, 1, cus, true, true, imw, false, sp, imw);
+            const Plan pl = make_plan(M, N, K, 1, cus, true, true, imw, false, sp, imw, false,
+                                      false, false, imr);
             // (with the weight gradient's row sums: M floats per split)
             w = std::max(w, pl.ws_bytes + (imw && pl.splits > 1 ? (size_t)pl.splits * M * 4 : 0));
-            if (!imw)   // the channels-last operand may take configuration 7
+            if (!imw && !imr)   // the channels-last operand may take configuration 7
                 w = std::max(w, make_plan(M, N, K, 1, cus, true, true, false, false, sp, false,
                                           true).ws_bytes);
         }
@@ -2527,10 +2592,26 @@ size_t implicit_gemm_ws(int64_t M, int64_t N, int64_t K, bool imw, bool im4 = fa
             w = std::max(w, make_plan(M, N, K, 1, cus, true, true, false, false, true, false,
                                       false, true).ws_bytes);
         return w;
-    });
+    }, imr);
     Plan f;
     if (forced_plan(M, N, K, 1, true, false, imw, true, &f, !imw)) ws = std::max(ws, f.ws_bytes);
     return ws;
+}
+
+// ... of the convolution d over an NCHW view.
+size_t nchw_gemm_ws(const mt_conv2d_desc* d, int64_t Ho, int64_t Wo) {
+    return implicit_gemm_ws(d->c_out, d->n * Ho * Wo, d->c_in * d->kh * d->kw, false, false,
+                            imr_price(nchw_geometry(d, Ho, Wo), d->n));
+}
+
+// The stride-1 convolution of dY (in NCHW, strides not set) that gives a phase of dX.
+ConvGeom phase_geometry(const mt_conv2d_desc* d, const DxPhase& f, int64_t Ho, int64_t Wo) {
+    ConvGeom g{};
+    g.c = (int)d->c_out; g.h = (int)Ho; g.w = (int)Wo;
+    g.kh = f.jh; g.kw = f.jw; g.stride = 1; g.pad = f.pad_h; g.pad_w = f.pad_w;
+    g.ho = f.hp; g.wo = f.wp;
+    set_halo_geometry(g);
+    return g;
 }
 
 // Layout of the phased dX workspace: [channels-last dY (cl)][phase weights]
@@ -2552,7 +2633,9 @@ DxPhasedWs dx_phased_ws(const mt_conv2d_desc* d, int64_t Ho, int64_t Wo, bool cl
             // stride 1: the one phase is dX itself, written in place
             if (t.s > 1)
                 w.z += align_up((size_t)d->n * d->c_in * f.hp * f.wp * sizeof(float), 256);
-            w.gemm = std::max(w.gemm, implicit_gemm_ws(d->c_in, d->n * f.hp * f.wp, f.k, false));
+            const int imr = cl ? 0 : imr_price(phase_geometry(d, f, Ho, Wo), d->n);
+            w.gemm = std::max(w.gemm, implicit_gemm_ws(d->c_in, d->n * f.hp * f.wp, f.k, false,
+                                                       false, imr));
         }
     }
     return w;
@@ -2573,7 +2656,7 @@ size_t dx_ws(const mt_conv2d_desc* d, int64_t Ho, int64_t Wo) {
         return iw.xt + iw.wt + implicit_gemm_ws(d->c_in, nx, kx, false);
     }
     if (dx_as_forward(d, Ho, Wo, &t) && nchw_implicit(&t))
-        return flipped_ws(d) + implicit_gemm_ws(d->c_in, nx, kx, false);
+        return flipped_ws(d) + nchw_gemm_ws(&t, d->h, d->w);
     bool cl = false;
     if (dx_phased(d, Ho, Wo, &cl) && dx_prefer_phased(d, Ho, Wo, cl)) {
         const DxPhasedWs w = dx_phased_ws(d, Ho, Wo, cl);
@@ -2662,14 +2745,9 @@ int run_dx_phased(const mt_conv2d_desc* d, int64_t Ho, int64_t Wo, bool cl,
         p.beta = 0.f;
         p.M = (int)d->c_in; p.N = (int)(d->n * f.hp * f.wp); p.K = f.k; p.batch = 1;
         ConvGeom& g = p.cv;
+        g = phase_geometry(d, f, Ho, Wo);
         g.img_stride = d->c_out * hw;
-        g.c = (int)d->c_out; g.h = (int)Ho; g.w = (int)Wo;
-        g.kh = f.jh; g.kw = f.jw; g.stride = 1; g.pad = f.pad_h; g.pad_w = f.pad_w;
-        g.ho = f.hp; g.wo = f.wp;
-        if (!cl) {
-            g.sc = hw; g.sh = Wo; g.sw = 1;
-            set_halo_geometry(g);
-        }
+        if (!cl) g.sc = hw, g.sh = Wo, g.sw = 1;
         const int rc = launch_gemm(p, true, L_KV, cl ? L_IM : L_IMR, gws, gws_b, s);
         if (rc != MT_OK) return rc;
     }
@@ -2792,7 +2870,7 @@ size_t mt_conv2d_workspace_f32(const mt_conv2d_desc* d) {
     // index takes the NCHW-view kernel instead
     if (pointwise(d))
         return std::max(plan_ws(d->c_out, d->h * d->w, d->c_in, d->n, device_cu_count()),
-                        nchw_weight_ws(d) + implicit_gemm_ws(d->c_out, np, kg, false));
+                        nchw_weight_ws(d) + nchw_gemm_ws(d, Ho, Wo));
     if (implicit_geometry(d) && d->h * d->w < kMaxDim) {   // channels-last kernel
         const ImplicitWs iw = implicit_ws(d);
         const size_t cl = iw.xt + iw.wt + implicit_gemm_ws(d->c_out, np, kg, false);
@@ -2802,7 +2880,7 @@ size_t mt_conv2d_workspace_f32(const mt_conv2d_desc* d) {
     }
     // the NCHW-view kernel: split-K partials, and room for an aligned copy of
     // the weights (used only when the caller's are not 16-byte aligned)
-    if (nchw_implicit(d)) return nchw_weight_ws(d) + implicit_gemm_ws(d->c_out, np, kg, false);
+    if (nchw_implicit(d)) return nchw_weight_ws(d) + nchw_gemm_ws(d, Ho, Wo);
     const size_t col = align_up((size_t)kg * np * sizeof(float), 256) +
                        plan_ws(d->c_out, np, kg, 1, device_cu_count());
     // a dense input takes the padded NCHW-view path; other views the column one
@@ -2810,7 +2888,9 @@ size_t mt_conv2d_workspace_f32(const mt_conv2d_desc* d) {
     if (fwd_padded(d, &d4)) {
         const DwPadWs pw = dw_pad_ws(&d4);
         return std::max(col, pw.xp + pw.dw4 +
-                                 implicit_gemm_ws(d->c_out, np, d4.c_in * d->kh * d->kw, false, true));
+                                 std::max(implicit_gemm_ws(d->c_out, np, d4.c_in * d->kh * d->kw,
+                                                           false, true),
+                                          nchw_gemm_ws(&d4, Ho, Wo)));
     }
     return col;
 }
