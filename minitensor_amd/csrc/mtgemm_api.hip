@@ -157,7 +157,11 @@ constexpr CfgCost kRsCost[kNumCfg] = {      // register-staged kernel, any strid
     {TileCfg<0>::BM, TileCfg<0>::BN, 0.80, 1},
     {TileCfg<1>::BM, TileCfg<1>::BN, 0.75, 2},
     {TileCfg<2>::BM, TileCfg<2>::BN, 0.57, 4}};
-// The same tiles on gemm_f32_sp, for contiguous operands of any alignment.
+// The same tiles on gemm_f32_sp, for contiguous operands of any alignment.  Held
+// against graph timings of them and of the wave-split tiles, 1-16 splits, on 381
+// drawn products: the 64x64 tile at 0.80 and 128x128 at 1.11 had the latter taken
+// at 50-400 of K where it is the slower one (91 of 322 x 235 x 88 40.8 us, 64x64
+// 34.2; 3710 x 2591 x 64 41.0, 36.5); none of the 381 picks loses 3 % by the change.
 constexpr int kRsSpCfg[kNumCfg] = {3, 1, 2};
 static_assert(SpCfg<3>::BM == TileCfg<0>::BM && SpCfg<3>::BN == TileCfg<0>::BN &&
                   SpCfg<1>::BM == TileCfg<1>::BM && SpCfg<1>::BN == TileCfg<1>::BN &&
@@ -165,8 +169,8 @@ static_assert(SpCfg<3>::BM == TileCfg<0>::BM && SpCfg<3>::BN == TileCfg<0>::BN &
               "the register-staged configurations' tiles on both kernels");
 constexpr CfgCost kRsSpCost[kNumCfg] = {
     {TileCfg<0>::BM, TileCfg<0>::BN, 1.54, 1, true},
-    {TileCfg<1>::BM, TileCfg<1>::BN, 1.11, 2, true},
-    {TileCfg<2>::BM, TileCfg<2>::BN, 0.80, 4, true}};
+    {TileCfg<1>::BM, TileCfg<1>::BN, 1.00, 2, true},
+    {TileCfg<2>::BM, TileCfg<2>::BN, 0.86, 4, true}};
 // Vector layouts.  The efficiencies of gemm_f32_sp's configurations (above 1:
 // bf16 units), its round latency and the factor of a workgroup alone on its CU
 // (kSpAlone) were fitted to graph timings of every configuration at 1-16 splits
@@ -210,8 +214,8 @@ constexpr int kImwShortK = 250;
 // pay (imr_price); a workgroup of either has a fixed price, its first gather or
 // patch, which two on a CU do not hide, and the sum of the splits costs what it
 // does in a graph.  Fitted to graph timings of configurations 0-3 at 1-24 splits
-// on 485 stride-1 layers (profiles/nchw_view_plans.md): the picks are 0.7 % above
-// the fastest on average and 7 more than 10 %; with the prices of matrix
+// on 485 stride-1 layers (profiles/nchw_view_plans.md): the picks are 1.5 % above
+// the fastest on average and 22 more than 10 %; with the prices of matrix
 // operands, as if patches were gathered on the bf16 units, 8.1 % and 127.
 constexpr CfgCost kImrCost[4] = {
     {DlCfg<0>::BM, DlCfg<0>::BN, 0.35, 2, true, 1.10, false, 7600},
