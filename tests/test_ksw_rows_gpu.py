@@ -21,6 +21,10 @@ def test_db_from_the_wave_split_dw(dev, cfg, rows, fin, fout):
     W = torch.zeros(fout, fin, device=dev)
     with mt.forced_config(mt.FAMILY_KSW, cfg, 1):
         mt.linear_backward(dY, X, W, need_dx=False, dw=dw, db=db, beta_w=1.0, beta_b=0.5)
+        name = mt.last_config()
+    # db out of this launch on 16x16 blocks (0: 32x32 ones, a launch of its own)
+    assert name.startswith("ksw ") and f" cfg={cfg}" in name, name
+    assert (" rows " in name) == (cfg != 0), name
     x64, y64 = x.astype(np.float64), dy.astype(np.float64)
     # rows + 2 roundings of 2^-24, each of at most the sum of the magnitudes
     eps = (rows + 2) * 2.0 ** -24

@@ -16,8 +16,26 @@ class Declined:
         return lambda *a, **k: None
 
 
+class Recorded:
+    """The binding, with what it answered."""
+
+    def __init__(self, real, answers):
+        self.real, self.answers = real, answers
+
+    def __getattr__(self, name):
+        def call(*a, **k):
+            r = getattr(self.real, name)(*a, **k)
+            self.answers.append(r)
+            return r
+        return call
+
+
 def both(monkeypatch, call):
-    got = call()
+    answers, real = [], mt.native()
+    with monkeypatch.context() as m:
+        m.setattr(mt, "native", lambda: Recorded(real, answers))
+        got = call()
+    assert answers and all(r is not None for r in answers)   # it took the call
     with monkeypatch.context() as m:
         m.setattr(mt, "native", Declined)
         want = call()

@@ -36,6 +36,12 @@ def check(got, a, b, extra, k):
     bound = (k + 4) * 2.0 ** -24 * (np.abs(a64) @ np.abs(b64) + np.abs(extra)) + 2.0 ** -126
     err = np.abs(got.double().cpu().numpy() - want)
     assert (err <= bound).all(), float((err / bound).max())
+    # A product of the six that is lost somewhere (2.4e-6 of the result's 2-norm for
+    # the smallest, from its definition on normal values) may hide below that bound:
+    # 1.5 times the 6.4e-9 sqrt(k) measured for sums of k, and roundings of the result
+    if want.size >= 1000 and k >= 16 and 1e-30 < np.abs(want).max() and np.abs(a).max() < 100:
+        norm = float(np.linalg.norm(err) / np.linalg.norm(want))
+        assert norm <= 3e-7 + 1.5 * 6.4e-9 * k ** 0.5, (norm, k, mt.last_config())
 
 
 @pytest.mark.parametrize("fam,cfg,bm,bn", TILES)
@@ -45,7 +51,7 @@ def test_tile_edges(dev, fam, cfg, bm, bn, a_k, b_k):
     aligned = fam == mt.FAMILY_DL
     step = 4 if aligned else 1   # the direct family's extents: multiples of four
     sizes = [(step, step, step), (bm, bn, 16), (bm - step, bn + step, 32 + step),
-             (bm + step, bn - step, 208 - step), (2 * bm + step, bn, 64)]
+             (bm + step, bn - step, 208 - step), (2 * bm + step, bn, 64), (bm, bn, 32)]
     for (m, n, k), splits in [(s, 1) for s in sizes] + [(sizes[3], 3)]:
         off = 0 if aligned else 1 + (m & 1)
         a, A = operand(rng, m, k, a_k, off, dev)
@@ -56,6 +62,8 @@ def test_tile_edges(dev, fam, cfg, bm, bn, a_k, b_k):
         with mt.forced_config(fam, cfg, splits):
             mt.gemm(A, B.t(), out=C, bias=torch.from_numpy(bias).to(dev), bias_axis=mt.BIAS_COL,
                     beta=0.5)
+        name = mt.last_config()
+        assert name.startswith("dl " if aligned else "rs ") and name.endswith(f" cfg={cfg}"), name
         want = 0.5 * c.astype(np.float64) + bias
         check(C, a, np.ascontiguousarray(b.T), want, k)
 
@@ -92,3 +100,20 @@ def test_values_outside_the_cut(dev, fam, cfg, bm, bn):
     assert (got[9] == (a[9, 2] * b[:, 2].astype(np.float64)).astype(np.float32)).all()
     rest = [r for r in range(m - 1) if r not in (1, 5, 6, 9)]
     check(torch.from_numpy(got[rest]), a[rest], np.ascontiguousarray(b.T), 0.0, k)
+
+
+@pytest.mark.parametrize("fam,cfg,bm,bn", TILES)
+def test_worst_operands(dev, fam, cfg, bm, bn):
+    """0x1.00ff8p+0 is cut into 1 + 2^-8 - 2^-17: the products left out come to 2^-24
+    of each product, all of one sign, and grow with the sum."""
+    v = float.fromhex("0x1.00ff8p+0")
+    for k in (16, 256, 4096, 16384):
+        with mt.forced_config(fam, cfg, 1):
+            got = mt.gemm(torch.full((bm, k), v, device=dev), torch.full((k, bn), v, device=dev))
+        # 2^-24 left out and 2^-24 of the last additions (h.h, all ones, sums exactly);
+        # the small products are 2^-7 of the sum, which the unit rounds to 2^-23 and
+        # not to nearest at each of 5 k/16 instructions
+        bound = 2.0 ** -23 + 5 * k / 16 * 2.0 ** -30
+        err = float((got.double() / (k * v * v) - 1).abs().max())
+        print(f"[worst] {mt.last_config()} k={k} {err:.3g} of {bound:.3g}", flush=True)
+        assert err <= bound, (k, err, bound)
