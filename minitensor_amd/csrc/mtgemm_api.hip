@@ -157,11 +157,7 @@ constexpr CfgCost kRsCost[kNumCfg] = {      // register-staged kernel, any strid
     {TileCfg<0>::BM, TileCfg<0>::BN, 0.80, 1},
     {TileCfg<1>::BM, TileCfg<1>::BN, 0.75, 2},
     {TileCfg<2>::BM, TileCfg<2>::BN, 0.57, 4}};
-// The same tiles on gemm_f32_sp, for contiguous operands of any alignment.  Held
-// against graph timings of them and of the wave-split tiles, 1-16 splits, on 381
-// drawn products: the 64x64 tile at 0.80 and 128x128 at 1.11 had the latter taken
-// at 50-400 of K where it is the slower one (91 of 322 x 235 x 88 40.8 us, 64x64
-// 34.2; 3710 x 2591 x 64 41.0, 36.5); none of the 381 picks loses 3 % by the change.
+// The same tiles on gemm_f32_sp, for contiguous operands of any alignment.
 constexpr int kRsSpCfg[kNumCfg] = {3, 1, 2};
 static_assert(SpCfg<3>::BM == TileCfg<0>::BM && SpCfg<3>::BN == TileCfg<0>::BN &&
                   SpCfg<1>::BM == TileCfg<1>::BM && SpCfg<1>::BN == TileCfg<1>::BN &&
@@ -169,8 +165,20 @@ static_assert(SpCfg<3>::BM == TileCfg<0>::BM && SpCfg<3>::BN == TileCfg<0>::BN &
               "the register-staged configurations' tiles on both kernels");
 constexpr CfgCost kRsSpCost[kNumCfg] = {
     {TileCfg<0>::BM, TileCfg<0>::BN, 1.54, 1, true},
-    {TileCfg<1>::BM, TileCfg<1>::BN, 1.00, 2, true},
-    {TileCfg<2>::BM, TileCfg<2>::BN, 0.86, 4, true}};
+    {TileCfg<1>::BM, TileCfg<1>::BN, 1.11, 2, true},
+    {TileCfg<2>::BM, TileCfg<2>::BN, 0.80, 4, true}};
+// ... over shorter sums, where the 64x64 tile is the faster one more often than
+// those efficiencies have it: at any size up to kRsShortK (of 340 timed products of
+// 17-128 the 128x128 tile wins one, by 4 %, and of 3954 later calls one by 11 %, 126 of
+// 472 x 204 x 82 32.4 us, 36.1: 256 x 65856 x 7 45.3 us, 64x64 32.2, the
+// fp32 kernel of 128x128 36.2; 3996 x 2735 x 34 56.5, 64x64 44; 91 of 322 x 235 x 88
+// 40.8, 34.2), and in outputs of few tiles up to kRsMidK.  Held against every
+// configuration at 1-16 splits and the wave-split tiles on 381 drawn products:
+// none loses 3 % to the plan by the efficiencies above, 7 fewer are more than 10 %
+// off the fastest.
+constexpr int kRsShortK = 128, kRsMidK = 400;
+constexpr double kRsShortEff[kNumCfg] = {0.85, 0.60, 0.86}, kRsMidEff[kNumCfg] = {1.54, 1.00, 0.86};
+
 // Vector layouts.  The efficiencies of gemm_f32_sp's configurations (above 1:
 // bf16 units), its round latency and the factor of a workgroup alone on its CU
 // (kSpAlone) were fitted to graph timings of every configuration at 1-16 splits
@@ -325,13 +333,6 @@ constexpr int kNarrowShortK = 160;
 // ranges: 2832 x 3904 x 864 128x128 138 us, 256x128 155.)
 constexpr double kSpBothMn128x128 = 1.10, kSpBothMn128x64 = 1.15;
 constexpr int kSpBothMnMaxK = 512;
-// Operands off 16-byte alignment over at most two chunks of K: the 64x64 tile,
-// at any size (256 x 65856 x 7: 32.2 us, 45.3 on 128x128, where the fp32 kernel of
-// that tile took 36.2; 432 x 24304 x 9: 26.8, 35.3, 26.7; 43 of 632 x 376 x 31:
-// 18.7, 21.9, 18.1; the largest loss 416 x 12544 x 31: 30.5, 29.4), which the
-// price of the 128x128 one at its other lengths does not say.
-constexpr int kRsShortK = 32;
-constexpr double kRsShortEff128 = 0.60;
 constexpr int kMaxForcedSplits = 64;
 
 // Tile grid and K split of configuration `cfg` asked for `s` splits (the
@@ -439,7 +440,7 @@ Plan make_plan_uncached(int64_t M, int64_t N, int64_t K, int64_t batch, int cus,
         const bool sp_product = dl && wide && !imw && cc.sp;   // matrix operands
         if (sp_product && cfg == 0) cc.eff = kProduct64x256;
         if (sp_product && cfg == 1 && K <= kThreeChunks) cc.eff = kShort128x128;
-        if (!dl && sp && cfg == 1 && K <= kRsShortK) cc.eff = kRsShortEff128;
+        if (!dl && sp && K <= kRsMidK) cc.eff = (K <= kRsShortK ? kRsShortEff : kRsMidEff)[cfg];
         for (int s = 1; s <= (imw ? kMaxImwSplits : kMaxSplits); ++s) {
             if (s > 1 && !allow_split) break;
             // this and every further split's partials cost more than the best plan
