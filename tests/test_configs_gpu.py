@@ -20,11 +20,11 @@ from util_parity import amax, assert_close
 
 pytestmark = pytest.mark.gpu
 
-# (family, configuration): 3 register-staged and 4 direct-to-LDS tiles that
-# take every operand form; direct-to-LDS configurations 4-6 (DLP, the
-# fragment-prefetching kernel with 256x256, 64x64 and 128x128 tiles) take only GEMMs
-# with K % 16 == 0 and no implicit-im2col operand or fused row sums, and have
-# tests of their own below.  (A CPU test pins the counts against the
+# (family, configuration): the 3 tiles of the family that takes any strides and 4
+# of the direct one that take every operand form (64x256, 128x128, 256x128 on the bf16
+# units, 64x64 on the fp32 ones); its configurations 4-6 (128x256 and 128x64 on the
+# bf16 units, the 64x64 fragment-prefetching kernel) take no forward im2col operand
+# and have tests of their own below.  (A CPU test pins the counts against the
 # library.)
 CONFIGS = [(mt.FAMILY_RS, c) for c in range(3)] + [(mt.FAMILY_DL, c) for c in range(4)]
 DL_CONFIGS = [c for f, c in CONFIGS if f == mt.FAMILY_DL]

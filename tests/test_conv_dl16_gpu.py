@@ -1,11 +1,11 @@
-"""The convolution kernel on 16x16 MFMA blocks (gemm_f32_dl16, direct-to-LDS
-configuration 7: 64x112 tiles, K-chunks split over two groups of waves)
-against the CPU oracle, forced through mt_gemm_force_config on the
-channels-last implicit-im2col operand, and taken by the cost model.
+"""The 64x112 convolution tile (gemm_f32_sp, configuration 7: blocks of 128
+columns of which 112 are the tile's; a kernel of its own on 16x16 MFMA blocks,
+gemm_f32_dl16, ran it before) against the CPU oracle, forced through
+mt_gemm_force_config on the channels-last implicit-im2col operand, and taken by
+the cost model.
 
 Cases: ragged output channels and pixels (tiles past M and N), K ranges of
-one chunk (empty wave groups), odd chunk counts (groups with one chunk less),
-1x1 to 5x5 kernels, strides 1-2, padding, bias, split-K on top, the input
+one chunk and odd chunk counts, 1x1 to 5x5 kernels, strides 1-2, padding, bias, split-K on top, the input
 gradient through the flipped-weight forward convolution, determinism, and
 the 5a layer at full size against the cost model's own plan.  Oracle: the
 reference's conv2d_cpu / conv2d_backward_input_cpu restated in
