@@ -318,7 +318,8 @@ constexpr int kSpAloneMinK = 512, kLoneStoreMaxK = 256;
 constexpr double kProduct64x256 = 1.04;   // efficiency of configuration 0 with matrix operands
 // Three chunks of K on outputs of many tiles: 64 of 512 x 512 x 48 25.1 us on
 // 128x128, 26.1 on the 64x64 fp32 tile, which the price of longer sums put first;
-// 4096 x 4096 x 40 25.9, 26.4.  (Two chunks: 22.4, 21.2; the 64x64 one stays.)
+// 4096 x 4096 x 40 25.9, 26.4.  (Two chunks: 22.4, 21.2; the 64x64 one stays, and with
+// both operands across rows, 1224 x 9216 x 42 48.3, 43.5.)
 constexpr int kThreeChunks = 48;
 constexpr double kShort128x128 = 1.30;
 // The 64x112 tile over short ranges of a split K, where its fill and drain weigh
@@ -330,9 +331,10 @@ constexpr int kNarrowShortK = 160;
 // a chunk wait for them (256-row and 256-column ones do not).  Measured over
 // predicted at 64-256 of K: 1.27-1.5 on 128x128, 1.3-1.4 on 128x64, 1.0 on
 // 256x128; 144 x 2656 x 2656: 31.6 us on 128x128, 29.5 on 256x128.  (Not over long
-// ranges: 2832 x 3904 x 864 128x128 138 us, 256x128 155.)
+// ranges: 2832 x 3904 x 864 128x128 138 us, 256x128 155; nor up to four chunks, where
+// 1224 x 18432 x 54 takes 76 us on 128x128 and 79 on the 64x64 fp32 tile.)
 constexpr double kSpBothMn128x128 = 1.10, kSpBothMn128x64 = 1.15;
-constexpr int kSpBothMnMaxK = 512;
+constexpr int kSpBothMnMinK = 64, kSpBothMnMaxK = 512;
 constexpr int kMaxForcedSplits = 64;
 
 // Tile grid and K split of configuration `cfg` asked for `s` splits (the
@@ -439,7 +441,7 @@ Plan make_plan_uncached(int64_t M, int64_t N, int64_t K, int64_t batch, int cus,
         if (dl && cfg == 0 && !wide && !im16 && !im4) cc.eff = kPhaseNarrowEff;
         const bool sp_product = dl && wide && !imw && cc.sp;   // matrix operands
         if (sp_product && cfg == 0) cc.eff = kProduct64x256;
-        if (sp_product && cfg == 1 && K <= kThreeChunks) cc.eff = kShort128x128;
+        if (sp_product && !mm && cfg == 1 && K <= kThreeChunks) cc.eff = kShort128x128;
         if (!dl && sp && K <= kRsMidK) cc.eff = (K <= kRsShortK ? kRsShortEff : kRsMidEff)[cfg];
         for (int s = 1; s <= (imw ? kMaxImwSplits : kMaxSplits); ++s) {
             if (s > 1 && !allow_split) break;
@@ -456,7 +458,7 @@ Plan make_plan_uncached(int64_t M, int64_t N, int64_t K, int64_t batch, int cus,
             if (sp_product) {
                 pc.lone_store = cfg <= 1 && pl.kps < kLoneStoreMaxK;
                 pc.alone = pc.lone_store || pl.kps >= kSpAloneMinK ? 1.0 : cc.occ > 1 ? kSpAlone : 0;
-                if (mm && pl.kps < kSpBothMnMaxK)
+                if (mm && pl.kps > kSpBothMnMinK && pl.kps < kSpBothMnMaxK)
                     pc.eff /= cfg == 1 ? kSpBothMn128x128 : cfg == 6 ? kSpBothMn128x64 : 1.0;
             }
             if (imw && cfg == 5 && pl.kps < kImwShortK) pc.alone = kImwShortAlone;
